@@ -292,6 +292,44 @@ def test_pack_lora_into_pool_equals_w_combined_index_put(gpu, dtype, hidden, pag
         assert np.array_equal(vals[l].float().cpu().numpy().reshape(n_pages, page_elems), want_v[l]), l
 
 
+@pytest.mark.parametrize("hidden,page_elems,h_out,rank", [
+    (4096, 4096, [4096] * 4, 64),               # whole tiles
+    (4096, 4096, [4096, 1024, 1024, 4096], 8),  # the longest tiles, narrow k/v
+    (1032, 1040, [1032, 8, 136, 1040], 72),     # two tiles over the rank, ragged long sides, padded pages
+    (5120, 5120, [5120] * 4, 24),               # tiles that are no power of two
+])
+def test_pack_lora_into_pool_tile_edges(gpu, hidden, page_elems, h_out, rank):
+    """The 16-byte packer at the edges of its tiles: the same bytes as the oracle's packer, byte for
+    byte (random 16-bit words, so every misplaced element shows)."""
+    from slora_hip.infer_adapter import pack_lora_into_pool
+    rng = np.random.default_rng(rank)
+    n_pages = 4 * rank + 5
+    loc_np = rng.permutation(n_pages)[: 4 * rank].astype(np.int64)
+
+    def words(*shape):
+        return rng.integers(1, 1 << 15, size=shape).astype(np.int16)
+
+    A = [words(hidden, rank) for _ in range(4)]
+    B = [words(rank, h) for h in h_out]
+    key, val = words(n_pages, page_elems), words(n_pages, page_elems)
+    want_k, want_v = key.copy(), val.copy()
+    for p in range(4):
+        loc = loc_np[p * rank: (p + 1) * rank]
+        want_k[loc] = 0
+        want_k[loc, :hidden] = A[p].T
+        flat = np.zeros(rank * page_elems, np.int16)
+        flat[: rank * h_out[p]] = B[p].T.reshape(-1)
+        want_v[loc] = flat.reshape(rank, page_elems)
+
+    def dev(a):
+        return torch.from_numpy(a).to(gpu).view(torch.float16)
+
+    gk, gv = dev(key).view(n_pages, 2, -1), dev(val).view(n_pages, 2, -1)
+    pack_lora_into_pool([gk], [gv], [[dev(a) for a in A]], [[dev(b) for b in B]], torch.from_numpy(loc_np).to(gpu), rank)
+    assert np.array_equal(gk.view(torch.int16).cpu().numpy().reshape(n_pages, -1), want_k)
+    assert np.array_equal(gv.view(torch.int16).cpu().numpy().reshape(n_pages, -1), want_v)
+
+
 @pytest.mark.parametrize("placement", [False, True])
 def test_infer_adapter_load_offload_and_decode(gpu, placement):
     """InferAdapter over a MemoryAllocator: adapters arrive in three loads (device matrices, and
