@@ -229,7 +229,7 @@ SLORA_API int slora_sgmm_shrink(void* o, const void* x, const void* w, const slo
  * aligned, owned by the caller); slora_sgmm_shrink_planned is slora_sgmm_shrink reading
  * that split: same arguments, same results bit for bit.
  *   *usable = 1: the plan was built.  0: this batch shape takes no plan (more than 256
- *   requests, more requests than workgroups, or nothing to do) -- call slora_sgmm_shrink.
+ *   requests, in large batches more requests than workgroups, or nothing to do) -- call slora_sgmm_shrink.
  * slora_sgmm_shrink_planned returns SLORA_ERR_BAD_SHAPE for such a shape.  The sizes
  * (n_requests, max_input_len, n_tokens, max_rank) must be those of the build call; a plan
  * of another launch shape makes the kernel leave `o` untouched. */
@@ -287,6 +287,19 @@ SLORA_API int slora_sgmm_expand_qkv(void* o_q, void* o_k, void* o_v, const void*
                           int64_t feat_out_kv, int64_t page_elems, int64_t max_rank, int64_t x_row_stride,
                           int64_t w_row_stride, int64_t o_row_stride_q, int64_t o_row_stride_kv, int64_t n_pages,
                           int dtype, void* stream);
+
+/* slora_sgmm_expand (nproj = 1: o0, x0, feat_out0, o_row_stride0, any qkvo) or slora_sgmm_expand_qkv (nproj = 3,
+ * qkvo = 0; k and v share feat_out12 and o_row_stride12) with a plan of slora_sgmm_plan_build for this batch: same
+ * results bit for bit.  Small batches (tokens times rank up to 32768) read their row spans from the plan
+ * instead of looking the requests up in every workgroup; larger ones leave the plan alone.  The sizes must
+ * be those of the build call, as for slora_sgmm_shrink_planned. */
+SLORA_API int slora_sgmm_expand_planned(const void* plan, int nproj, void* o0, void* o1, void* o2, const void* x0,
+                          const void* x1, const void* x2, const void* w, const slora_tables* tables, const void* scales,
+                          int scales_dtype, const int32_t* b_start_loc, const int32_t* b_seq_len,
+                          const int64_t* b_indicies, int64_t n_requests, int64_t max_input_len, int64_t n_tokens,
+                          int64_t feat_out0, int64_t feat_out12, int64_t page_elems, int64_t max_rank,
+                          int64_t x_row_stride, int64_t w_row_stride, int64_t o_row_stride0, int64_t o_row_stride12,
+                          int64_t n_pages, int qkvo, int dtype, void* stream);
 
 /* ---- moving adapters in and out of the pool --------------------------------- */
 

@@ -1050,8 +1050,275 @@ __global__ __launch_bounds__(kShrThreads, RING ? 2 : 1) void sgmm_shrink_kernel(
 constexpr int kSegPlanMagic = 0x53475031;
 constexpr int kSegPlanHeaderWords = 16;
 constexpr int kSegPartWords = 8;
-enum SegPlanHeader { SP_MAGIC = 0, SP_PARTS, SP_SPLIT, SP_NREQ, SP_NTOKENS, SP_MAXRANK, SP_ROWCAP, SP_STATUS };  // SP_STATUS: as PH_STATUS of the decode plan (word 7)
-enum SegPart { PT_ROW = 0, PT_ROWS, PT_RANK, PT_START_LO, PT_START_HI };
+enum SegPlanHeader {
+  SP_MAGIC = 0, SP_PARTS, SP_SPLIT, SP_NREQ, SP_NTOKENS, SP_MAXRANK, SP_ROWCAP,
+  SP_STATUS,  // as PH_STATUS of the decode plan (word 7)
+  SP_SPANS    // small batches: records of the expand behind the SP_PARTS of the shrink (0: none)
+};
+enum SegPart { PT_ROW = 0, PT_ROWS, PT_RANK, PT_START_LO, PT_START_HI, PT_ADAPTER };
+
+// ---------------------------------------------------------------------------
+// shrink of small batches: K split over the wavefronts of a workgroup
+// ---------------------------------------------------------------------------
+// Up to a few thousand tokens a launch has fewer 64-row tiles than compute units, and what it waits for
+// is one workgroup's chain of round trips.  Here a part is 16 rows of one request, and its
+// (projection, group of 16 * NT rank columns) pairs are workgroups of their own.  The eight
+// wavefronts share K in chunks of 8 * C elements (C 16-byte pieces: 512 elements, or 320 where the
+// hidden size is a multiple of 2560), and a wavefront requests all of a chunk -- 16 rows of x
+// and 16 * NT weight rows -- before it needs any of it: at hidden 4096 that is the whole K
+// loop, one round trip.  Each load instruction covers 1 KiB of one row.  That is what makes the
+// difference: loads that touch 8 rows by 128 bytes (the order the other kernels load in) have
+// one compute unit move about 26 GB/s, and a launch of 64 tokens of rank 8 takes 8.3 us; with
+// whole rows it takes 6.7 (14 us through the register-fed kernels below).  The rows become MFMA fragments through a strip of LDS per wavefront (pieces
+// xor-swizzled by row: no bank conflicts either way, no barrier).  The eight partial tiles are
+// summed in wavefront order through LDS: the sums do not depend on how the rows were cut into
+// parts, and q, k and v in one launch are bit for bit the three calls.
+constexpr int kSplitThreads = 512;
+constexpr int kSplitWaves = kSplitThreads / kWave;
+constexpr int kSplitRows = 16;
+constexpr int kSegMaxReqs = 256;   // requests a plan (or a workgroup without one) describes: one per thread
+constexpr int kSegMaxParts = 512;  // records of either kind in a plan
+
+template <int NT>
+constexpr int kSplitLd = 16 * NT + 4;  // row pitch (floats) of a partial tile
+template <int C>
+constexpr int kSplitStrip = kSplitRows * C * 16;  // LDS bytes of a wavefront: a chunk of 16 rows, later its partial tile
+
+// What a record of a plan says about a part: rows row_first .. + m_rows of one request.
+struct SegPartRec {
+  int row_first, m_rows, rank;
+  int64_t start;
+};
+
+// All threads of the workgroup: one part, rank columns nb .. + 16 * NT (those below max_rank) of projection pj.
+template <typename T, int NT, int C>
+__device__ __forceinline__ void split_part(const SegShrinkArgs& p, unsigned char* s_all, const SegPartRec& rec, int pj,
+                                           int nb) {
+  constexpr int kLd = kSplitLd<NT>, kL = C / 4;  // kL: load instructions, and MFMA steps, of 16 rows of a chunk
+  static_assert(C % 8 == 0 && kSplitRows * kLd * 4 <= kSplitStrip<C>, "the swizzle keeps to groups of 8 pieces");
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r_eff = rec.rank < p.max_rank ? rec.rank : p.max_rank;
+  const int nb_cnt = p.max_rank - nb < 16 * NT ? p.max_rank - nb : 16 * NT;
+  const int own = r_eff - nb;  // columns of the adapter among them
+  const int64_t base_li = rec.start + (int64_t)rec.rank * (p.qkvo + pj);
+  uint16_t* og = reinterpret_cast<uint16_t*>(pj == 2 ? p.o[2] : (pj == 1 ? p.o[1] : p.o[0]));
+  const uint16_t* xg = reinterpret_cast<const uint16_t*>(p.x);
+  const uint16_t* wg = reinterpret_cast<const uint16_t*>(p.w);
+  unsigned char* strip = s_all + wave * kSplitStrip<C>;
+  const int lr = lane & 15, lg = lane >> 4;
+  // lane l: the page of weight row nb + l; a row that does not exist reads pool page 0, and its products
+  // only reach columns that are written as zeros
+  int64_t page = seg_page_nobranch(p.t, base_li + nb + lane, lane < own && p.t.n_loc > 0);
+  if (page < 0) page = 0;
+  const int page_lo = (int)(uint32_t)page, page_hi = (int)((uint64_t)page >> 32);
+  // piece i * 64 + lane of a chunk's 16 rows: its row and its place in the row
+  auto row_of = [&](int i) { return C == 64 ? i : (i * 64 + lane) / C; };
+  auto piece_of = [&](int i) { return C == 64 ? lane : (i * 64 + lane) % C; };
+  auto slot = [&](int row, int piece) { return reinterpret_cast<u32x4*>(strip + (row * C + (piece ^ (row & 7))) * 16); };
+  const int chunks = (p.h_in + 8 * C - 1) / (8 * C);
+  for (int m0 = 0; m0 < rec.m_rows; m0 += kSplitRows) {
+    const int m_cnt = rec.m_rows - m0 < kSplitRows ? rec.m_rows - m0 : kSplitRows;
+    const int64_t row0 = (int64_t)rec.row_first + m0;
+    f32x4 acc[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int ch = wave; own > 0 && ch < chunks; ch += kSplitWaves) {
+      const int k0 = ch * 8 * C;
+      const int n_pieces = (p.h_in - k0) >> 3;  // C unless the last chunk is cut short: zeros behind it
+      u32x4 x[kL], w[NT][kL];
+#pragma unroll
+      for (int i = 0; i < kL; ++i) {
+        int row = row_of(i);
+        if (row >= m_cnt) row = m_cnt - 1;  // rows past the end repeat the last one and are not stored
+        const int pc = piece_of(i) < n_pieces ? piece_of(i) : 0;
+        x[i] = ldg16(xg + (row0 + row) * p.x_stride + k0 + pc * 8);
+      }
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int i = 0; i < kL; ++i) {
+          const int j = t * 16 + row_of(i);
+          const int lo = C == 64 ? __builtin_amdgcn_readlane(page_lo, j) : __shfl(page_lo, j, kWave);
+          const int hi = C == 64 ? __builtin_amdgcn_readlane(page_hi, j) : __shfl(page_hi, j, kWave);
+          const int64_t pg = (int64_t)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
+          const int pc = piece_of(i) < n_pieces ? piece_of(i) : 0;
+          w[t][i] = ldg16(wg + pg * p.w_stride + k0 + pc * 8);
+        }
+#pragma unroll
+      for (int i = 0; i < kL; ++i) *slot(row_of(i), piece_of(i)) = piece_of(i) < n_pieces ? x[i] : zero16();
+#pragma unroll
+      for (int s = 0; s < kL; ++s) x[s] = *slot(lr, 4 * s + lg);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+#pragma unroll
+        for (int i = 0; i < kL; ++i) *slot(row_of(i), piece_of(i)) = piece_of(i) < n_pieces ? w[t][i] : zero16();
+#pragma unroll
+        for (int s = 0; s < kL; ++s) acc[t] = mfma16<T>(x[s], *slot(lr, 4 * s + lg), acc[t]);
+      }
+    }
+    if (own > 0) {
+      float* mine = reinterpret_cast<float*>(strip);
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) mine[(lg * 4 + i) * kLd + t * 16 + lr] = acc[t][i];
+    }
+    __syncthreads();
+    // two neighbouring columns per thread
+    const bool pairs = (p.o_stride & 1) == 0 && (reinterpret_cast<uintptr_t>(og) & 3) == 0;
+    for (int idx = tid; idx < kSplitRows * 8 * NT; idx += kSplitThreads) {
+      const int m = idx / (8 * NT), c = (idx - m * (8 * NT)) * 2;
+      if (m >= m_cnt || c >= nb_cnt) continue;
+      float v0 = 0.f, v1 = 0.f;
+      if (c < own) {
+#pragma unroll
+        for (int wv = 0; wv < kSplitWaves; ++wv) {
+          const float* q = reinterpret_cast<const float*>(s_all + wv * kSplitStrip<C>) + m * kLd + c;
+          v0 += q[0];
+          v1 += q[1];
+        }
+        if (c + 1 >= own) v1 = 0.f;
+      }
+      uint16_t* op = og + (row0 + m) * p.o_stride + nb + c;
+      const uint16_t lo = T::from_float(v0), hi = T::from_float(v1);
+      if (pairs && c + 1 < nb_cnt) {  // (nb + c is even)
+        *reinterpret_cast<uint32_t*>(op) = (uint32_t)lo | ((uint32_t)hi << 16);
+      } else {
+        op[0] = lo;
+        if (c + 1 < nb_cnt) op[1] = hi;
+      }
+    }
+    __syncthreads();  // the strips are rewritten for the next rows
+  }
+}
+
+// Thread j of the first kSegMaxReqs describes request j: rows clipped to the buffers and to row_cap, 0 if it has
+// nothing to do.  Loads outside every branch, in two dependent groups.
+__device__ __forceinline__ void seg_describe(const SegTables& t, int row_cap, int64_t& a, int64_t& start, int& r,
+                                             int& row0, int& rows) {
+  const bool mine = (int)threadIdx.x < t.n_requests;
+  const int rq = mine ? (int)threadIdx.x : 0;
+  a = t.b_indicies[rq];
+  row0 = t.b_start_loc[rq];
+  rows = t.b_seq_len[rq];
+  const bool a_ok = (uint64_t)a < (uint64_t)t.n_adapters;
+  const int64_t len = t.a_len[a_ok ? a : 0];
+  start = t.a_start[a_ok ? a : 0];
+  r = (int)(len >> 2);
+  if (mine && a_ok && row0 >= 0 && rows > 0 && row0 < t.n_tokens) {
+    if (rows > t.n_tokens - row0) rows = t.n_tokens - row0;
+    if (rows > row_cap) rows = row_cap;
+  } else {
+    rows = 0;
+  }
+}
+
+// Inclusive prefix sum over a workgroup of W wavefronts; *total receives the sum.
+template <int W>
+__device__ __forceinline__ int seg_scan(int v, int* s_wave, int* total) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int inc = v;
+#pragma unroll
+  for (int o = 1; o < kWave; o <<= 1) {
+    const int up = __shfl_up(inc, o, kWave);
+    if (lane >= o) inc += up;
+  }
+  if (lane == kWave - 1) s_wave[wave] = inc;
+  __syncthreads();
+  int before = 0, tot = 0;
+#pragma unroll
+  for (int wv = 0; wv < W; ++wv) {
+    const int c = s_wave[wv];
+    if (wv < wave) before += c;
+    tot += c;
+  }
+  __syncthreads();
+  *total = tot;
+  return before + inc;
+}
+
+// Cuts the described requests into parts of `unit` rows; if that gives more than `parts` of them (requests that
+// overlap in the batch), of twice as many, and so on: one part per request always fits.  Returns the
+// number of parts of this thread's request; `before`: parts in front of them, `n`: all parts.
+template <int W>
+__device__ __forceinline__ int seg_cut(int rows, int& unit, int parts, int* s_wave, int& before, int& n) {
+  for (;;) {
+    const int mine = (rows + unit - 1) / unit;
+    const int inc = seg_scan<W>(mine, s_wave, &n);
+    if (n <= parts || unit > (1 << 29)) {
+      before = inc - mine;
+      return mine;
+    }
+    unit <<= 1;
+  }
+}
+
+// Part i of n -> its record.  Consecutive workgroup ids go to the 8 XCDs in turn and record
+// q * (parts / 8) + j belongs to XCD q: every XCD gets a contiguous eighth of the parts, so that
+// the parts of a request, which read the same weight rows, share an L2.
+__device__ __forceinline__ int seg_xcd_slot(int i, int n, int parts) {
+  const int q = (8 * (i + 1) - 1) / n;
+  return q * (parts >> 3) + i - (int)((int64_t)n * q / 8);
+}
+
+// Grid: (part, projection, rank group) as seg_xcd_slot lays the parts out.  With a plan the part is
+// one group of scalar loads away; without one the workgroup describes the requests itself.
+template <typename T, int NT, int C>
+__global__ __launch_bounds__(kSplitThreads) void sgmm_shrink_split_kernel(const SegShrinkArgs p, const int* plan,
+                                                                          int parts, int groups) {
+  extern __shared__ __align__(16) unsigned char s_strips[];  // [kSplitWaves][kSplitStrip<C>]
+  __shared__ int s_wave[kSplitWaves];
+  __shared__ int s_rec[4];
+  __shared__ int64_t s_start;
+  const int sub_n = groups * p.nproj;
+  const int within = (int)(blockIdx.x >> 3);
+  const int j = __builtin_amdgcn_readfirstlane(within / sub_n);
+  const int sub = within - j * sub_n;
+  const int pj = __builtin_amdgcn_readfirstlane(sub / groups);
+  const int nb = (sub - pj * groups) * 16 * NT;
+  const int slot = (int)(blockIdx.x & 7) * (parts >> 3) + j;
+  SegPartRec rec;
+  if (plan != nullptr) {
+    typedef const int __attribute__((address_space(4))) * ConstWords;
+    ConstWords head = (ConstWords)plan;
+    ConstWords w = head + kSegPlanHeaderWords + slot * kSegPartWords;
+    int magic = head[SP_MAGIC], n_parts = head[SP_PARTS], split = head[SP_SPLIT], n_tok = head[SP_NTOKENS];
+    int row = w[PT_ROW], rows = w[PT_ROWS], r = w[PT_RANK], lo = w[PT_START_LO], hi = w[PT_START_HI];
+    asm volatile("" : "+s"(magic), "+s"(n_parts), "+s"(split), "+s"(n_tok), "+s"(row), "+s"(rows), "+s"(r), "+s"(lo), "+s"(hi));
+    if (magic != kSegPlanMagic || n_parts != parts || split != -kSplitRows || n_tok != p.t.n_tokens) {
+      if (magic == kSegPlanMagic && blockIdx.x == 0 && threadIdx.x == 0) const_cast<int*>(plan)[SP_STATUS] = 1;
+      return;
+    }
+    rec = {row, rows, r, (int64_t)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo)};
+  } else {
+    int64_t a = 0, start = 0;
+    int r = 0, row0 = 0, rows = 0, unit = kSplitRows, before = 0, n = 0;
+    seg_describe(p.t, p.m_tiles * kShrTM, a, start, r, row0, rows);
+    if (threadIdx.x == 0) s_rec[1] = 0;
+    const int mine = seg_cut<kSplitWaves>(rows, unit, parts, s_wave, before, n);
+    // my part: number i = first of this XCD + j, if this XCD has that many
+    const int q = (int)(blockIdx.x & 7);
+    const int i = (int)((int64_t)n * q / 8) + j;
+    if (i < (int)((int64_t)n * (q + 1) / 8) && i >= before && i < before + mine) {
+      const int m0 = (i - before) * unit;
+      s_rec[0] = row0 + m0;
+      s_rec[1] = rows - m0 < unit ? rows - m0 : unit;
+      s_rec[2] = r;
+      s_start = start;
+    }
+    __syncthreads();
+    auto uni = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
+    rec.row_first = uni(s_rec[0]);
+    rec.m_rows = uni(s_rec[1]);
+    rec.rank = uni(s_rec[2]);
+    const int64_t st = s_start;
+    rec.start = (int64_t)(((uint64_t)(uint32_t)uni((int)((uint64_t)st >> 32)) << 32) | (uint32_t)uni((int)(uint32_t)st));
+  }
+  if (rec.m_rows <= 0 || rec.row_first < 0 || rec.m_rows > p.t.n_tokens - rec.row_first) return;
+  split_part<T, NT, C>(p, s_strips, rec, pj, nb);
+}
 
 // One workgroup.  Same scheme as the few-requests case of sgmm_shrink_kernel (request j
 // in n_j even chunks, T bisected), with more rounds; record `part` = chunk `part` in
@@ -1124,6 +1391,50 @@ __global__ __launch_bounds__(kShrThreads) void sgmm_plan_kernel(int* plan, SegTa
     plan[SP_MAXRANK] = max_rank;
     plan[SP_ROWCAP] = row_cap;
     plan[SP_STATUS] = 0;
+  }
+}
+
+// The plan of a small batch, one workgroup: the parts of the shrink (kSplitRows rows, laid out by
+// seg_xcd_slot; SP_SPLIT holds -kSplitRows) and behind them the spans of the expand (span_rows rows, in order).
+__global__ __launch_bounds__(kSegMaxReqs) void sgmm_plan_small_kernel(int* plan, SegTables t, int parts, int spans,
+                                                                      int span_rows, int max_rank, int row_cap,
+                                                                      int row_cap_exp) {
+  constexpr int W = kSegMaxReqs / kWave;
+  __shared__ int s_wave[W];
+  const int tid = threadIdx.x;
+  for (int i = tid; i < (parts + spans) * kSegPartWords; i += kSegMaxReqs) plan[kSegPlanHeaderWords + i] = 0;
+  int64_t a = 0, start = 0;
+  int r = 0, row0 = 0, rows = 0;
+  seg_describe(t, row_cap > row_cap_exp ? row_cap : row_cap_exp, a, start, r, row0, rows);
+  auto emit = [&](int* rec, int m0, int cnt) {
+    rec[PT_ROW] = row0 + m0;
+    rec[PT_ROWS] = cnt;
+    rec[PT_RANK] = r;
+    rec[PT_START_LO] = (int)(uint32_t)start;
+    rec[PT_START_HI] = (int)((uint64_t)start >> 32);
+    rec[PT_ADAPTER] = (int)a;
+  };
+  int before = 0, n = 0, unit = kSplitRows;
+  const int rows_s = rows < row_cap ? rows : row_cap, rows_e = rows < row_cap_exp ? rows : row_cap_exp;
+  int mine = seg_cut<W>(rows_s, unit, parts, s_wave, before, n);  // (its barriers also separate the zeros from the records)
+  for (int i = 0; i < mine; ++i)
+    emit(plan + kSegPlanHeaderWords + seg_xcd_slot(before + i, n, parts) * kSegPartWords, i * unit,
+         rows_s - i * unit < unit ? rows_s - i * unit : unit);
+  unit = span_rows;
+  mine = seg_cut<W>(rows_e, unit, spans, s_wave, before, n);
+  for (int i = 0; i < mine; ++i)
+    emit(plan + kSegPlanHeaderWords + (parts + before + i) * kSegPartWords, i * unit,
+         rows_e - i * unit < unit ? rows_e - i * unit : unit);
+  if (tid == 0) {
+    plan[SP_MAGIC] = kSegPlanMagic;
+    plan[SP_PARTS] = parts;
+    plan[SP_SPLIT] = -kSplitRows;
+    plan[SP_NREQ] = t.n_requests;
+    plan[SP_NTOKENS] = t.n_tokens;
+    plan[SP_MAXRANK] = max_rank;
+    plan[SP_ROWCAP] = row_cap;
+    plan[SP_STATUS] = 0;
+    plan[SP_SPANS] = spans;
   }
 }
 
@@ -1276,17 +1587,14 @@ template <int KS>
 constexpr int kExpLdsRow = KS * 64 + 16;
 constexpr int kExpChunkRows = 4 * kExpTMW;  // rows staged at a time
 
-// B^T fragments of outputs nb .. nb + 63 (MFMA A operand)
-template <typename T, int KS>
-__device__ __forceinline__ void expand_load_weights(const SegExpandArgs& p, int r, int r_eff, int64_t base_li, int nb,
-                                                    u32x4 (&a)[4][KS]) {
+// B^T fragments of outputs nb .. nb + 63 (MFMA A operand), in two phases: every page id (loads back to back, no
+// branch in between), then every fragment, from a valid dummy address where there is none.
+template <int KS>
+__device__ __forceinline__ void expand_weight_pages(const SegExpandArgs& p, int r, int r_eff, int64_t base_li, int nb,
+                                                    int64_t (&page)[4][KS], uint32_t (&off)[4][KS]) {
   const int lane = threadIdx.x & 63;
   const int lr = lane & 15, lg = lane >> 4;
-  const uint16_t* wg = reinterpret_cast<const uint16_t*>(p.w);
   const uint32_t page_elems = (uint32_t)p.page_elems;
-  // phase 1: every page id (loads back to back, no branch in between)
-  int64_t page[4][KS];
-  uint32_t off[4][KS];
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
     const int n = nb + 32 * (t >> 1) + 8 * (lr >> 2) + 4 * (t & 1) + (lr & 3);
@@ -1300,7 +1608,12 @@ __device__ __forceinline__ void expand_load_weights(const SegExpandArgs& p, int 
       page[t][s] = seg_page_nobranch(p.t, base_li + pg, want);
     }
   }
-  // phase 2: every fragment, from a valid dummy address where there is none
+}
+
+template <int KS>
+__device__ __forceinline__ void expand_weight_frags(const SegExpandArgs& p, const int64_t (&page)[4][KS],
+                                                    const uint32_t (&off)[4][KS], u32x4 (&a)[4][KS]) {
+  const uint16_t* wg = reinterpret_cast<const uint16_t*>(p.w);
 #pragma unroll
   for (int t = 0; t < 4; ++t)
 #pragma unroll
@@ -1367,6 +1680,28 @@ __device__ __forceinline__ void expand_chunk_store(const ExpandChunk<KS>& c, cha
   }
 }
 
+// y (line order) + scale * the sums of one 16-row fragment; C tile t: lane holds token column lr, rows
+// 4*lg + i  ->  output 32*(t/2) + 8*lg + 4*(t%2) + i
+template <typename T>
+__device__ __forceinline__ void expand_add(const f32x4 (&acc)[4], float scale, u32x4 y0, u32x4 y1, u32x4 (&out)[2]) {
+  swap_halves(y0, y1);  // line order -> MFMA order: y0 = outputs nb + 8*lg .., y1 = outputs nb + 32 + 8*lg ..
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const u32x4& yv = h == 0 ? y0 : y1;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      // outputs n + 2q, n + 2q + 1  <-  tile 2h + (2q)/4, element (2q)%4 and the next
+      const int e0 = 2 * q;
+      const float d0 = acc[2 * h + (e0 >> 2)][e0 & 3] * scale;
+      const float d1 = acc[2 * h + ((e0 + 1) >> 2)][(e0 + 1) & 3] * scale;
+      const uint16_t lo = T::from_float(T::lo(yv[q]) + d0);
+      const uint16_t hi = T::from_float(T::hi(yv[q]) + d1);
+      out[h][q] = (uint32_t)lo | ((uint32_t)hi << 16);
+    }
+  }
+  swap_halves(out[0], out[1]);  // back to line order
+}
+
 // One row tile: multiply the staged delta rows m_rel .. m_rel + 31 of the span by the
 // block's B^T fragments, add to y and store.
 template <typename T, int KS>
@@ -1394,28 +1729,11 @@ __device__ __forceinline__ void expand_finish(const SegExpandArgs& p, float scal
 #pragma unroll
       for (int s = 0; s < KS; ++s) acc[f][t] = mfma16<T>(a[t][s], b[f][s], acc[f][t]);
     }
-  // C tile t: lane holds token column lr, rows 4*lg + i  ->  output 32*(t/2) + 8*lg + 4*(t%2) + i
   const int n_line = nb + 8 * (lg + 4 * (lr >> 3));
 #pragma unroll
   for (int f = 0; f < kExpMF; ++f) {
-    u32x4 y0 = st.y[f][0], y1 = st.y[f][1];
-    swap_halves(y0, y1);  // line order -> MFMA order: y0 = outputs nb + 8*lg .., y1 = outputs nb + 32 + 8*lg ..
     u32x4 out[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const u32x4& yv = h == 0 ? y0 : y1;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        // outputs n + 2q, n + 2q + 1  <-  tile 2h + (2q)/4, element (2q)%4 and the next
-        const int e0 = 2 * q;
-        const float d0 = acc[f][2 * h + (e0 >> 2)][e0 & 3] * scale;
-        const float d1 = acc[f][2 * h + ((e0 + 1) >> 2)][(e0 + 1) & 3] * scale;
-        const uint16_t lo = T::from_float(T::lo(yv[q]) + d0);
-        const uint16_t hi = T::from_float(T::hi(yv[q]) + d1);
-        out[h][q] = (uint32_t)lo | ((uint32_t)hi << 16);
-      }
-    }
-    swap_halves(out[0], out[1]);  // back to line order
+    expand_add<T>(acc[f], scale, st.y[f][0], st.y[f][1], out);
 #pragma unroll
     for (int g = 0; g < 2; ++g) {
       const int m = m0w + f * 16 + 8 * g + (lr & 7);
@@ -1441,7 +1759,10 @@ __device__ __forceinline__ void expand_mfma(const SegExpandArgs& p, int r, int r
   // row), then the B^T fragments behind their page ids
   expand_load_rows(p, row0, m0, m_end, m0, nb, cur);
   expand_chunk_load<KS>(p, row0, m0, m_end, m0, chunk);
-  expand_load_weights<T, KS>(p, r, r_eff, base_li, live ? nb : 0, a);
+  int64_t page[4][KS];
+  uint32_t off[4][KS];
+  expand_weight_pages<KS>(p, r, r_eff, base_li, live ? nb : 0, page, off);
+  expand_weight_frags<KS>(p, page, off, a);
   expand_chunk_store<KS>(chunk, s_x);
   __syncthreads();
   int buf = 0;
@@ -1610,6 +1931,96 @@ __global__ __launch_bounds__(kExpThreads) void sgmm_expand_walk_kernel(const Seg
   }
 }
 
+// Small batches with a plan: workgroup = (span of up to kExpTMW rows of one request, 256 outputs), one
+// group of scalar loads away from its rows.  Everything a wavefront needs is requested at once -- y
+// in line order, the delta rows straight from memory in MFMA order (a few KB that the four
+// wavefronts and the other output groups share in L2), B^T behind its page ids -- and nothing waits for another
+// wavefront: no LDS, no barrier.  XCD q owns output groups q, q + 8, ... of all requests, so
+// that every L2 holds its own eighth of B^T.
+template <typename T, int KS>
+__global__ __launch_bounds__(kExpThreads) void sgmm_expand_span_kernel(const SegExpandArgs p_all, const int* plan,
+                                                                       int parts, int spans, int groups_per_xcd) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int within = (int)(blockIdx.x >> 3);
+  const int span = __builtin_amdgcn_readfirstlane(within / groups_per_xcd);
+  int group = (within - span * groups_per_xcd) * 8 + (int)(blockIdx.x & 7);
+  if (group >= p_all.n_chunks) return;
+  typedef const int __attribute__((address_space(4))) * ConstWords;
+  ConstWords head = (ConstWords)plan;
+  ConstWords w = head + kSegPlanHeaderWords + (parts + span) * kSegPartWords;
+  int magic = head[SP_MAGIC], n_parts = head[SP_PARTS], n_spans = head[SP_SPANS], n_tok = head[SP_NTOKENS];
+  int row0 = w[PT_ROW], rows = w[PT_ROWS], r = w[PT_RANK], lo = w[PT_START_LO], hi = w[PT_START_HI], ad = w[PT_ADAPTER];
+  asm volatile("" : "+s"(magic), "+s"(n_parts), "+s"(n_spans), "+s"(n_tok), "+s"(row0), "+s"(rows), "+s"(r), "+s"(lo), "+s"(hi), "+s"(ad));
+  if (magic != kSegPlanMagic || n_parts != parts || n_spans != spans || n_tok != p_all.t.n_tokens) {
+    if (magic == kSegPlanMagic && blockIdx.x == 0 && threadIdx.x == 0) const_cast<int*>(plan)[SP_STATUS] = 1;
+    return;
+  }
+  if (rows <= 0 || row0 < 0 || rows > p_all.t.n_tokens - row0 || (uint64_t)(int64_t)ad >= (uint64_t)p_all.t.n_adapters) return;
+  const SegExpandArgs p = p_all.nproj == 3 ? expand_select<3>(p_all, group) : p_all;
+  const int r_eff = r < p.max_rank ? r : p.max_rank;
+  if (r_eff <= 0) return;
+  const int64_t base_li = (int64_t)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo) + (int64_t)r * p.qkvo;
+  const float scale = load_scale(p.scales, p.scales_dtype, ad);
+  const int n0 = group * kExpGroup;
+  if (!p.vec_ok || (r & 7) != 0 || (r_eff & 7) != 0 || r_eff > 128) {
+    const int n_end = n0 + kExpGroup < p.feat_out ? n0 + kExpGroup : p.feat_out;
+    expand_generic<T>(p, r, r_eff, base_li, scale, row0, 0, rows, n0, n_end - n0);
+    return;
+  }
+  const int nb = n0 + wave * kExpOB;
+  if (nb >= p.feat_out) return;
+  const int lr = lane & 15, lg = lane >> 4;
+  const uint16_t* xg = reinterpret_cast<const uint16_t*>(p.x);
+  uint16_t* og = reinterpret_cast<uint16_t*>(p.o);
+  const int n_line = nb + 8 * (lg + 4 * (lr >> 3));
+  const bool n_in = n_line < p.feat_out;
+  int64_t page[4][KS];
+  uint32_t off[4][KS];
+  expand_weight_pages<KS>(p, r, r_eff, base_li, nb, page, off);
+  u32x4 a[4][KS];
+  // (a span holds more than kExpTMW rows only where requests overlap in the batch)
+#pragma unroll 1
+  for (int m0 = 0; m0 < rows; m0 += kExpTMW) {
+    u32x4 y[kExpMF][2], b[kExpMF][KS];
+#pragma unroll
+    for (int f = 0; f < kExpMF; ++f)
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+        const int m = m0 + f * 16 + 8 * g + (lr & 7);
+        y[f][g] = ldg16_stream(og + (int64_t)(row0 + (m < rows ? m : rows - 1)) * p.o_stride + (n_in ? n_line : 0));
+      }
+#pragma unroll
+    for (int f = 0; f < kExpMF; ++f)
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        const int m = m0 + f * 16 + lr, d = s * 32 + lg * 8;
+        b[f][s] = ldg16(xg + (int64_t)(row0 + (m < rows ? m : rows - 1)) * p.x_stride + (d < r_eff ? d : 0));
+      }
+    if (m0 == 0) expand_weight_frags<KS>(p, page, off, a);
+#pragma unroll
+    for (int f = 0; f < kExpMF; ++f) {
+#pragma unroll
+      for (int s = 0; s < KS; ++s)
+        if (s * 32 + lg * 8 >= r_eff) b[f][s] = zero16();
+      f32x4 acc[4];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < KS; ++s) acc[t] = mfma16<T>(a[t][s], b[f][s], acc[t]);
+      }
+      u32x4 out[2];
+      expand_add<T>(acc, scale, y[f][0], y[f][1], out);
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+        const int m = m0 + f * 16 + 8 * g + (lr & 7);
+        if (m < rows && n_in) stg16_stream(og + (int64_t)(row0 + m) * p.o_stride + n_line, out[g]);
+      }
+    }
+  }
+}
+
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
@@ -1670,6 +2081,81 @@ void shrink_geometry(int64_t n_tokens, int64_t n_requests, int64_t m_tiles, int6
 // a plan holds one record per row part: usable where no part spans two requests
 bool shrink_plan_usable(int64_t n_requests, int64_t m_tiles, int64_t grid, int cs) {
   return grid > 0 && n_requests <= kShrChunk && n_requests <= grid / cs && m_tiles <= 1024;
+}
+
+// Which batches take sgmm_shrink_split_kernel.  It reads a request's weight rows once per 16 token rows, the
+// other kernels once per 64, so the line falls with the rank.  us per launch (one projection / q, k and v; hidden
+// 4096, f16, rank 64), split kernel against the register-fed ones: 512 tokens 7.2 / 10.0 against 14.2 / 30, 1024 12.5 /
+// 18.1 against 14.3 / 31.7, 2311 18.1 / 35.9 against 19 / 37; 4096 27 / 46 against 23.2 / 42.1.  A whole layer at rank
+// 32: 2311 tokens 88.6 against 100.7 us, 4096 137 against 135.
+bool small_batch(int64_t n_tokens, int64_t n_requests, int64_t max_rank) {
+  return n_tokens > 0 && n_tokens <= 3584 && n_requests > 0 && n_requests <= kSegMaxReqs && max_rank > 0 &&
+         n_tokens * ((max_rank + 31) / 32) <= 4608;
+}
+
+struct SmallGeometry {
+  int parts;  // shrink: parts of kSplitRows rows, a multiple of 8 of them
+  int spans;  // expand: spans of kExpTMW rows
+};
+
+SmallGeometry small_geometry(int64_t n_tokens, int64_t n_requests, int64_t max_input_len) {
+  auto pieces = [&](int rows) {  // at least one per request, and enough for requests that do not overlap
+    const int64_t by_tokens = n_tokens / rows + n_requests, by_len = n_requests * ((max_input_len + rows - 1) / rows);
+    return (int)(by_tokens < by_len ? by_tokens : by_len);
+  };
+  return {(pieces(kSplitRows) + 7) / 8 * 8, pieces(kExpTMW)};
+}
+
+template <typename T, int NT, int C>
+int launch_split(const SegShrinkArgs& p, const int* plan, int parts, hipStream_t stream) {
+  auto kernel = sgmm_shrink_split_kernel<T, NT, C>;
+  constexpr int lds = kSplitWaves * kSplitStrip<C>;
+  static PerDeviceOnce once;
+  if (!raise_dynamic_lds(reinterpret_cast<const void*>(kernel), lds, once)) return SLORA_ERR_LAUNCH;
+  const int groups = (p.max_rank + 16 * NT - 1) / (16 * NT);
+  hipLaunchKernelGGL(kernel, dim3((uint32_t)(parts * groups * p.nproj)), dim3(kSplitThreads), lds, stream, p, plan, parts,
+                     groups);
+  return hipGetLastError() == hipSuccess ? SLORA_OK : SLORA_ERR_LAUNCH;
+}
+
+template <typename T>
+int launch_small_shrink(const SegShrinkArgs& p, const int* plan, int64_t max_input_len, hipStream_t stream) {
+  const SmallGeometry g = small_geometry(p.t.n_tokens, p.t.n_requests, max_input_len);
+  // 16 rank columns per workgroup while all of them are resident at once (one per compute unit), else 32: a
+  // launch of 128 takes 5.7 us and one of 64 with 32 columns 7.2, but 384 of them 10.2 against 7.6 for 192 (loads and
+  // products alone, without the way through LDS)
+  const int64_t tiles = (p.max_rank + 15) / 16;
+  const bool narrow = tiles == 1 || ((p.t.n_tokens + kSplitRows - 1) / kSplitRows) * tiles * p.nproj <= kShrMaxGrid;
+  const bool even = p.h_in % 4096 != 0 && p.h_in % 2560 == 0;  // 5120: two chunks of 320 for every wavefront
+  if (even) return narrow ? launch_split<T, 1, 40>(p, plan, g.parts, stream) : launch_split<T, 2, 40>(p, plan, g.parts, stream);
+  return narrow ? launch_split<T, 1, 64>(p, plan, g.parts, stream) : launch_split<T, 2, 64>(p, plan, g.parts, stream);
+}
+
+// Which of those batches expand from the plan's spans.  A span reads its B^T pages for 32 rows, the walking kernel
+// for all rows of a request that it owns: us per launch (one projection / q, k and v), spans against walk, hidden 4096:
+// 64 tokens of rank 8 4.8 / 6.1 against 5.4 / 6.0, 1024 tokens of rank 8 8.1 / 14.7 against 8.7 / 15.7, of rank 32
+// 8.6 / 15.8 against 8.7 / 16.7, 512 of rank 64 6.7 / 12.2 against 7.4 / 13.0; beyond the line 1024 of rank 64 11.1 / 21.8
+// against 11.7 / 18.6.
+bool small_expand(int64_t n_tokens, int64_t n_requests, int64_t max_rank) {
+  return small_batch(n_tokens, n_requests, max_rank) && n_tokens * max_rank <= 32 * 1024;
+}
+
+template <typename T, int KS>
+int launch_span(const SegExpandArgs& p, const int* plan, const SmallGeometry& g, hipStream_t stream) {
+  const int per_xcd = (p.n_chunks + 7) / 8;
+  const int64_t grid = (int64_t)g.spans * per_xcd * 8;
+  if (grid > 0x7fffffffLL) return SLORA_ERR_UNSUPPORTED;
+  hipLaunchKernelGGL((sgmm_expand_span_kernel<T, KS>), dim3((uint32_t)grid), dim3(kExpThreads), 0, stream, p, plan,
+                     g.parts, g.spans, per_xcd);
+  return hipGetLastError() == hipSuccess ? SLORA_OK : SLORA_ERR_LAUNCH;
+}
+
+template <typename T>
+int launch_small_expand(const SegExpandArgs& p, const int* plan, int64_t max_input_len, hipStream_t stream) {
+  const SmallGeometry g = small_geometry(p.t.n_tokens, p.t.n_requests, max_input_len);
+  if (p.max_rank <= 32) return launch_span<T, 1>(p, plan, g, stream);
+  if (p.max_rank <= 64) return launch_span<T, 2>(p, plan, g, stream);
+  return launch_span<T, 4>(p, plan, g, stream);
 }
 
 // DEEP: the instantiation whose single-projection K loop keeps three blocks in flight (for
@@ -1776,6 +2262,12 @@ int seg_shrink_common(const int* plan, bool planned, void* const o[3], int nproj
   p.col_split = 1;
   p.vec_ok = (h_in % 8 == 0) && (x_row_stride % 8 == 0) && (w_row_stride % 8 == 0) && aligned16(x) && aligned16(w);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  if (small_batch(n_tokens, n_requests, max_rank)) {
+    if (p.vec_ok && (h_in & 63) == 0)
+      return dtype == SLORA_DTYPE_F16 ? launch_small_shrink<F16>(p, plan, max_input_len, s)
+                                      : launch_small_shrink<BF16>(p, plan, max_input_len, s);
+    plan = nullptr;  // a small batch's plan is for that kernel only
+  }
   if (nproj == 3)
     return dtype == SLORA_DTYPE_F16 ? launch_seg_shrink<F16, 3, false>(p, plan, s)
                                     : launch_seg_shrink<BF16, 3, false>(p, plan, s);
@@ -1788,7 +2280,7 @@ int seg_shrink_common(const int* plan, bool planned, void* const o[3], int nproj
 
 // One projection (nproj 1: o[0], x[0], feat_out[0], o_row_stride[0], any qkvo) or q, k and v in one
 // launch (nproj 3, qkvo 0): the output groups of the three projections side by side in one grid.
-int seg_expand_common(void* const o[3], const void* const x[3], int nproj, const void* w, const slora_tables* tables,
+int seg_expand_common(const int* plan, void* const o[3], const void* const x[3], int nproj, const void* w, const slora_tables* tables,
                       const void* scales, int scales_dtype, const int32_t* b_start_loc, const int32_t* b_seq_len,
                       const int64_t* b_indicies, int64_t n_requests, int64_t max_input_len, int64_t n_tokens,
                       const int64_t feat_out[3], int64_t page_elems, int64_t max_rank, int64_t x_row_stride,
@@ -1855,6 +2347,9 @@ int seg_expand_common(void* const o[3], const void* const x[3], int nproj, const
   p.row_cap = max_input_len > (1 << 30) ? (1 << 30) : (int)((max_input_len + kExpTMW - 1) / kExpTMW * kExpTMW);
   p.m_tiles = (int)((max_input_len + p.m_span - 1) / p.m_span);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  if (plan != nullptr && small_expand(n_tokens, n_requests, max_rank))
+    return dtype == SLORA_DTYPE_F16 ? launch_small_expand<F16>(p, plan, max_input_len, s)
+                                    : launch_small_expand<BF16>(p, plan, max_input_len, s);
   return dtype == SLORA_DTYPE_F16 ? launch_seg_expand<F16>(p, s) : launch_seg_expand<BF16>(p, s);
 }
 
@@ -1874,7 +2369,7 @@ int slora_sgmm_shrink(void* o, const void* x, const void* w, const slora_tables*
 }
 
 int64_t slora_sgmm_plan_bytes(void) {
-  return (int64_t)sizeof(int) * (slora::kSegPlanHeaderWords + slora::kShrMaxGrid * slora::kSegPartWords);
+  return (int64_t)sizeof(int) * (slora::kSegPlanHeaderWords + 2 * slora::kSegMaxParts * slora::kSegPartWords);
 }
 
 int slora_sgmm_plan_build(void* plan, int64_t plan_bytes, const slora_tables* tables, const int32_t* b_start_loc,
@@ -1895,6 +2390,15 @@ int slora_sgmm_plan_build(void* plan, int64_t plan_bytes, const slora_tables* ta
   if (t.n_adapters == 0) return SLORA_OK;
   if (max_input_len > n_tokens) max_input_len = n_tokens;
   const int64_t m_tiles = (max_input_len + kShrTM - 1) / kShrTM;
+  if (small_batch(n_tokens, n_requests, max_rank)) {
+    const SmallGeometry g = small_geometry(n_tokens, n_requests, max_input_len);
+    hipLaunchKernelGGL(sgmm_plan_small_kernel, dim3(1), dim3(kSegMaxReqs), 0, reinterpret_cast<hipStream_t>(stream),
+                       static_cast<int*>(plan), t, g.parts, g.spans, kExpTMW, (int)max_rank, (int)(m_tiles * kShrTM),
+                       (int)((max_input_len + kExpTMW - 1) / kExpTMW * kExpTMW));
+    if (hipGetLastError() != hipSuccess) return SLORA_ERR_LAUNCH;
+    *usable = 1;
+    return SLORA_OK;
+  }
   int64_t grid = 0;
   int cs = 1;
   shrink_geometry(n_tokens, n_requests, m_tiles, max_rank, grid, cs);
@@ -1938,7 +2442,7 @@ int slora_sgmm_expand(void* o, const void* x, const void* w, const slora_tables*
   void* const os[3] = {o, nullptr, nullptr};
   const void* const xs[3] = {x, nullptr, nullptr};
   const int64_t feats[3] = {feat_out, 0, 0}, o_strides[3] = {o_row_stride, 0, 0};
-  return slora::seg_expand_common(os, xs, 1, w, tables, scales, scales_dtype, b_start_loc, b_seq_len, b_indicies,
+  return slora::seg_expand_common(nullptr, os, xs, 1, w, tables, scales, scales_dtype, b_start_loc, b_seq_len, b_indicies,
                                   n_requests, max_input_len, n_tokens, feats, page_elems, max_rank, x_row_stride,
                                   w_row_stride, o_strides, n_pages, qkvo, dtype, stream);
 }
@@ -1954,9 +2458,29 @@ int slora_sgmm_expand_qkv(void* o_q, void* o_k, void* o_v, const void* x_q, cons
   const void* const xs[3] = {x_q, x_k, x_v};
   const int64_t feats[3] = {feat_out_q, feat_out_kv, feat_out_kv};
   const int64_t o_strides[3] = {o_row_stride_q, o_row_stride_kv, o_row_stride_kv};
-  return slora::seg_expand_common(os, xs, 3, w, tables, scales, scales_dtype, b_start_loc, b_seq_len, b_indicies,
+  return slora::seg_expand_common(nullptr, os, xs, 3, w, tables, scales, scales_dtype, b_start_loc, b_seq_len, b_indicies,
                                   n_requests, max_input_len, n_tokens, feats, page_elems, max_rank, x_row_stride,
                                   w_row_stride, o_strides, n_pages, 0, dtype, stream);
+}
+
+int slora_sgmm_expand_planned(const void* plan, int nproj, void* o0, void* o1, void* o2, const void* x0, const void* x1,
+                              const void* x2, const void* w, const slora_tables* tables, const void* scales,
+                              int scales_dtype, const int32_t* b_start_loc, const int32_t* b_seq_len,
+                              const int64_t* b_indicies, int64_t n_requests, int64_t max_input_len, int64_t n_tokens,
+                              int64_t feat_out0, int64_t feat_out12, int64_t page_elems, int64_t max_rank,
+                              int64_t x_row_stride, int64_t w_row_stride, int64_t o_row_stride0, int64_t o_row_stride12,
+                              int64_t n_pages, int qkvo, int dtype, void* stream) {
+  if (plan == nullptr) return SLORA_ERR_NULL_POINTER;
+  if ((reinterpret_cast<uintptr_t>(plan) & 15) != 0) return SLORA_ERR_ALIGNMENT;
+  if ((nproj != 1 && nproj != 3) || (nproj == 3 && qkvo != 0)) return SLORA_ERR_BAD_SHAPE;
+  void* const os[3] = {o0, o1, o2};
+  const void* const xs[3] = {x0, x1, x2};
+  const int64_t feats[3] = {feat_out0, feat_out12, feat_out12};
+  const int64_t o_strides[3] = {o_row_stride0, o_row_stride12, o_row_stride12};
+  return slora::seg_expand_common(static_cast<const int*>(plan), os, xs, nproj, w, tables, scales, scales_dtype,
+                                  b_start_loc, b_seq_len, b_indicies, n_requests, max_input_len, n_tokens, feats,
+                                  page_elems, max_rank, x_row_stride, w_row_stride, o_strides, n_pages, qkvo, dtype,
+                                  stream);
 }
 
 }  // extern "C"

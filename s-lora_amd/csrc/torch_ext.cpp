@@ -737,6 +737,26 @@ class PrefillPlanCache {
     ++builds_;
     return slot->plan;
   }
+  // The plan the shrink calls of this step built, if it is still there: nothing is built and nothing counted.
+  std::shared_ptr<SgmmPlan> find(const Tensor& b_lora_start, const Tensor& b_lora_ranks, const Tensor& b_start_loc,
+                                 const Tensor& b_seq_len, const Tensor& b_indicies, int64_t n_tokens, int64_t max_rank,
+                                 int64_t max_input_len, void* stream) {
+    if (!g_cache_enabled) return nullptr;
+    if (!cacheable({&b_lora_start, &b_lora_ranks, &b_start_loc, &b_seq_len, &b_indicies})) return nullptr;
+    const uint64_t capture = capture_id_of(stream);
+    std::lock_guard<std::mutex> lock(mu_);
+    const Tensor* ts[5] = {&b_lora_start, &b_lora_ranks, &b_start_loc, &b_seq_len, &b_indicies};
+    const int device = b_seq_len.get_device();
+    for (const Entry& e : entries_) {
+      if (!e.plan || !e.plan->usable || e.n_tokens != n_tokens || e.max_rank != max_rank ||
+          e.max_input_len != max_input_len || e.stream != stream || e.device != device || e.capture != capture)
+        continue;
+      bool same = true;
+      for (int i = 0; i < 5 && same; ++i) same = e.ids[i].matches(*ts[i]);
+      if (same) return e.plan;
+    }
+    return nullptr;
+  }
   int64_t hits() const { return hits_; }
   int64_t builds() const { return builds_; }
   void reset_stats() { hits_ = builds_ = 0; }
@@ -842,11 +862,20 @@ void lora_get_qkvo_fwd_expand(const Tensor& x, const Tensor& w, const Tensor& o,
   const int sc = dtype_code(scale, "scale");
   TORCH_CHECK(scale.numel() >= b_lora_start.numel(), "scale must have one entry per adapter");
   TORCH_CHECK(o.size(1) >= feat_out && x.size(1) >= max_rank, "o narrower than feat_out or x narrower than max_rank");
-  const int rc = slora_sgmm_expand(o.data_ptr(), x.data_ptr(), w.data_ptr(), &t, scale.data_ptr(), sc,
-                                   b_start_loc.data_ptr<int32_t>(), b_seq_len.data_ptr<int32_t>(),
-                                   b_indicies.data_ptr<int64_t>(), b_seq_len.numel(), max_input_len, x.size(0), feat_out,
-                                   w.size(1), max_rank, x.stride(0), w.stride(0), o.stride(0), w.size(0), (int)qkvo,
-                                   dtype_code(x, "x"), stream_of(x));
+  void* stream = stream_of(x);
+  const std::shared_ptr<SgmmPlan> p = prefill_plan_cache().find(b_lora_start, b_lora_ranks, b_start_loc, b_seq_len,
+                                                                b_indicies, x.size(0), max_rank, max_input_len, stream);
+  const int code = dtype_code(x, "x");
+  const int rc =
+      p ? slora_sgmm_expand_planned(p->buf.data_ptr(), 1, o.data_ptr(), nullptr, nullptr, x.data_ptr(), nullptr, nullptr,
+                                    w.data_ptr(), &t, scale.data_ptr(), sc, b_start_loc.data_ptr<int32_t>(),
+                                    b_seq_len.data_ptr<int32_t>(), b_indicies.data_ptr<int64_t>(), b_seq_len.numel(),
+                                    max_input_len, x.size(0), feat_out, 0, w.size(1), max_rank, x.stride(0), w.stride(0),
+                                    o.stride(0), 0, w.size(0), (int)qkvo, code, stream)
+        : slora_sgmm_expand(o.data_ptr(), x.data_ptr(), w.data_ptr(), &t, scale.data_ptr(), sc,
+                            b_start_loc.data_ptr<int32_t>(), b_seq_len.data_ptr<int32_t>(),
+                            b_indicies.data_ptr<int64_t>(), b_seq_len.numel(), max_input_len, x.size(0), feat_out,
+                            w.size(1), max_rank, x.stride(0), w.stride(0), o.stride(0), w.size(0), (int)qkvo, code, stream);
   if (rc != SLORA_OK)
     check_rc(rc, "lora_get_qkvo_fwd_expand",
              "(feat_out=" + std::to_string(feat_out) + " max_rank=" + std::to_string(max_rank) +
@@ -877,12 +906,22 @@ void lora_get_qkvo_fwd_expand_qkv(const Tensor& x_q, const Tensor& x_k, const Te
   TORCH_CHECK(scale.numel() >= b_lora_start.numel(), "scale must have one entry per adapter");
   TORCH_CHECK(o_q.size(1) >= feat_out_q && o_k.size(1) >= feat_out_kv && x_q.size(1) >= max_rank,
               "o narrower than feat_out or x narrower than max_rank");
-  const int rc = slora_sgmm_expand_qkv(o_q.data_ptr(), o_k.data_ptr(), o_v.data_ptr(), x_q.data_ptr(), x_k.data_ptr(),
-                                       x_v.data_ptr(), w.data_ptr(), &t, scale.data_ptr(), sc,
-                                       b_start_loc.data_ptr<int32_t>(), b_seq_len.data_ptr<int32_t>(),
-                                       b_indicies.data_ptr<int64_t>(), b_seq_len.numel(), max_input_len, x_q.size(0),
-                                       feat_out_q, feat_out_kv, w.size(1), max_rank, x_q.stride(0), w.stride(0),
-                                       o_q.stride(0), o_k.stride(0), w.size(0), dtype_code(x_q, "x"), stream_of(x_q));
+  void* stream = stream_of(x_q);
+  const std::shared_ptr<SgmmPlan> p = prefill_plan_cache().find(b_lora_start, b_lora_ranks, b_start_loc, b_seq_len,
+                                                                b_indicies, x_q.size(0), max_rank, max_input_len, stream);
+  const int code = dtype_code(x_q, "x");
+  const int rc =
+      p ? slora_sgmm_expand_planned(p->buf.data_ptr(), 3, o_q.data_ptr(), o_k.data_ptr(), o_v.data_ptr(), x_q.data_ptr(),
+                                    x_k.data_ptr(), x_v.data_ptr(), w.data_ptr(), &t, scale.data_ptr(), sc,
+                                    b_start_loc.data_ptr<int32_t>(), b_seq_len.data_ptr<int32_t>(),
+                                    b_indicies.data_ptr<int64_t>(), b_seq_len.numel(), max_input_len, x_q.size(0),
+                                    feat_out_q, feat_out_kv, w.size(1), max_rank, x_q.stride(0), w.stride(0),
+                                    o_q.stride(0), o_k.stride(0), w.size(0), 0, code, stream)
+        : slora_sgmm_expand_qkv(o_q.data_ptr(), o_k.data_ptr(), o_v.data_ptr(), x_q.data_ptr(), x_k.data_ptr(),
+                                x_v.data_ptr(), w.data_ptr(), &t, scale.data_ptr(), sc, b_start_loc.data_ptr<int32_t>(),
+                                b_seq_len.data_ptr<int32_t>(), b_indicies.data_ptr<int64_t>(), b_seq_len.numel(),
+                                max_input_len, x_q.size(0), feat_out_q, feat_out_kv, w.size(1), max_rank, x_q.stride(0),
+                                w.stride(0), o_q.stride(0), o_k.stride(0), w.size(0), code, stream);
   if (rc != SLORA_OK)
     check_rc(rc, "lora_get_qkvo_fwd_expand_qkv",
              "(feat_out_q=" + std::to_string(feat_out_q) + " feat_out_kv=" + std::to_string(feat_out_kv) +

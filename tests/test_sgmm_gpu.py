@@ -452,6 +452,62 @@ def test_prefill_shrink_above_4096_tokens(gpu, dtype, hidden, ranks, n_req, lo, 
         assert torch.all(ob[:, :o_off] == keep) and torch.all(ob[:, o_off + R:] == keep) and torch.all(ob[T:] == keep)
 
 
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("hidden,ranks,lens", [
+    (4096, [64, 8], [1, 15, 16, 17, 33]),          # one chunk of K per wavefront; rows at the edges of a part
+    (5120, [16, 40], [31, 64, 5]),                 # chunks of 320, two per wavefront; a rank that ends inside a tile
+    (2560, [8], [7]),                              # chunks of 320, one per wavefront
+    (576, [24, 8], [40, 3]),                       # a last chunk of 64; wavefronts with nothing to do
+    (8192, [128, 32], [20, 9]),                    # two chunks of 512 per wavefront; four groups of 32 columns
+    (512, [64, 32, 16, 8], [90] * 40),             # more workgroups than compute units
+    (512, [8, 16], [3] * 256),                     # as many requests as a plan describes
+])
+def test_prefill_small_batches(gpu, dtype, hidden, ranks, lens):
+    """The kernels of small batches (K split over the wavefronts in the shrink, plan spans in the expand)
+    against the oracle, and the expand with a plan bit for bit the one without."""
+    import slora_hip
+    from slora_hip import (lora_get_qkvo_fwd_expand, lora_get_qkvo_fwd_expand_qkv, lora_get_qkvo_fwd_shrink,
+                           lora_get_qkvo_fwd_shrink_qkv)
+    lens = np.asarray(lens, np.int32)
+    T, n = int(lens.sum()), len(lens)
+    rng = np.random.default_rng(hidden + n)
+    ids = rng.integers(0, len(ranks), size=n)
+    ids[0] = 0
+    c = make_case(hidden, hidden, ranks, batch=T, dtype=dtype, bins=np.repeat(ids, lens))
+    start_np = np.concatenate([[0], np.cumsum(lens)[:-1]]).astype(np.int32)
+    g = GpuCase(c, gpu)
+    start, ln, rq = dev(start_np, torch.int32, gpu), dev(lens, torch.int32, gpu), dev(ids, torch.int64, gpu)
+    R, max_len = max(ranks), int(lens.max())
+    t = (g.a_loc, g.a_start, g.a_len, start, ln, rq)
+    w_a, w_b = g.key.view(c.n_pages, hidden), g.value.view(c.n_pages, hidden)
+    d = [torch.full((T, R), 7.0, dtype=g.tdt, device=gpu) for _ in range(3)]
+    lora_get_qkvo_fwd_shrink_qkv(g.x, w_a, *d, *t, hidden, R, max_len)
+    plain = torch.full((T, R), 7.0, dtype=g.tdt, device=gpu)
+    lora_get_qkvo_fwd_shrink(g.x, w_a, plain, *t, hidden, 2, R, max_len, plan=False)
+    assert torch.equal(plain, d[2])
+    for p in (0, 2):
+        d_ref = O.ref_prefill_shrink(np.zeros((T, R), np.float32), c.x, c.key, c.a_loc, c.a_start, c.a_len, start_np, lens,
+                                     ids, p, R, c.dtype)
+        np.testing.assert_allclose(host(d[p]), d_ref, rtol=RTOL, atol=ATOL)
+    y0 = [torch.randn((T, hidden), device=gpu).to(g.tdt) for _ in range(3)]
+    y = [v.clone() for v in y0]
+    lora_get_qkvo_fwd_expand_qkv(*d, w_b, *y, g.scales, *t, hidden, hidden, R, max_len)
+    single = y0[1].clone()
+    lora_get_qkvo_fwd_expand(d[1], w_b, single, g.scales, *t, hidden, 1, R, max_len)
+    slora_hip.set_plan_cache_enabled(False)
+    try:
+        walk = [v.clone() for v in y0]
+        lora_get_qkvo_fwd_expand_qkv(*d, w_b, *walk, g.scales, *t, hidden, hidden, R, max_len)
+    finally:
+        slora_hip.set_plan_cache_enabled(True)
+    assert torch.equal(single, y[1])
+    for p in range(3):
+        assert torch.equal(walk[p], y[p]), p
+    y_ref = O.ref_prefill_expand(host(y0[2]), host(d[2]), c.value, c.scales, c.a_loc, c.a_start, c.a_len, start_np, lens, ids,
+                                 2, R, c.dtype)
+    np.testing.assert_allclose(host(y[2]), y_ref, rtol=RTOL, atol=ATOL)
+
+
 def test_prefill_qkv_shrink_rejects_mismatched_outputs(gpu):
     from slora_hip import lora_get_qkvo_fwd_shrink_qkv
     c = seg_case(33, 256, [16, 8], 6, 1, 50, "f16")
