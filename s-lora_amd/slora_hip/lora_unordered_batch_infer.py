@@ -31,11 +31,17 @@ import torch
 from ._kernels import (dispatch_bgmv, dispatch_bgmv_qkv_expand, dispatch_bgmv_qkv_shrink, lora_get_qkvo_fwd_expand,
                        lora_get_qkvo_fwd_expand_qkv, lora_get_qkvo_fwd_shrink, lora_get_qkvo_fwd_shrink_qkv)
 
-# lora_unordered_batch_infer.py:334: the segmented kernels serve batches with a long
-# request, adapters of rank >= 64 and at least two requests; everything else is BGMV
+# lora_unordered_batch_infer.py:334: in the reference the segmented kernels serve batches with a long
+# request, adapters of rank >= 64 and at least two requests, and everything else is BGMV
 PREFILL_MIN_SEQ_LEN = 200
 PREFILL_MIN_LORA_DIM = 64
 PREFILL_MIN_REQUESTS = 2
+# Here a prompt's rows are a matrix whatever their number: 64 tokens of rank 8 in one prompt take 35.3 us per
+# layer (hidden 4096, calls from Python) in the segmented kernels against 36.3 token by token, 1024 tokens of ranks
+# 8..64 in 4 prompts 68 against 105, 8192 in 64 prompts 208 against 584.  The limits are those of their vector paths (and of what a plan describes); beyond them the
+# per-token kernels are the faster ones.
+SEGMENTED_MAX_REQUESTS = 256
+SEGMENTED_MAX_RANK = 128
 
 
 class LoraUnorderedBatchInfer:
@@ -77,6 +83,11 @@ class LoraUnorderedBatchInfer:
         self.batch_req_bins: Optional[torch.Tensor] = None
         self.max_b_seq_len = 0
         self._bins: Optional[torch.Tensor] = None
+        # a BGMV batch of the reference whose tokens are rows of prompts: (starts, lengths), or None
+        self._prompts: Optional[tuple] = None
+        self._matrix_ranks = (0 < len(adapters) <= SEGMENTED_MAX_REQUESTS and self.max_lora_dim <= SEGMENTED_MAX_RANK and
+                              all(int(a.r) % 8 == 0 for a in adapters) and self.page_elems % 8 == 0 and
+                              self.delta_dtype == kb.dtype)
 
     # ---- per step (forward(), :44-80) -----------------------------------------------------
     def begin_step(self, b_start_loc: torch.Tensor, b_seq_len: torch.Tensor, is_prefill: bool,
@@ -99,13 +110,34 @@ class LoraUnorderedBatchInfer:
             self.use_segmented = (self.max_b_seq_len >= PREFILL_MIN_SEQ_LEN and
                                   self.max_lora_dim >= PREFILL_MIN_LORA_DIM and n_req >= PREFILL_MIN_REQUESTS)
             self._bins = self.batch_req_bins
+            self._prompts = None
+            if self._matrix_ranks and not self.use_segmented and n_tok > 0:
+                # where the rows of a prompt start follows from the lengths alone, as batch_req_bins does
+                lens = b_seq_len.to(torch.int32).contiguous()
+                self._prompts = (torch.cumsum(lens, 0, dtype=torch.int32) - lens, lens)
         else:
+            self._prompts = None
             self.batch_req_bins = None
             n_tok = n_req
             self.use_segmented = False
             self._bins = self.req_bins
         dev = self.req_bins.device
         self.delta = [torch.zeros((n_tok, self.max_lora_dim), dtype=self.delta_dtype, device=dev) for _ in range(3)]
+
+    def _segments(self, x: torch.Tensor, *outs: torch.Tensor):
+        """Index tensors and longest request for the segmented kernels, or None where the per-token
+        kernels serve the call: what they refuse (strided rows, another row count) they still refuse."""
+        ia = self.infer_adapter
+        if self.use_segmented:
+            return (ia.a_loc, ia.a_start, ia.a_len, self.b_start_loc, self.b_seq_len, self.req_bins), self.max_b_seq_len
+        if self._prompts is None or x.dim() != 2 or x.shape[1] % 64 != 0:
+            return None
+        n, dtype, dev = self._bins.shape[0], self.key_buffer[0].dtype, self.req_bins.device
+        for t in (x,) + outs:
+            if (t.dim() != 2 or t.shape[0] != n or t.dtype != dtype or t.device != dev or not t.is_contiguous() or
+                    t.shape[1] % 8 != 0 or t.shape[1] > self.page_elems or t.data_ptr() % 16 != 0):
+                return None
+        return (ia.a_loc, ia.a_start, ia.a_len, *self._prompts, self.req_bins), n
 
     # ---- q, k, v of one layer (:254-318 decode, :321-408 prefill) --------------------------
     def lora_get_qkv(self, layer_id: int, input_embs: torch.Tensor, q: torch.Tensor, cache_k: torch.Tensor,
@@ -120,25 +152,26 @@ class LoraUnorderedBatchInfer:
         outs = (q, cache_k, cache_v)
         if self.max_lora_dim == 0 or input_embs.shape[0] == 0:
             return
-        if self.use_segmented:
+        segments = self._segments(input_embs, q, cache_k, cache_v)
+        if segments is not None:
             key2, val2 = key.view(-1, self.page_elems), val.view(-1, self.page_elems)
-            seg = (ia.a_loc, ia.a_start, ia.a_len, self.b_start_loc, self.b_seq_len, self.req_bins)
+            seg, longest = segments
             hidden = int(input_embs.shape[1])
             if self.fused:
                 lora_get_qkvo_fwd_shrink_qkv(input_embs, key2, d[0], d[1], d[2], *seg, hidden, self.max_lora_dim,
-                                             self.max_b_seq_len)
+                                             longest)
             else:
                 for p in range(3):
                     lora_get_qkvo_fwd_shrink(input_embs, key2, d[p], *seg, hidden, p, self.max_lora_dim,
-                                             self.max_b_seq_len)
+                                             longest)
             if self.fused and cache_k.shape == cache_v.shape and cache_k.stride(0) == cache_v.stride(0):
                 lora_get_qkvo_fwd_expand_qkv(d[0], d[1], d[2], val2, q, cache_k, cache_v, ia.a_scaling, *seg,
                                              int(q.shape[1]), int(cache_k.shape[1]), self.max_lora_dim,
-                                             self.max_b_seq_len)
+                                             longest)
                 return
             for p in range(3):
                 lora_get_qkvo_fwd_expand(d[p], val2, outs[p], ia.a_scaling, *seg, int(outs[p].shape[1]), p,
-                                         self.max_lora_dim, self.max_b_seq_len)
+                                         self.max_lora_dim, longest)
             return
         tabs = (ia.a_start, ia.a_len, ia.a_loc, self._bins)
         if self.fused:
@@ -157,13 +190,14 @@ class LoraUnorderedBatchInfer:
         d = self.delta[0]
         if self.max_lora_dim == 0 or input.shape[0] == 0:
             return
-        if self.use_segmented:
+        segments = self._segments(input, o)
+        if segments is not None:
             key2, val2 = key.view(-1, self.page_elems), val.view(-1, self.page_elems)
-            seg = (ia.a_loc, ia.a_start, ia.a_len, self.b_start_loc, self.b_seq_len, self.req_bins)
+            seg, longest = segments
             lora_get_qkvo_fwd_shrink(input, key2, d, *seg, int(input.shape[1]), 3, self.max_lora_dim,
-                                     self.max_b_seq_len)
+                                     longest)
             lora_get_qkvo_fwd_expand(d, val2, o, ia.a_scaling, *seg, int(o.shape[1]), 3, self.max_lora_dim,
-                                     self.max_b_seq_len)
+                                     longest)
             return
         tabs = (ia.a_start, ia.a_len, ia.a_loc, self._bins)
         dispatch_bgmv(d, input, key, *tabs, 3, ia.a_scaling)

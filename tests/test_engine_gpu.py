@@ -159,6 +159,30 @@ def test_prefill_step_kernel_choice_and_results(gpu, lens, segmented):
             close(res[True][l][p], m.ref(l, p, base[l][p], xin, bins))
 
 
+@pytest.mark.parametrize("ranks,start", [
+    ({"a": 16, "b": 8}, [0, 0, 0]),     # the starts of the rows follow from the lengths, whatever b_start_loc holds
+    ({"a": 12, "b": 8}, [0, 5, 45]),    # a rank the segmented kernels have no vector path for: token by token
+])
+def test_prefill_short_prompts(gpu, ranks, start):
+    """A prefill batch that the reference's rule leaves to the per-token operator: right with any
+    starts, as there, and strided activations stay refused."""
+    from slora_hip import LoraUnorderedBatchInfer
+    m = _Model(gpu, "f16", 512, 128, 1, ranks, heads=4)
+    lens_np = np.asarray([5, 40, 17], np.int32)
+    req = ["a", "b", "a"]
+    bins = np.repeat([m.names.index(n) for n in req], lens_np)
+    eng = LoraUnorderedBatchInfer(m.ia, [m.adapters[n] for n in req])
+    eng.begin_step(torch.tensor(start, dtype=torch.int32, device=gpu), torch.from_numpy(lens_np).to(gpu), is_prefill=True)
+    assert not eng.use_segmented
+    x, base = _inputs(m, np.random.default_rng(3), int(lens_np.sum()))
+    out = _run_layers(m, eng, gpu, x, base)
+    for p in range(4):
+        close(out[0][p], m.ref(0, p, base[0][p], x[0][1] if p == 3 else x[0][0], bins))
+    wide = torch.zeros((int(lens_np.sum()), 1024), dtype=torch.float16, device=gpu)
+    with pytest.raises(RuntimeError, match="must be contiguous"):
+        eng.lora_get_o(0, wide[:, :512], wide[:, 512:].contiguous())
+
+
 def test_engine_takes_buffers_from_the_adapter_table_itself(gpu):
     """The reference's NaiveInferAdapter keeps key_buffer / value_buffer on itself
     (lora_unordered_batch_infer.py:28-30); such an object works as well."""
