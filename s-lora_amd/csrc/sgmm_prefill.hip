@@ -1064,15 +1064,16 @@ enum SegPart { PT_ROW = 0, PT_ROWS, PT_RANK, PT_START_LO, PT_START_HI, PT_ADAPTE
 // is one workgroup's chain of round trips.  Here a part is 16 rows of one request, and its
 // (projection, group of 16 * NT rank columns) pairs are workgroups of their own.  The eight
 // wavefronts share K in chunks of 8 * C elements (C 16-byte pieces: 512 elements, or 320 where the
-// hidden size is a multiple of 2560), and a wavefront requests all of a chunk -- 16 rows of x
-// and 16 * NT weight rows -- before it needs any of it: at hidden 4096 that is the whole K
-// loop, one round trip.  Each load instruction covers 1 KiB of one row.  That is what makes the
+// hidden size is a multiple of 2560), and a wavefront requests a chunk's 16 rows of x and two of its
+// tiles of 16 weight rows before it needs any of them: at hidden 4096 and rank 32 that is the whole K
+// loop in one round trip.  Each load instruction covers 1 KiB of one row.  That is what makes the
 // difference: loads that touch 8 rows by 128 bytes (the order the other kernels load in) have
 // one compute unit move about 26 GB/s, and a launch of 64 tokens of rank 8 takes 8.3 us; with
-// whole rows it takes 6.7 (14 us through the register-fed kernels below).  The rows become MFMA fragments through a strip of LDS per wavefront (pieces
-// xor-swizzled by row: no bank conflicts either way, no barrier).  The eight partial tiles are
-// summed in wavefront order through LDS: the sums do not depend on how the rows were cut into
-// parts, and q, k and v in one launch are bit for bit the three calls.
+// whole rows it takes 6.4 (14 us through the register-fed kernels).  The rows become MFMA
+// fragments through a strip of LDS per wavefront (pieces xor-swizzled by row: no bank conflicts
+// either way, no barrier).  The eight partial tiles are summed in wavefront order through LDS: the
+// sums do not depend on how the rows were cut into parts, and q, k and v in one launch are bit for
+// bit the three calls.
 constexpr int kSplitThreads = 512;
 constexpr int kSplitWaves = kSplitThreads / kWave;
 constexpr int kSplitRows = 16;
@@ -1127,7 +1128,8 @@ __device__ __forceinline__ void split_part(const SegShrinkArgs& p, unsigned char
     for (int ch = wave; own > 0 && ch < chunks; ch += kSplitWaves) {
       const int k0 = ch * 8 * C;
       const int n_pieces = (p.h_in - k0) >> 3;  // C unless the last chunk is cut short: zeros behind it
-      u32x4 x[kL], w[NT][kL];
+      constexpr int kAhead = NT < 2 ? NT : 2;  // tiles of weight rows in flight
+      u32x4 x[kL], w[kAhead][kL];
 #pragma unroll
       for (int i = 0; i < kL; ++i) {
         int row = row_of(i);
@@ -1135,8 +1137,7 @@ __device__ __forceinline__ void split_part(const SegShrinkArgs& p, unsigned char
         const int pc = piece_of(i) < n_pieces ? piece_of(i) : 0;
         x[i] = ldg16(xg + (row0 + row) * p.x_stride + k0 + pc * 8);
       }
-#pragma unroll
-      for (int t = 0; t < NT; ++t)
+      auto load_w = [&](int t) {
 #pragma unroll
         for (int i = 0; i < kL; ++i) {
           const int j = t * 16 + row_of(i);
@@ -1144,8 +1145,11 @@ __device__ __forceinline__ void split_part(const SegShrinkArgs& p, unsigned char
           const int hi = C == 64 ? __builtin_amdgcn_readlane(page_hi, j) : __shfl(page_hi, j, kWave);
           const int64_t pg = (int64_t)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
           const int pc = piece_of(i) < n_pieces ? piece_of(i) : 0;
-          w[t][i] = ldg16(wg + pg * p.w_stride + k0 + pc * 8);
+          w[t % kAhead][i] = ldg16(wg + pg * p.w_stride + k0 + pc * 8);
         }
+      };
+#pragma unroll
+      for (int t = 0; t < kAhead; ++t) load_w(t);
 #pragma unroll
       for (int i = 0; i < kL; ++i) *slot(row_of(i), piece_of(i)) = piece_of(i) < n_pieces ? x[i] : zero16();
 #pragma unroll
@@ -1153,7 +1157,8 @@ __device__ __forceinline__ void split_part(const SegShrinkArgs& p, unsigned char
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
 #pragma unroll
-        for (int i = 0; i < kL; ++i) *slot(row_of(i), piece_of(i)) = piece_of(i) < n_pieces ? w[t][i] : zero16();
+        for (int i = 0; i < kL; ++i) *slot(row_of(i), piece_of(i)) = piece_of(i) < n_pieces ? w[t % kAhead][i] : zero16();
+        if (t + kAhead < NT) load_w(t + kAhead);  // (a tile without columns of the adapter repeats pool page 0)
 #pragma unroll
         for (int s = 0; s < kL; ++s) acc[t] = mfma16<T>(x[s], *slot(lr, 4 * s + lg), acc[t]);
       }
@@ -2085,12 +2090,12 @@ bool shrink_plan_usable(int64_t n_requests, int64_t m_tiles, int64_t grid, int c
 
 // Which batches take sgmm_shrink_split_kernel.  It reads a request's weight rows once per 16 token rows, the
 // other kernels once per 64, so the line falls with the rank.  us per launch (one projection / q, k and v; hidden
-// 4096, f16, rank 64), split kernel against the register-fed ones: 512 tokens 7.2 / 10.0 against 14.2 / 30, 1024 12.5 /
-// 18.1 against 14.3 / 31.7, 2311 18.1 / 35.9 against 19 / 37; 4096 27 / 46 against 23.2 / 42.1.  A whole layer at rank
-// 32: 2311 tokens 88.6 against 100.7 us, 4096 137 against 135.
+// 4096, f16, rank 64), split kernel against the register-fed ones: 512 tokens 7.1 / 9.8 against 14.2 / 30, 1024 9.5 /
+// 13.6 against 14.3 / 31.7, 2311 14.0 / 27.8 against 19 / 37; 4096 29 / 55 against 23.2 / 42.1.  A whole layer at rank
+// 32: 2311 tokens 87 against 100.7 us, 4096 137 against 135.
 bool small_batch(int64_t n_tokens, int64_t n_requests, int64_t max_rank) {
   return n_tokens > 0 && n_tokens <= 3584 && n_requests > 0 && n_requests <= kSegMaxReqs && max_rank > 0 &&
-         n_tokens * ((max_rank + 31) / 32) <= 4608;
+         n_tokens * ((max_rank + 31) / 32) <= 6144;
 }
 
 struct SmallGeometry {
@@ -2121,14 +2126,20 @@ int launch_split(const SegShrinkArgs& p, const int* plan, int parts, hipStream_t
 template <typename T>
 int launch_small_shrink(const SegShrinkArgs& p, const int* plan, int64_t max_input_len, hipStream_t stream) {
   const SmallGeometry g = small_geometry(p.t.n_tokens, p.t.n_requests, max_input_len);
-  // 16 rank columns per workgroup while all of them are resident at once (one per compute unit), else 32: a
-  // launch of 128 takes 5.7 us and one of 64 with 32 columns 7.2, but 384 of them 10.2 against 7.6 for 192 (loads and
-  // products alone, without the way through LDS)
-  const int64_t tiles = (p.max_rank + 15) / 16;
-  const bool narrow = tiles == 1 || ((p.t.n_tokens + kSplitRows - 1) / kSplitRows) * tiles * p.nproj <= kShrMaxGrid;
+  // A workgroup fills a compute unit (LDS): the fewest rank columns each with which all are resident at once, or
+  // the most.  Rank 64: 1024 tokens 9.5 / 13.6 us with 32 / 64 columns, where 16 / 32 took 12.5 / 18.1 in two
+  // rounds of workgroups; 512 tokens 7.1 with 16 columns.
+  const int64_t tiles = (p.max_rank + 15) / 16, rows = (int64_t)g.parts * p.nproj;
+  const int nt = tiles == 1 || rows * tiles <= kShrMaxGrid ? 1 : (tiles == 2 || rows * ((tiles + 1) / 2) <= kShrMaxGrid ? 2 : 4);
   const bool even = p.h_in % 4096 != 0 && p.h_in % 2560 == 0;  // 5120: two chunks of 320 for every wavefront
-  if (even) return narrow ? launch_split<T, 1, 40>(p, plan, g.parts, stream) : launch_split<T, 2, 40>(p, plan, g.parts, stream);
-  return narrow ? launch_split<T, 1, 64>(p, plan, g.parts, stream) : launch_split<T, 2, 64>(p, plan, g.parts, stream);
+  if (even) {
+    if (nt == 1) return launch_split<T, 1, 40>(p, plan, g.parts, stream);
+    if (nt == 2) return launch_split<T, 2, 40>(p, plan, g.parts, stream);
+    return launch_split<T, 4, 40>(p, plan, g.parts, stream);
+  }
+  if (nt == 1) return launch_split<T, 1, 64>(p, plan, g.parts, stream);
+  if (nt == 2) return launch_split<T, 2, 64>(p, plan, g.parts, stream);
+  return launch_split<T, 4, 64>(p, plan, g.parts, stream);
 }
 
 // Which of those batches expand from the plan's spans.  A span reads its B^T pages for 32 rows, the walking kernel
