@@ -85,9 +85,7 @@ class LoraUnorderedBatchInfer:
         self._bins: Optional[torch.Tensor] = None
         # a BGMV batch of the reference whose tokens are rows of prompts: (starts, lengths), or None
         self._prompts: Optional[tuple] = None
-        self._matrix_ranks = (0 < len(adapters) <= SEGMENTED_MAX_REQUESTS and self.max_lora_dim <= SEGMENTED_MAX_RANK and
-                              all(int(a.r) % 8 == 0 for a in adapters) and self.page_elems % 8 == 0 and
-                              self.delta_dtype == kb.dtype)
+        self._adapters = adapters
 
     # ---- per step (forward(), :44-80) -----------------------------------------------------
     def begin_step(self, b_start_loc: torch.Tensor, b_seq_len: torch.Tensor, is_prefill: bool,
@@ -111,7 +109,9 @@ class LoraUnorderedBatchInfer:
                                   self.max_lora_dim >= PREFILL_MIN_LORA_DIM and n_req >= PREFILL_MIN_REQUESTS)
             self._bins = self.batch_req_bins
             self._prompts = None
-            if self._matrix_ranks and not self.use_segmented and n_tok > 0:
+            if (not self.use_segmented and n_tok > 0 and n_req <= SEGMENTED_MAX_REQUESTS and
+                    self.max_lora_dim <= SEGMENTED_MAX_RANK and all(int(a.r) % 8 == 0 for a in self._adapters) and
+                    self.page_elems % 8 == 0 and self.delta_dtype == self.key_buffer[0].dtype):
                 # where the rows of a prompt start follows from the lengths alone, as batch_req_bins does
                 lens = b_seq_len.to(torch.int32).contiguous()
                 self._prompts = (torch.cumsum(lens, 0, dtype=torch.int32) - lens, lens)
@@ -152,7 +152,7 @@ class LoraUnorderedBatchInfer:
         outs = (q, cache_k, cache_v)
         if self.max_lora_dim == 0 or input_embs.shape[0] == 0:
             return
-        segments = self._segments(input_embs, q, cache_k, cache_v)
+        segments = self._segments(input_embs, q, cache_k, cache_v) if self.is_prefill else None
         if segments is not None:
             key2, val2 = key.view(-1, self.page_elems), val.view(-1, self.page_elems)
             seg, longest = segments
@@ -190,7 +190,7 @@ class LoraUnorderedBatchInfer:
         d = self.delta[0]
         if self.max_lora_dim == 0 or input.shape[0] == 0:
             return
-        segments = self._segments(input, o)
+        segments = self._segments(input, o) if self.is_prefill else None
         if segments is not None:
             key2, val2 = key.view(-1, self.page_elems), val.view(-1, self.page_elems)
             seg, longest = segments
