@@ -528,9 +528,10 @@ def measure_prefill(args, torch, device, w=None, seg=None):
     flops1 = seg.flops(w, H)
     ring = "true" if T > 4096 and H % 64 == 0 else "false"   # the instantiation that streams through LDS
     for label, sweep, kname, nbytes, flops in (
-            ("shrink", shrink_sweep, f"sgmm_shrink_planned_kernel<{ty}, 1, {'true' if T <= 4096 else 'false'}, {ring}>",
+            # (batches of up to 4096 tokens: one of several kernels by tokens and rank, without a traffic figure here)
+            ("shrink", shrink_sweep, f"sgmm_shrink_planned_kernel<{ty}, 1, false, {ring}>" if T > 4096 else "sgmm_shrink",
              seg.shrink_bytes(w), flops1),
-            ("qkv_shrink", qkv_shrink_sweep, f"sgmm_shrink_planned_kernel<{ty}, 3, false, {ring}>",
+            ("qkv_shrink", qkv_shrink_sweep, f"sgmm_shrink_planned_kernel<{ty}, 3, false, {ring}>" if T > 4096 else "sgmm_shrink_qkv",
              3 * seg.shrink_bytes(w) - 2 * T * H * 2, 3 * flops1),
             ("expand", expand_sweep, f"sgmm_expand_walk_kernel<{ty}, {ks}, 1>", seg.expand_bytes(w, H), flops1),
             ("qkv_expand", qkv_expand_sweep, f"sgmm_expand_walk_kernel<{ty}, {ks}, 3>", 3 * seg.expand_bytes(w, H),
