@@ -2092,9 +2092,9 @@ bool shrink_plan_usable(int64_t n_requests, int64_t m_tiles, int64_t grid, int c
 // other kernels once per 64, so the line falls with the rank.  us per launch (one projection / q, k and v; hidden
 // 4096, f16, rank 64), split kernel against the register-fed ones: 512 tokens 7.1 / 9.8 against 14.2 / 30, 1024 9.5 /
 // 13.6 against 14.3 / 31.7, 2311 14.0 / 27.8 against 19 / 37; 4096 29 / 55 against 23.2 / 42.1.  A whole layer at rank
-// 32: 2311 tokens 87 against 100.7 us, 4096 137 against 135.
+// 32: 2311 tokens 87 against 100.7 us, 4096 137 against 135; at rank 16 4096 tokens 121 against 128.
 bool small_batch(int64_t n_tokens, int64_t n_requests, int64_t max_rank) {
-  return n_tokens > 0 && n_tokens <= 3584 && n_requests > 0 && n_requests <= kSegMaxReqs && max_rank > 0 &&
+  return n_tokens > 0 && n_tokens <= (max_rank <= 16 ? 4096 : 3584) && n_requests > 0 && n_requests <= kSegMaxReqs && max_rank > 0 &&
          n_tokens * ((max_rank + 31) / 32) <= 6144;
 }
 
