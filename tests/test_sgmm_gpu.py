@@ -508,6 +508,42 @@ def test_prefill_small_batches(gpu, dtype, hidden, ranks, lens):
     np.testing.assert_allclose(host(y[2]), y_ref, rtol=RTOL, atol=ATOL)
 
 
+@pytest.mark.parametrize("hidden,lens", [
+    (512, [5, 40, 17]),           # small batches: K split over the wavefronts
+    (520, [5, 40, 17]),           # the same fed through registers (a hidden size that is no multiple of 64)
+    (517, [5, 40, 17]),           # element by element
+    (512, [1700, 1400, 1100]),    # the LDS ring
+])
+def test_page_ids_outside_the_pool_count_as_zero_rows(gpu, hidden, lens):
+    """A rank column whose page id is outside the pool is zero, whichever shrink kernel serves the batch
+    (the per-token operator skips such a row), and the expand leaves such a page out."""
+    from slora_hip import lora_get_qkvo_fwd_shrink_qkv
+    lens = np.asarray(lens, np.int32)
+    ids = np.asarray([0, 1, 0], np.int64)
+    T, R = int(lens.sum()), 16
+    c = make_case(41, hidden, [16, 8], batch=T, dtype="f16", bins=np.repeat(ids, lens))
+    c.lens, c.ids = lens, ids
+    c.start = np.concatenate([[0], np.cumsum(lens)[:-1]]).astype(np.int32)
+    bad = [2, 16 + 15, 64 + 3]    # adapter 0: q column 2, k column 15; adapter 1: q column 3
+    g = GpuCase(c, gpu)
+    loc = c.a_loc.copy()
+    loc[bad] = [c.n_pages, -1, c.n_pages + 7]
+    g.a_loc = dev(loc, torch.int64, gpu)
+    # the oracle's view of it: those rows lie on a page of zeros
+    c.key, c.value = (np.concatenate([b, np.zeros_like(b[:1])]) for b in (c.key, c.value))
+    c.a_loc = c.a_loc.copy()
+    c.a_loc[bad] = c.n_pages
+    for p in (0, 1):
+        check(c, g, p, R, gpu)
+    t = (g.a_loc, g.a_start, g.a_len, dev(c.start, torch.int32, gpu), dev(lens, torch.int32, gpu), dev(ids, torch.int64, gpu))
+    d = [torch.full((T, R), 7.0, dtype=g.tdt, device=gpu) for _ in range(3)]
+    lora_get_qkvo_fwd_shrink_qkv(g.x, g.key.view(c.n_pages, hidden), *d, *t, hidden, R, int(lens.max()))
+    for p in range(3):
+        d_ref = O.ref_prefill_shrink(np.zeros((T, R), np.float32), c.x, c.key, c.a_loc, c.a_start, c.a_len, c.start, lens,
+                                     ids, p, R, c.dtype)
+        np.testing.assert_allclose(host(d[p]), d_ref, rtol=RTOL, atol=ATOL)
+
+
 def test_prefill_qkv_shrink_rejects_mismatched_outputs(gpu):
     from slora_hip import lora_get_qkvo_fwd_shrink_qkv
     c = seg_case(33, 256, [16, 8], 6, 1, 50, "f16")
