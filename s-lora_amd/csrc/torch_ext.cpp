@@ -681,6 +681,7 @@ class PrefillPlanCache {
     std::shared_ptr<SgmmPlan> plan;
     uint64_t used = 0;
     uint64_t capture = 0;  // as in PlanCache::Entry
+    bool for_expand = false;  // the last shrink call of these tensors took this plan
   };
   void clear() {
     std::lock_guard<std::mutex> lock(mu_);
@@ -711,6 +712,7 @@ class PrefillPlanCache {
       for (int i = 0; i < 5 && same; ++i) same = e.ids[i].matches(*ts[i]);
       if (!same) continue;
       e.used = clock_;
+      e.for_expand = true;
       ++hits_;
       streak_ = 0;
       return e.plan;
@@ -733,9 +735,23 @@ class PrefillPlanCache {
     slot->stream = stream;
     slot->device = device;
     slot->capture = capture;
+    slot->for_expand = true;
     slot->used = clock_;
     ++builds_;
     return slot->plan;
+  }
+  // A shrink call of these tensors came with plan=False or a plan of its own: what the cache holds for them
+  // may be older than their contents (that is what such callers say), so their expand calls read the tensors.
+  void opt_out(const Tensor& b_lora_start, const Tensor& b_lora_ranks, const Tensor& b_start_loc, const Tensor& b_seq_len,
+               const Tensor& b_indicies) {
+    if (!cacheable({&b_lora_start, &b_lora_ranks, &b_start_loc, &b_seq_len, &b_indicies})) return;
+    std::lock_guard<std::mutex> lock(mu_);
+    const Tensor* ts[5] = {&b_lora_start, &b_lora_ranks, &b_start_loc, &b_seq_len, &b_indicies};
+    for (Entry& e : entries_) {
+      bool same = true;
+      for (int i = 0; i < 5 && same; ++i) same = e.ids[i].matches(*ts[i]);
+      if (same) e.for_expand = false;
+    }
   }
   // The plan the shrink calls of this step built, if it is still there: nothing is built and nothing counted.
   std::shared_ptr<SgmmPlan> find(const Tensor& b_lora_start, const Tensor& b_lora_ranks, const Tensor& b_start_loc,
@@ -748,7 +764,7 @@ class PrefillPlanCache {
     const Tensor* ts[5] = {&b_lora_start, &b_lora_ranks, &b_start_loc, &b_seq_len, &b_indicies};
     const int device = b_seq_len.get_device();
     for (const Entry& e : entries_) {
-      if (!e.plan || !e.plan->usable || e.n_tokens != n_tokens || e.max_rank != max_rank ||
+      if (!e.plan || !e.plan->usable || !e.for_expand || e.n_tokens != n_tokens || e.max_rank != max_rank ||
           e.max_input_len != max_input_len || e.stream != stream || e.device != device || e.capture != capture)
         continue;
       bool same = true;
@@ -784,8 +800,10 @@ std::shared_ptr<SgmmPlan> resolve_prefill_plan(const py::object& plan, const Ten
                                  max_input_len, stream);
   } else if (py::isinstance<py::bool_>(plan)) {
     TORCH_CHECK(!plan.cast<bool>(), "plan must be an SgmmPlan, None or False");
+    prefill_plan_cache().opt_out(b_lora_start, b_lora_ranks, b_start_loc, b_seq_len, b_indicies);
   } else {
     p = plan.cast<std::shared_ptr<SgmmPlan>>();
+    prefill_plan_cache().opt_out(b_lora_start, b_lora_ranks, b_start_loc, b_seq_len, b_indicies);
     TORCH_CHECK(p->n_requests == b_seq_len.numel() && p->n_tokens == n_tokens && p->max_rank == max_rank &&
                     p->max_input_len == max_input_len,
                 what, ": the plan was built for another batch (", p->n_requests, " requests, ", p->n_tokens,

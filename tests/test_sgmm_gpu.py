@@ -345,6 +345,35 @@ def test_prefill_plan_cache_follows_the_index_tensors(gpu, prefill_plan_mode):
     assert stats()[0] == built
 
 
+def test_expand_leaves_the_cached_plan_to_callers_of_the_automatic_shrink(gpu):
+    """Index tensors written behind torch's back: a caller that says so with plan=False (or an explicit
+    plan) on its shrink calls gets an expand that reads the tensors too, whatever earlier calls cached."""
+    from slora_hip import (lora_get_qkvo_fwd_expand, lora_get_qkvo_fwd_expand_qkv, lora_get_qkvo_fwd_shrink, make_prefill_plan)
+    c = seg_case(43, 256, [16, 8], 3, 20, 20, "f16")
+    g = GpuCase(c, gpu)
+    start, lens, ids = dev(c.start, torch.int32, gpu), dev(c.lens, torch.int32, gpu), dev(c.ids, torch.int64, gpu)
+    t = (g.a_loc, g.a_start, g.a_len, start, lens, ids)
+    w_a, w_b = g.key.view(c.n_pages, c.page_elems), g.value.view(c.n_pages, c.page_elems)
+    d = torch.zeros((c.batch, 16), dtype=g.tdt, device=gpu)
+    y0 = torch.randn((c.batch, 256), device=gpu).to(g.tdt)
+    for how in ("none", "explicit"):
+        lens.copy_(dev(c.lens, torch.int32, gpu))
+        lora_get_qkvo_fwd_shrink(g.x, w_a, d, *t, 256, 0, 16, 20)                  # the cache holds a plan of these lengths
+        short = c.lens.copy()
+        short[:] = [12, 20, 5]
+        lens.data.copy_(dev(short, torch.int32, gpu))                             # (leaves the version as it is)
+        plan = make_prefill_plan(g.a_start, g.a_len, start, lens, ids, c.batch, 16, 20) if how == "explicit" else False
+        lora_get_qkvo_fwd_shrink(g.x, w_a, d, *t, 256, 0, 16, 20, plan=plan)
+        y_ref = O.ref_prefill_expand(host(y0), host(d), c.value, c.scales, c.a_loc, c.a_start, c.a_len, c.start, short, c.ids,
+                                     0, 16, c.dtype)
+        y = y0.clone()
+        lora_get_qkvo_fwd_expand(d, w_b, y, g.scales, *t, 256, 0, 16, 20)
+        fused = [y0.clone() for _ in range(3)]
+        lora_get_qkvo_fwd_expand_qkv(d, d, d, w_b, *fused, g.scales, *t, 256, 256, 16, 20)
+        np.testing.assert_allclose(host(y), y_ref, rtol=RTOL, atol=ATOL)
+        assert torch.equal(fused[0], y)
+
+
 def test_prefill_plan_of_another_batch_is_rejected(gpu):
     from slora_hip import lora_get_qkvo_fwd_shrink, make_prefill_plan
     c = seg_case(32, 256, [16, 8], 6, 1, 50, "f16")
