@@ -115,8 +115,9 @@ class LoraUnorderedBatchInfer:
                     (self.max_lora_dim > 8 or not 3072 < n_tok <= 4096) and
                     self.max_lora_dim <= SEGMENTED_MAX_RANK and all(int(a.r) % 8 == 0 for a in self._adapters) and
                     self.page_elems % 8 == 0 and self.delta_dtype == self.key_buffer[0].dtype):
-                # where the rows of a prompt start follows from the lengths alone, as batch_req_bins does
-                lens = b_seq_len.to(torch.int32).contiguous()
+                # where the rows of a prompt start follows from the lengths alone, as batch_req_bins does; like that
+                # one both are this step's own, whatever the caller writes into b_seq_len before the last layer
+                lens = b_seq_len.to(torch.int32, copy=True).contiguous()
                 self._prompts = (torch.cumsum(lens, 0, dtype=torch.int32) - lens, lens)
         else:
             self._prompts = None

@@ -1,0 +1,42 @@
+"""Which kernels LoraUnorderedBatchInfer picks for a prefill batch, and what it keeps of its caller's
+tensors, without a GPU: the engine's per-step part runs on CPU tensors, no kernel is called."""
+import pytest
+import torch
+
+
+class _Adapter:
+    def __init__(self, lora_dir, r):
+        self.lora_dir, self.r = lora_dir, r
+
+
+class _Table:
+    """What the engine asks of an adapter table: two adapters of rank r over a pool of pages."""
+
+    def __init__(self, r, width=4096, dtype=torch.float16):
+        self.adapter_dirs = ["a", "b"]
+        self.key_buffer = [torch.zeros((8, width // 64, 64), dtype=dtype)]
+        self.value_buffer = [torch.zeros((8, width // 64, 64), dtype=dtype)]
+        self.a_loc = torch.arange(8 * r, dtype=torch.long) % 8
+        self.a_start = torch.tensor([0, 4 * r])
+        self.a_len = torch.tensor([4 * r, 4 * r])
+        self.a_scaling = torch.ones(2, dtype=torch.float16)
+
+
+def engine(lens, r, width=4096, dtype=torch.float16, **kw):
+    from slora_hip import LoraUnorderedBatchInfer
+    eng = LoraUnorderedBatchInfer(_Table(r, width, dtype), [_Adapter("ab"[i % 2], r) for i in range(len(lens))])
+    b_seq_len = torch.tensor(lens, dtype=torch.int32)
+    eng.begin_step(torch.cumsum(b_seq_len, 0, dtype=torch.int32) - b_seq_len, b_seq_len, True, **kw)
+    return eng, b_seq_len
+
+
+@pytest.mark.parametrize("known", [False, True])
+def test_a_step_keeps_its_own_lengths(known):
+    """Lengths advanced in place between two layers (a server preparing its next step) do not reach the
+    step that is running: its rows were laid out by begin_step."""
+    lens = [300, 200, 500, 600]
+    eng, b_seq_len = engine(lens, 32, **({"max_b_seq_len": 600, "total_token_num": 1600} if known else {}))
+    starts, kept = eng._prompts
+    b_seq_len += 1
+    assert kept.tolist() == lens and starts.tolist() == [0, 300, 500, 1000]
+    assert eng.batch_req_bins.tolist() == [0] * 300 + [1] * 200 + [0] * 500 + [1] * 600
