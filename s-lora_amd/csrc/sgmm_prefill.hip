@@ -1415,6 +1415,7 @@ __global__ __launch_bounds__(kShrThreads) void sgmm_plan_kernel(int* plan, SegTa
     plan[SP_MAXRANK] = max_rank;
     plan[SP_ROWCAP] = row_cap;
     plan[SP_STATUS] = 0;
+    plan[SP_SPANS] = 0;
   }
 }
 

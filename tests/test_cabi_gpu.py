@@ -234,3 +234,46 @@ def test_a_prefill_plan_of_another_batch_does_nothing_and_says_so(hip):
                                  0, R, dtype)
     np.testing.assert_allclose(o_gpu, o_ref, rtol=RTOL, atol=ATOL)
     assert lib.slora_plan_status(plan, C.byref(status), None) == A.OK and status.value == 0
+
+
+def _sgmm_case(hip, seed, H, ranks, lens, dtype="f16"):
+    """Device copies of a prefill case: what the segmented entry points take."""
+    import cabi_ctypes as A
+    lens = np.asarray(lens, np.int32)
+    ids = np.arange(len(lens)) % len(ranks)
+    c = make_case(seed, H, ranks, int(lens.sum()), dtype=dtype, bins=np.repeat(ids, lens))
+    c.start, c.lens, c.ids = np.concatenate([[0], np.cumsum(lens)[:-1]]).astype(np.int32), lens, ids.astype(np.int64)
+    c.d_key, c.d_val = hip.upload(to_bits(c.key, dtype)), hip.upload(to_bits(c.value, dtype))
+    c.tables = A.SloraTables(hip.upload(c.a_start.astype(np.int64)), hip.upload(c.a_len.astype(np.int64)),
+                             hip.upload(c.a_loc.astype(np.int64)), len(ranks), int(c.a_loc.size))
+    c.seg = (hip.upload(c.start), hip.upload(lens), hip.upload(c.ids))
+    c.scal, c.d_x = hip.upload(c.scales.astype(np.float16)), hip.upload(to_bits(c.x, dtype))
+    return c
+
+
+def test_an_expand_does_not_take_what_an_older_plan_left_in_the_buffer(hip):
+    """A plan buffer that is built for a small batch and then for a launch that describes no spans: an
+    expand of the small batch's shape leaves its output alone and sets the status word, also where the
+    two launches have as many row parts."""
+    import cabi_ctypes as A
+    lib = A.load_library()
+    H, R = 512, 32
+    c = _sgmm_case(hip, 25, H, [32, 16], [250] * 4)
+    T, n = 1000, 4
+    nbytes = lib.slora_sgmm_plan_bytes()
+    plan = hip.upload(np.zeros(nbytes // 4, np.int32))
+    usable, status = C.c_int(0), C.c_int(-1)
+    delta = hip.upload(to_bits(O.round_to(np.random.default_rng(3).standard_normal((T, R)).astype(np.float32), "f16"), "f16"))
+    y = hip.upload(np.full((T, H), 0x3c00, np.uint16))
+    n_parts = []
+    for max_rank in (R, 256):   # 1000 tokens of rank 32 are a small batch, of rank 256 they are not
+        rc = lib.slora_sgmm_plan_build(plan, nbytes, C.byref(c.tables), *c.seg, n, 250, T, max_rank, C.byref(usable), None)
+        assert rc == A.OK and usable.value == 1
+        n_parts.append(int(hip.download(plan, (16,), np.int32)[1]))
+    assert n_parts[0] == n_parts[1]   # the case this test is about
+    print("c-abi expand with a buffer that held a plan of its shape before", flush=True)
+    rc = lib.slora_sgmm_expand_planned(plan, 1, y, None, None, delta, None, None, c.d_val, C.byref(c.tables), c.scal, A.DTYPE_F16,
+                                       *c.seg, n, 250, T, H, 0, H, R, R, H, H, 0, c.n_pages, 0, A.DTYPE_F16, None)
+    assert rc == A.OK, A.strerror(rc)
+    assert np.all(hip.download(y, (T, H), np.uint16) == 0x3c00)
+    assert lib.slora_plan_status(plan, C.byref(status), None) == A.OK and status.value == 1
