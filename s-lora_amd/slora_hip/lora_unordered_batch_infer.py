@@ -128,13 +128,19 @@ class LoraUnorderedBatchInfer:
         dev = self.req_bins.device
         self.delta = [torch.zeros((n_tok, self.max_lora_dim), dtype=self.delta_dtype, device=dev) for _ in range(3)]
 
-    def _segments(self, x: torch.Tensor, *outs: torch.Tensor):
+    def _segments(self, key: torch.Tensor, val: torch.Tensor, x: torch.Tensor, *outs: torch.Tensor):
         """Index tensors and longest request for the segmented kernels, or None where the per-token
-        kernels serve the call: what they refuse (strided rows, another row count) they still refuse."""
+        kernels serve the call: what they refuse (strided rows or pools, another row count) they still
+        refuse, and what only they take (tables that are not 1-D, pools of two page widths) they still take."""
         ia = self.infer_adapter
         if self.use_segmented:
             return (ia.a_loc, ia.a_start, ia.a_len, self.b_start_loc, self.b_seq_len, self.req_bins), self.max_b_seq_len
         if self._prompts is None or x.dim() != 2 or x.shape[1] % 64 != 0:
+            return None
+        for pool in (key, val):
+            if pool.dim() != 3 or pool.shape[1] * pool.shape[2] != self.page_elems or not pool.is_contiguous():
+                return None
+        if ia.a_loc.dim() != 1 or ia.a_start.dim() != 1 or ia.a_len.dim() != 1:
             return None
         n, dtype, dev = self._bins.shape[0], self.key_buffer[0].dtype, self.req_bins.device
         for t in (x,) + outs:
@@ -156,7 +162,7 @@ class LoraUnorderedBatchInfer:
         outs = (q, cache_k, cache_v)
         if self.max_lora_dim == 0 or input_embs.shape[0] == 0:
             return
-        segments = self._segments(input_embs, q, cache_k, cache_v) if self.is_prefill else None
+        segments = self._segments(key, val, input_embs, q, cache_k, cache_v) if self.is_prefill else None
         if segments is not None:
             key2, val2 = key.view(-1, self.page_elems), val.view(-1, self.page_elems)
             seg, longest = segments
@@ -194,7 +200,7 @@ class LoraUnorderedBatchInfer:
         d = self.delta[0]
         if self.max_lora_dim == 0 or input.shape[0] == 0:
             return
-        segments = self._segments(input, o) if self.is_prefill else None
+        segments = self._segments(key, val, input, o) if self.is_prefill else None
         if segments is not None:
             key2, val2 = key.view(-1, self.page_elems), val.view(-1, self.page_elems)
             seg, longest = segments

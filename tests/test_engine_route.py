@@ -40,3 +40,27 @@ def test_a_step_keeps_its_own_lengths(known):
     b_seq_len += 1
     assert kept.tolist() == lens and starts.tolist() == [0, 300, 500, 1000]
     assert eng.batch_req_bins.tolist() == [0] * 300 + [1] * 200 + [0] * 500 + [1] * 600
+
+
+def segments(eng, rows, layer=0):
+    x, q, k, v = (torch.zeros((rows, eng.page_elems), dtype=eng.delta_dtype) for _ in range(4))
+    return eng._segments(eng.key_buffer[layer], eng.value_buffer[layer], x, q, k, v)
+
+
+def test_tables_and_pools_the_segmented_kernels_do_not_take_stay_with_the_per_token_operator():
+    """What the per-token operator accepts (tables of any number of dimensions, a value pool of another page
+    width) it still serves; what it refuses (a pool that is not contiguous) reaches it and is refused."""
+    lens = [300, 200, 500, 600]
+    eng, _ = engine(lens, 32)
+    assert segments(eng, 1600) is not None
+    for field in ("a_loc", "a_start", "a_len"):
+        eng, _ = engine(lens, 32)
+        setattr(eng.infer_adapter, field, getattr(eng.infer_adapter, field).view(2, -1))
+        assert segments(eng, 1600) is None, field
+    eng, _ = engine(lens, 32)
+    eng.value_buffer[0] = torch.zeros((8, 16, 64), dtype=torch.float16)
+    assert segments(eng, 1600) is None
+    for buffers in ("key_buffer", "value_buffer"):
+        eng, _ = engine(lens, 32)
+        getattr(eng, buffers)[0] = torch.zeros((8, 128, 64), dtype=torch.float16)[:, :64]
+        assert segments(eng, 1600) is None, buffers
