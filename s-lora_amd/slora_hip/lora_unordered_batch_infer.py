@@ -109,10 +109,7 @@ class LoraUnorderedBatchInfer:
                                   self.max_lora_dim >= PREFILL_MIN_LORA_DIM and n_req >= PREFILL_MIN_REQUESTS)
             self._bins = self.batch_req_bins
             self._prompts = None
-            # (at rank 8 the two are level between 3072 tokens and the large batches' kernels: 4096 tokens in 32 prompts
-            # 117 us per layer token by token, 119 otherwise)
             if (not self.use_segmented and n_tok > 0 and n_req <= SEGMENTED_MAX_REQUESTS and
-                    (self.max_lora_dim > 8 or not 3072 < n_tok <= 4096) and
                     self.max_lora_dim <= SEGMENTED_MAX_RANK and all(int(a.r) % 8 == 0 for a in self._adapters) and
                     self.page_elems % 8 == 0 and self.delta_dtype == self.key_buffer[0].dtype):
                 # where the rows of a prompt start follows from the lengths alone, as batch_req_bins does; like that

@@ -64,3 +64,10 @@ def test_tables_and_pools_the_segmented_kernels_do_not_take_stay_with_the_per_to
         eng, _ = engine(lens, 32)
         getattr(eng, buffers)[0] = torch.zeros((8, 128, 64), dtype=torch.float16)[:, :64]
         assert segments(eng, 1600) is None, buffers
+
+
+@pytest.mark.parametrize("tokens", [2311, 3073, 3500, 4096, 4097])
+def test_prefill_of_rank_8_has_one_route(tokens):
+    """The same kernels serve a handful of rank-8 prompts on both sides of 3072 and of 4096 tokens."""
+    eng, _ = engine([tokens // 4, tokens // 4, tokens // 4, tokens - 3 * (tokens // 4)], 8)
+    assert segments(eng, tokens) is not None
