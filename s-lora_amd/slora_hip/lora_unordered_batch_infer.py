@@ -36,12 +36,45 @@ from ._kernels import (dispatch_bgmv, dispatch_bgmv_qkv_expand, dispatch_bgmv_qk
 PREFILL_MIN_SEQ_LEN = 200
 PREFILL_MIN_LORA_DIM = 64
 PREFILL_MIN_REQUESTS = 2
-# Here a prompt's rows are a matrix whatever their number: 64 tokens of rank 8 in one prompt take 35.3 us per
-# layer (hidden 4096, calls from Python) in the segmented kernels against 36.3 token by token, 1024 tokens of ranks
-# 8..64 in 4 prompts 68 against 105, 8192 in 64 prompts 208 against 584.  The limits are those of their vector paths (and of what a plan describes); beyond them the
-# per-token kernels are the faster ones.
+# Beyond these the segmented kernels have no plan or no vector path, and such batches stay with BGMV
 SEGMENTED_MAX_REQUESTS = 256
 SEGMENTED_MAX_RANK = 128
+
+
+def segmented_pays(n_tok: int, n_req: int, max_rank: int, hidden: int) -> bool:
+    """Whether the segmented kernels are the faster ones for a prefill batch.
+
+    Their four launches of a layer cost the same however few rows there are, plus a share per 16 rows of each
+    prompt; the per-token ones cost least at one token and grow with tokens times rank.  us per layer, token
+    by token against segmented (f16, calls from Python, prompts of equal length):
+
+    ====================  ==================  ==================  ==================  ==================
+    prompts x tokens      4096, rank 8        4096, rank 16       4096, rank 64       8192, rank 64
+    ====================  ==================  ==================  ==================  ==================
+    1 x 1                  15.0 /  21.2        14.8 /  21.9        16.2 /  24.1        21.1 /  30.3
+    1 x 16                 22.4 /  23.0        22.2 /  23.1        24.7 /  25.7        34.4 /  31.9
+    1 x 64                 24.8 /  24.0        25.2 /  24.5        32.7 /  27.2        45.3 /  33.5
+    4 x 16                 21.9 /  23.5        22.8 /  23.9        27.6 /  26.8        41.8 /  33.3
+    16 x 4                 22.2 /  24.5        23.3 /  25.2        29.2 /  35.4        43.7 /  51.1
+    64 x 16                41.6 /  47.8        55.2 /  52.5       142.8 /  96.5       245.7 / 142.2
+    256 x 1                27.9 /  82.5        32.9 /  89.0        71.8 / 183.2       114.9 / 256.8
+    ====================  ==================  ==================  ==================  ==================
+
+    A prompt of fewer rows than a part of 16 pays for the whole part: 16 rows per prompt.  Wide rows (5120 and
+    8192) make a token dearer than a launch: up to eight prompts from four rows (8 x 4 tokens of ranks 8 / 64 at
+    hidden 5120: 0.86 / 1.01 of the per-token time; 16 x 4: 0.93 / 1.14).  Narrow rows of low rank are so cheap per
+    token that several prompts need enough of them.  Rank 16: 256 tokens (8 x 16: 1.07, 8 x 32: 1.00, 4 x 64:
+    0.98).  Rank 8: about 1000 tokens in prompts of 64 (64 x 36: 1.18, 64 x 56: 0.98, 64 x 66: 0.94, 100 x 40: 1.20),
+    or of 40 where the kernels of more than 4096 tokens run (100 x 48: 1.00, 128 x 40: 0.97, 200 x 33: 1.06, 200 x 40:
+    0.92); above 8192 tokens the per-token operator's plan costs milliseconds a step (256 x 33, a step of 8 layers:
+    6.6 ms against 1.7).  Hidden 1024 and 2048 and bf16 measure the same or better for the segmented kernels."""
+    if hidden > 4096 and n_req <= 8:
+        return n_tok >= 4 * n_req
+    if hidden > 4096 or n_req == 1 or max_rank > 16:
+        return n_tok >= 16 * n_req
+    if max_rank > 8:
+        return n_tok >= max(256, 16 * n_req)
+    return n_tok > 8192 or n_tok >= max(1024, (40 if n_tok > 4096 else 64) * n_req)
 
 
 class LoraUnorderedBatchInfer:
@@ -110,6 +143,7 @@ class LoraUnorderedBatchInfer:
             self._bins = self.batch_req_bins
             self._prompts = None
             if (not self.use_segmented and n_tok > 0 and n_req <= SEGMENTED_MAX_REQUESTS and
+                    segmented_pays(n_tok, n_req, self.max_lora_dim, self.page_elems) and
                     self.max_lora_dim <= SEGMENTED_MAX_RANK and all(int(a.r) % 8 == 0 for a in self._adapters) and
                     self.page_elems % 8 == 0 and self.delta_dtype == self.key_buffer[0].dtype):
                 # where the rows of a prompt start follows from the lengths alone, as batch_req_bins does; like that

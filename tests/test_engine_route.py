@@ -71,3 +71,17 @@ def test_prefill_of_rank_8_has_one_route(tokens):
     """The same kernels serve a handful of rank-8 prompts on both sides of 3072 and of 4096 tokens."""
     eng, _ = engine([tokens // 4, tokens // 4, tokens // 4, tokens - 3 * (tokens // 4)], 8)
     assert segments(eng, tokens) is not None
+
+
+@pytest.mark.parametrize("width,r,prompts,rows,segmented", [
+    (4096, 8, 1, 1, False), (4096, 64, 1, 1, False), (8192, 8, 1, 1, False), (8192, 64, 1, 1, False),  # one short prompt
+    (4096, 8, 1, 15, False), (4096, 8, 1, 16, True), (4096, 64, 1, 16, True),
+    (4096, 8, 4, 255, False), (4096, 8, 4, 256, True), (4096, 8, 16, 64, True), (4096, 8, 32, 63, False),
+    (4096, 8, 100, 40, False), (4096, 8, 128, 40, True), (4096, 8, 200, 39, False), (4096, 8, 256, 33, True),
+    (4096, 16, 4, 63, False), (4096, 16, 4, 64, True), (4096, 16, 64, 15, False), (4096, 16, 64, 16, True),
+    (4096, 64, 4, 15, False), (4096, 64, 4, 16, True), (4096, 64, 200, 2, False), (4096, 64, 256, 1, False),
+    (5120, 8, 8, 3, False), (5120, 8, 8, 4, True), (8192, 64, 9, 15, False), (8192, 64, 9, 16, True), (8192, 8, 256, 4, False),
+])
+def test_short_prompts_stay_token_by_token(width, r, prompts, rows, segmented):
+    eng, _ = engine([rows] * prompts, r, width, max_b_seq_len=rows, total_token_num=prompts * rows)
+    assert not eng.use_segmented and (segments(eng, prompts * rows) is not None) == segmented
