@@ -116,6 +116,7 @@ class LoraUnorderedBatchInfer:
         self.batch_req_bins: Optional[torch.Tensor] = None
         self.max_b_seq_len = 0
         self._bins: Optional[torch.Tensor] = None
+        self._n_tok = 0
         # a BGMV batch of the reference whose tokens are rows of prompts: (starts, lengths), or None
         self._prompts: Optional[tuple] = None
         self._adapters = adapters
@@ -156,6 +157,7 @@ class LoraUnorderedBatchInfer:
             n_tok = n_req
             self.use_segmented = False
             self._bins = self.req_bins
+        self._n_tok = n_tok
         dev = self.req_bins.device
         self.delta = [torch.zeros((n_tok, self.max_lora_dim), dtype=self.delta_dtype, device=dev) for _ in range(3)]
 
@@ -166,18 +168,21 @@ class LoraUnorderedBatchInfer:
         ia = self.infer_adapter
         if self.use_segmented:
             return (ia.a_loc, ia.a_start, ia.a_len, self.b_start_loc, self.b_seq_len, self.req_bins), self.max_b_seq_len
-        if self._prompts is None or x.dim() != 2 or x.shape[1] % 64 != 0:
+        if self._prompts is None:
             return None
-        for pool in (key, val):
-            if pool.dim() != 3 or pool.shape[1] * pool.shape[2] != self.page_elems or not pool.is_contiguous():
-                return None
-        if ia.a_loc.dim() != 1 or ia.a_start.dim() != 1 or ia.a_len.dim() != 1:
+        first = self.key_buffer[0]
+        pages = first.shape
+        if (len(pages) != 3 or key.shape != pages or val.shape != pages or not key.is_contiguous() or not val.is_contiguous() or
+                ia.a_loc.dim() != 1 or ia.a_start.dim() != 1 or ia.a_len.dim() != 1):
             return None
-        n, dtype, dev = self._bins.shape[0], self.key_buffer[0].dtype, self.req_bins.device
+        n, width, dtype, dev = self._n_tok, self.page_elems, first.dtype, first.device
         for t in (x,) + outs:
-            if (t.dim() != 2 or t.shape[0] != n or t.dtype != dtype or t.device != dev or not t.is_contiguous() or
-                    t.shape[1] % 8 != 0 or t.shape[1] > self.page_elems or t.data_ptr() % 16 != 0):
+            shape = t.shape
+            if (len(shape) != 2 or shape[0] != n or shape[1] % 8 != 0 or shape[1] > width or t.dtype != dtype or
+                    t.device != dev or not t.is_contiguous() or t.data_ptr() % 16 != 0):
                 return None
+        if x.shape[1] % 64 != 0:
+            return None
         return (ia.a_loc, ia.a_start, ia.a_len, *self._prompts, self.req_bins), n
 
     # ---- q, k, v of one layer (:254-318 decode, :321-408 prefill) --------------------------

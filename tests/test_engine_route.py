@@ -60,6 +60,10 @@ def test_tables_and_pools_the_segmented_kernels_do_not_take_stay_with_the_per_to
     eng, _ = engine(lens, 32)
     eng.value_buffer[0] = torch.zeros((8, 16, 64), dtype=torch.float16)
     assert segments(eng, 1600) is None
+    eng, _ = engine(lens, 32)
+    eng.key_buffer[0] = eng.key_buffer[0].view(8, 64, 64, 1)
+    eng.value_buffer[0] = eng.value_buffer[0].view(8, 64, 64, 1)
+    assert segments(eng, 1600) is None
     for buffers in ("key_buffer", "value_buffer"):
         eng, _ = engine(lens, 32)
         getattr(eng, buffers)[0] = torch.zeros((8, 128, 64), dtype=torch.float16)[:, :64]
