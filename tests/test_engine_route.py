@@ -89,3 +89,14 @@ def test_prefill_of_rank_8_has_one_route(tokens):
 def test_short_prompts_stay_token_by_token(width, r, prompts, rows, segmented):
     eng, _ = engine([rows] * prompts, r, width, max_b_seq_len=rows, total_token_num=prompts * rows)
     assert not eng.use_segmented and (segments(eng, prompts * rows) is not None) == segmented
+
+
+def test_the_longest_prompt_is_the_one_begin_step_saw():
+    """The segmented kernels are told the longest prompt where begin_step read it from the lengths; a caller's
+    max_b_seq_len decides the reference's rule only, so that a wrong one loses no rows."""
+    lens = [300, 200, 500, 600]
+    eng, _ = engine(lens, 32)
+    assert segments(eng, 1600)[1] == 600
+    for claimed in (1, 600, 9999):
+        eng, _ = engine(lens, 32, max_b_seq_len=claimed, total_token_num=1600)
+        assert segments(eng, 1600)[1] == 1600
