@@ -1108,6 +1108,14 @@ struct SegPartRec {
   int64_t start;
 };
 
+// Between accesses of a wavefront's lanes to each other's LDS words: what is written before is read after.  The
+// LDS serves a wavefront in order, so this only binds the compiler and costs no instruction.
+__device__ __forceinline__ void strip_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 // All threads of the workgroup: one part, rank columns nb .. + 16 * NT (those below max_rank) of projection pj.
 template <typename T, int NT, int C>
 __device__ __forceinline__ void split_part(const SegShrinkArgs& p, unsigned char* s_all, const SegPartRec& rec, int pj,
@@ -1170,15 +1178,19 @@ __device__ __forceinline__ void split_part(const SegShrinkArgs& p, unsigned char
       for (int t = 0; t < kAhead; ++t) load_w(t);
 #pragma unroll
       for (int i = 0; i < kL; ++i) *slot(row_of(i), piece_of(i)) = piece_of(i) < n_pieces ? x[i] : zero16();
+      strip_sync();
 #pragma unroll
       for (int s = 0; s < kL; ++s) x[s] = *slot(lr, 4 * s + lg);
+      strip_sync();
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
 #pragma unroll
         for (int i = 0; i < kL; ++i) *slot(row_of(i), piece_of(i)) = piece_of(i) < n_pieces ? w[t % kAhead][i] : zero16();
+        strip_sync();
         if (t + kAhead < NT) load_w(t + kAhead);  // (a tile without columns of the adapter repeats pool page 0)
 #pragma unroll
         for (int s = 0; s < kL; ++s) acc[t] = mfma16<T>(x[s], *slot(lr, 4 * s + lg), acc[t]);
+        strip_sync();
       }
     }
     if (own > 0) {
