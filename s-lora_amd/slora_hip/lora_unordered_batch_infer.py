@@ -148,9 +148,12 @@ class LoraUnorderedBatchInfer:
                     self.max_lora_dim <= SEGMENTED_MAX_RANK and all(int(a.r) % 8 == 0 for a in self._adapters) and
                     self.page_elems % 8 == 0 and self.delta_dtype == self.key_buffer[0].dtype):
                 # where the rows of a prompt start follows from the lengths alone, as batch_req_bins does; like that
-                # one both are this step's own, whatever the caller writes into b_seq_len before the last layer
-                lens = b_seq_len.to(torch.int32, copy=True).contiguous()
-                self._prompts = (torch.cumsum(lens, 0, dtype=torch.int32) - lens, lens)
+                # one starts and lengths are this step's own, whatever the caller writes into b_seq_len before the
+                # last layer (lengths as a difference: a copy of a tensor is a transfer, 10 us dearer than a kernel)
+                lens = b_seq_len.to(torch.int32)
+                ends = torch.cumsum(lens, 0, dtype=torch.int32)
+                starts = ends - lens
+                self._prompts = (starts, ends - starts)
                 # the longest prompt, if it was read here: a caller's figure has only decided the rule above, where a
                 # wrong one does no harm, and no prompt is longer than the batch.  (It matters above 65536 tokens,
                 # where that bound hides that a plan could be built: 70000 tokens of rank 32 in 64 prompts 1636 us
@@ -165,7 +168,12 @@ class LoraUnorderedBatchInfer:
             self._bins = self.req_bins
         self._n_tok = n_tok
         dev = self.req_bins.device
-        self.delta = [torch.zeros((n_tok, self.max_lora_dim), dtype=self.delta_dtype, device=dev) for _ in range(3)]
+        # (one fill for all three where each starts on 16 bytes, as an allocation of its own would)
+        shape = (n_tok, self.max_lora_dim)
+        if self.max_lora_dim % 8 == 0:
+            self.delta = list(torch.zeros((3, *shape), dtype=self.delta_dtype, device=dev).unbind(0))
+        else:
+            self.delta = [torch.zeros(shape, dtype=self.delta_dtype, device=dev) for _ in range(3)]
 
     def _segments(self, key: torch.Tensor, val: torch.Tensor, x: torch.Tensor, *outs: torch.Tensor):
         """Index tensors and longest request for the segmented kernels, or None where the per-token
