@@ -37,6 +37,8 @@ extern "C" {
 /* major * 100 + minor.  The major number changes when an entry point is removed or its
  * signature changes (callers built against an older major must be rebuilt), the minor one when
  * entry points are added.
+ *   2.1 (201): + slora_sgmm_expand_planned; prefill plans hold spans for it (slora_sgmm_plan_bytes
+ *              grew from 8 to 33 KB).
  *   2.0 (200): slora_bgmv_lora_planned (shrink and expand in one launch) has a new signature and a
  *              new plan layout behind it -- the 1.0 form was removed in 1.1 without a major bump,
  *              which this number corrects; plans hold hand-over counters (slora_bgmv_plan_bytes
@@ -44,7 +46,7 @@ extern "C" {
  *   1.2 (102): + slora_sgmm_expand_qkv.
  *   1.1 (101): + slora_sgmm_shrink_qkv, slora_pool_page_checksums, slora_pool_pack_transposed,
  *              slora_pool_alloc_contiguous_static; - slora_bgmv_lora_planned. */
-#define SLORA_VERSION 200
+#define SLORA_VERSION 201
 
 #define SLORA_API __attribute__((visibility("default")))
 
