@@ -110,6 +110,32 @@ def test_sgmm_argument_checks(lib):
              1024, 100, A.DTYPE_F16, None) == A.ERR_NULL_POINTER
 
 
+def test_planned_expand_argument_checks(lib):
+    import cabi_ctypes as A
+    t = _tables()
+    P = 0x10000
+    # plan nproj o0 o1 o2 x0 x1 x2 w tables scales scales_dtype b_start_loc b_seq_len b_indicies n_requests max_input_len
+    # n_tokens feat_out0 feat_out12 page_elems max_rank x_stride w_stride o_stride0 o_stride12 n_pages qkvo dtype stream
+    f = lib.slora_sgmm_expand_planned
+
+    def call(plan=P, nproj=1, o=(P, P, P), x=(P, P, P), n_req=4, max_rank=64, x_stride=64, o12=1024, qkvo=0, dtype=A.DTYPE_F16):
+        return f(plan, nproj, *o, *x, P, C.byref(t), P, A.DTYPE_F16, P, P, P, n_req, 16, 64, 4096, 1024, 4096, max_rank, x_stride,
+                 4096, 4096, o12, 100, qkvo, dtype, None)
+
+    assert call(n_req=0) == A.OK and call(n_req=0, nproj=3) == A.OK          # nothing to do
+    assert call(n_req=0, qkvo=3, o=(P, None, None), x=(P, None, None)) == A.OK
+    assert call(plan=None) == A.ERR_NULL_POINTER
+    assert call(plan=P + 8) == A.ERR_ALIGNMENT
+    assert call(nproj=2) == A.ERR_BAD_SHAPE and call(nproj=0) == A.ERR_BAD_SHAPE
+    assert call(nproj=3, qkvo=1) == A.ERR_BAD_SHAPE                          # q, k and v start at projection 0
+    assert call(qkvo=4) == A.ERR_BAD_SHAPE
+    assert call(nproj=3, o=(P, None, P)) == A.ERR_NULL_POINTER
+    assert call(nproj=3, x=(P, P, None)) == A.ERR_NULL_POINTER
+    assert call(nproj=3, o12=512) == A.ERR_BAD_SHAPE                         # o1 rows narrower than feat_out12
+    assert call(x_stride=32) == A.ERR_BAD_SHAPE                              # x rows narrower than max_rank
+    assert call(dtype=7) == A.ERR_BAD_DTYPE
+
+
 def test_python_mirror_rejects_cpu_tensors():
     """Reference behaviour: CHECK_CUDA -> RuntimeError (lora_ops.cc:29, 79-85)."""
     import torch

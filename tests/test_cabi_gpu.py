@@ -277,3 +277,180 @@ def test_an_expand_does_not_take_what_an_older_plan_left_in_the_buffer(hip):
     assert rc == A.OK, A.strerror(rc)
     assert np.all(hip.download(y, (T, H), np.uint16) == 0x3c00)
     assert lib.slora_plan_status(plan, C.byref(status), None) == A.OK and status.value == 1
+
+
+class _Segmented:
+    """The segmented entry points on one case, with a plan and without."""
+
+    def __init__(self, hip, c, R, dtype, max_len=None):
+        import cabi_ctypes as A
+        self.A, self.lib, self.hip, self.c, self.R, self.dtype = A, A.load_library(), hip, c, R, dtype
+        self.dt = A.DTYPE_F16 if dtype == "f16" else A.DTYPE_BF16
+        self.T, self.H, self.n = c.batch, c.hidden, len(c.lens)
+        self.max_len = int(c.lens.max()) if max_len is None else max_len
+        self.nbytes = self.lib.slora_sgmm_plan_bytes()
+        self.plan = hip.upload(np.zeros(self.nbytes // 4, np.int32))
+
+    def build(self):
+        """Builds the plan and returns its header; word 1: row parts, word 2: -16 for a small batch, word 8: spans."""
+        usable = C.c_int(0)
+        rc = self.lib.slora_sgmm_plan_build(self.plan, self.nbytes, C.byref(self.c.tables), *self.c.seg, self.n, self.max_len,
+                                            self.T, self.R, C.byref(usable), None)
+        assert rc == self.A.OK and usable.value == 1
+        return self.hip.download(self.plan, (16,), np.int32)
+
+    def status(self):
+        status = C.c_int(-1)
+        assert self.lib.slora_plan_status(self.plan, C.byref(status), None) == self.A.OK
+        return status.value
+
+    def shrink(self, p, planned):
+        o = self.hip.upload(np.full((self.T, self.R), 0x3c00, np.uint16))
+        f = self.lib.slora_sgmm_shrink_planned if planned else self.lib.slora_sgmm_shrink
+        rc = f(*((self.plan,) if planned else ()), o, self.c.d_x, self.c.d_key, C.byref(self.c.tables), *self.c.seg, self.n,
+               self.max_len, self.T, self.H, self.R, self.H, self.H, self.R, self.c.n_pages, p, self.dt, None)
+        assert rc == self.A.OK, self.A.strerror(rc)
+        return self.hip.download(o, (self.T, self.R), np.uint16)
+
+    def shrink_qkv(self, planned):
+        o = [self.hip.upload(np.full((self.T, self.R), 0x3c00, np.uint16)) for _ in range(3)]
+        rc = self.lib.slora_sgmm_shrink_qkv(self.plan if planned else None, *o, self.c.d_x, self.c.d_key, C.byref(self.c.tables),
+                                            *self.c.seg, self.n, self.max_len, self.T, self.H, self.R, self.H, self.H, self.R,
+                                            self.c.n_pages, self.dt, None)
+        assert rc == self.A.OK, self.A.strerror(rc)
+        return [self.hip.download(q, (self.T, self.R), np.uint16) for q in o]
+
+    def expand(self, y0, d, planned, p=None):
+        """Projection p, or q, k and v in one launch; y0 and d: bit patterns."""
+        y = [self.hip.upload(y0) for _ in range(3 if p is None else 1)]
+        x = [self.hip.upload(q) for q in d]
+        lib, c, H, R = self.lib, self.c, self.H, self.R
+        tail = (c.d_val, C.byref(c.tables), c.scal, self.A.DTYPE_F16, *c.seg, self.n, self.max_len, self.T)
+        if planned:
+            pad = (None,) * (3 - len(y))
+            rc = lib.slora_sgmm_expand_planned(self.plan, len(y), *y, *pad, *x, *pad, *tail, H, H, H, R, R, H, H, H, c.n_pages,
+                                               p or 0, self.dt, None)
+        elif p is None:
+            rc = lib.slora_sgmm_expand_qkv(*y, *x, *tail, H, H, H, R, R, H, H, H, c.n_pages, self.dt, None)
+        else:
+            rc = lib.slora_sgmm_expand(*y, *x, *tail, H, H, R, R, H, H, c.n_pages, p, self.dt, None)
+        assert rc == self.A.OK, self.A.strerror(rc)
+        return [self.hip.download(q, (self.T, H), np.uint16) for q in y]
+
+    def ref_shrink(self, p):
+        c = self.c
+        return O.ref_prefill_shrink(np.ones((self.T, self.R), np.float32), c.x, c.key, c.a_loc, c.a_start, c.a_len, c.start, c.lens,
+                                    c.ids, p, self.R, self.dtype)
+
+    def ref_expand(self, y0, d, p):
+        c = self.c
+        return O.ref_prefill_expand(from_bits(y0, self.dtype), from_bits(d, self.dtype), c.value, c.scales, c.a_loc, c.a_start,
+                                    c.a_len, c.start, c.lens, c.ids, p, self.R, self.dtype)
+
+
+def _random_bits(seed, shape, dtype):
+    return to_bits(O.round_to(np.random.default_rng(seed).standard_normal(shape).astype(np.float32), dtype), dtype)
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("H,ranks,lens,one,three", [
+    # `one`, `three`: tiles of 16 rank columns a workgroup of the single and of the q/k/v shrink takes
+    (4096, [64, 8], [1, 15, 16, 17, 33], 1, 1),           # rows at the edges of a part
+    (5120, [32, 16], [256] * 4, 1, 2),                    # chunks of 320 elements, two per wavefront; two tiles
+    (5120, [64, 40], [256] * 5, 2, 4),                    # the same with four tiles; ranks that end inside one
+    (2560, [48, 16, 8], [150, 17, 200, 33, 129, 1], 1, 2),   # one chunk of 320 per wavefront, the third tile alone in its group
+    (4096, [64, 24], [250] * 5, 2, 4),                    # chunks of 512; rows that end inside a part
+    (576, [64, 8], [256] * 5, 2, 4),                      # a last chunk of 64 elements; wavefronts with nothing to do
+    (8192, [128, 32], [300, 300], 2, 4),                  # two chunks of 512 per wavefront; four groups of 32 columns
+    (512, [64, 32, 16, 8], [70] * 40, 4, 4),              # more workgroups than compute units
+    (512, [16, 8], [3] * 256, 1, 1),                      # as many requests as a plan describes
+])
+def test_small_prefill_batches_through_the_c_abi(hip, dtype, H, ranks, lens, one, three):
+    """Every shape of the split-K shrink, planned and not, one projection and three, and the expand from the
+    plan's spans: bit for bit each other, and the oracle's results."""
+    R = max(ranks)
+    c = _sgmm_case(hip, H + R, H, ranks, lens, dtype)
+    g = _Segmented(hip, c, R, dtype)
+    head = g.build()
+    assert head[2] == -16                                    # a small batch
+    tiles, parts = -(-R // 16), int(head[1])
+
+    def columns(nproj):   # as few tiles per workgroup as keep the launch within 256 of them, or four
+        return next((nt for nt in (1, 2) if nt >= tiles or parts * nproj * -(-tiles // nt) <= 256), 4)
+
+    assert (columns(1), columns(3)) == (one, three)
+    print(f"c-abi small prefill {dtype} hidden {H} ranks {ranks} {len(lens)} requests", flush=True)
+    d = g.shrink_qkv(True)
+    for p in range(3):
+        np.testing.assert_allclose(from_bits(d[p], dtype), g.ref_shrink(p), rtol=RTOL, atol=ATOL)
+        assert np.array_equal(g.shrink(p, True), d[p]), p
+    assert np.array_equal(g.shrink(1, False), d[1])
+    assert all(np.array_equal(a, b) for a, b in zip(g.shrink_qkv(False), d))
+    y0 = _random_bits(7, (c.batch, H), dtype)
+    y = g.expand(y0, d, True)
+    assert all(np.array_equal(a, b) for a, b in zip(g.expand(y0, d, False), y))
+    assert np.array_equal(g.expand(y0, d[1:2], True, 1)[0], y[1]) and np.array_equal(g.expand(y0, d[1:2], False, 1)[0], y[1])
+    np.testing.assert_allclose(from_bits(y[2], dtype), g.ref_expand(y0, d[2], 2), rtol=RTOL, atol=ATOL)
+    assert g.status() == 0
+
+
+@pytest.mark.parametrize("lens,start,max_len", [
+    ([40] * 8, [0] * 8, None),         # requests that overlap in the batch: parts of 32 rows
+    ([40] * 16, [0] * 16, None),       # ... of 64
+    ([60] * 8, None, 10),              # lengths beyond max_input_len, clipped at a whole tile: one part of 60 rows each
+])
+def test_split_shrink_parts_of_more_than_16_rows(hip, lens, start, max_len):
+    H, R = 1024, 32
+    ids_one = start is not None        # overlapping requests name one adapter: all write the same values
+    c = _sgmm_case(hip, 26, H, [R] if ids_one else [R, 16], lens)
+    if ids_one:                        # the batch is the rows they share
+        c.batch, c.start = lens[0], np.asarray(start, np.int32)
+        c.x = c.x[: c.batch]
+        c.seg = (hip.upload(c.start), *c.seg[1:])
+    g = _Segmented(hip, c, R, "f16", max_len)
+    head = g.build()
+    assert head[2] == -16 and int(head[1]) < sum(-(-n // 16) for n in lens)   # fewer parts than pieces of 16 rows
+    print(f"c-abi split shrink {lens[:2]} x {len(lens)} max_len {max_len}", flush=True)
+    d = g.shrink(2, True)
+    np.testing.assert_allclose(from_bits(d, "f16"), g.ref_shrink(2), rtol=RTOL, atol=ATOL)
+    assert np.array_equal(g.shrink(2, False), d) and np.array_equal(g.shrink_qkv(True)[2], d)
+    assert g.status() == 0
+
+
+def test_expand_spans_of_more_than_32_rows(hip):
+    """Requests without an adapter's rank lie over the same rows: they take spans but touch nothing, and the one
+    request that does gets a span of all its rows."""
+    H, R, T, n = 1024, 16, 100, 8
+    c = _sgmm_case(hip, 27, H, [R, 0], [T] * n)
+    c.batch, c.start, c.ids = T, np.zeros(n, np.int32), np.array([1, 1, 0, 1, 1, 1, 1, 1], np.int64)
+    c.seg = (hip.upload(c.start), c.seg[1], hip.upload(c.ids))
+    g = _Segmented(hip, c, R, "f16")
+    head = g.build()
+    assert head[2] == -16 and int(head[8]) < n * 4           # fewer spans than pieces of 32 rows
+    y0, d = _random_bits(8, (T, H), "f16"), _random_bits(9, (T, R), "f16")
+    print("c-abi expand spans of more than 32 rows", flush=True)
+    y = g.expand(y0, [d], True, 3)[0]
+    np.testing.assert_allclose(from_bits(y, "f16"), g.ref_expand(y0, d, 3), rtol=RTOL, atol=ATOL)
+    assert np.array_equal(g.expand(y0, [d], False, 3)[0], y) and g.status() == 0
+
+
+def test_expand_with_the_plan_of_another_batch_does_nothing_and_says_so(hip):
+    """slora_sgmm_expand_planned with the plan of another batch shape leaves its output alone and sets the
+    status word; a batch too large for spans leaves the plan alone."""
+    H, R = 512, 16
+    other = _Segmented(hip, _sgmm_case(hip, 28, H, [R, 8], [30, 41]), R, "f16")
+    g = _Segmented(hip, _sgmm_case(hip, 29, H, [R, 8], [30, 41, 50]), R, "f16")
+    other.build()
+    g.plan = other.plan
+    y0, d = _random_bits(10, (g.T, H), "f16"), _random_bits(11, (g.T, R), "f16")
+    print("c-abi expand with the plan of another batch", flush=True)
+    assert g.status() == 0
+    assert np.array_equal(g.expand(y0, [d], True, 0)[0], y0) and g.status() == 1
+    assert all(np.array_equal(y, y0) for y in g.expand(y0, [d] * 3, True)) and g.status() == 1
+    g.build()
+    assert g.status() == 0
+    assert np.array_equal(g.expand(y0, [d], True, 0)[0], g.expand(y0, [d], False, 0)[0]) and g.status() == 0
+    big = _Segmented(hip, _sgmm_case(hip, 30, H, [R, 8], [1200, 1300]), R, "f16")   # 2500 tokens x 16 > 32768
+    big.plan = other.plan
+    y0, d = _random_bits(12, (big.T, H), "f16"), _random_bits(13, (big.T, R), "f16")
+    assert np.array_equal(big.expand(y0, [d], True, 0)[0], big.expand(y0, [d], False, 0)[0]) and big.status() == 0

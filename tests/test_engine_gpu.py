@@ -159,23 +159,30 @@ def test_prefill_step_kernel_choice_and_results(gpu, lens, segmented):
             close(res[True][l][p], m.ref(l, p, base[l][p], xin, bins))
 
 
-@pytest.mark.parametrize("ranks,start", [
-    ({"a": 16, "b": 8}, [0, 0, 0]),     # the starts of the rows follow from the lengths, whatever b_start_loc holds
-    ({"a": 12, "b": 8}, [0, 5, 45]),    # a rank the segmented kernels have no vector path for: token by token
+@pytest.mark.parametrize("ranks,lens,start,segmented", [
+    ({"a": 16, "b": 8}, [5, 40, 17], [0, 0, 0], False),         # too few rows to pay for the segmented launches
+    ({"a": 16, "b": 8}, [105, 140, 77], [0, 0, 0], True),       # the starts of the rows follow from the lengths, whatever b_start_loc holds
+    ({"a": 12, "b": 8}, [105, 140, 77], [0, 105, 245], False),  # a rank the segmented kernels have no vector path for: token by token
 ])
-def test_prefill_short_prompts(gpu, ranks, start):
+def test_prefill_short_prompts(gpu, ranks, lens, start, segmented):
     """A prefill batch that the reference's rule leaves to the per-token operator: right with any
     starts, as there, and strided activations stay refused."""
+    import slora_hip
     from slora_hip import LoraUnorderedBatchInfer
     m = _Model(gpu, "f16", 512, 128, 1, ranks, heads=4)
-    lens_np = np.asarray([5, 40, 17], np.int32)
+    lens_np = np.asarray(lens, np.int32)
     req = ["a", "b", "a"]
     bins = np.repeat([m.names.index(n) for n in req], lens_np)
     eng = LoraUnorderedBatchInfer(m.ia, [m.adapters[n] for n in req])
     eng.begin_step(torch.tensor(start, dtype=torch.int32, device=gpu), torch.from_numpy(lens_np).to(gpu), is_prefill=True)
     assert not eng.use_segmented
     x, base = _inputs(m, np.random.default_rng(3), int(lens_np.sum()))
+    slora_hip.clear_plan_cache()
+    slora_hip.clear_prefill_plan_cache()
+    slora_hip.plan_cache_stats(reset=True)
     out = _run_layers(m, eng, gpu, x, base)
+    stats = slora_hip.plan_cache_stats()   # which plans the step built tells which kernels served it
+    assert (stats["prefill_builds"], stats["builds"]) == ((1, 0) if segmented else (0, 1))
     for p in range(4):
         close(out[0][p], m.ref(0, p, base[0][p], x[0][1] if p == 3 else x[0][0], bins))
     wide = torch.zeros((int(lens_np.sum()), 1024), dtype=torch.float16, device=gpu)

@@ -487,8 +487,9 @@ def test_prefill_shrink_above_4096_tokens(gpu, dtype, hidden, ranks, n_req, lo, 
     (5120, [16, 40], [31, 64, 5]),                 # chunks of 320, two per wavefront; a rank that ends inside a tile
     (2560, [8], [7]),                              # chunks of 320, one per wavefront
     (576, [24, 8], [40, 3]),                       # a last chunk of 64; wavefronts with nothing to do
-    (8192, [128, 32], [20, 9]),                    # two chunks of 512 per wavefront; four groups of 32 columns
-    (512, [64, 32, 16, 8], [90] * 40),             # more workgroups than compute units
+    (8192, [128, 32], [20, 9]),                    # two chunks of 512 per wavefront; eight groups of 16 columns
+    (5120, [64, 16], [256] * 5),                   # 32 columns per workgroup, 64 of q, k and v
+    (512, [64, 32, 16, 8], [70] * 40),             # more workgroups than compute units
     (512, [8, 16], [3] * 256),                     # as many requests as a plan describes
 ])
 def test_prefill_small_batches(gpu, dtype, hidden, ranks, lens):
@@ -510,9 +511,9 @@ def test_prefill_small_batches(gpu, dtype, hidden, ranks, lens):
     t = (g.a_loc, g.a_start, g.a_len, start, ln, rq)
     w_a, w_b = g.key.view(c.n_pages, hidden), g.value.view(c.n_pages, hidden)
     d = [torch.full((T, R), 7.0, dtype=g.tdt, device=gpu) for _ in range(3)]
-    lora_get_qkvo_fwd_shrink_qkv(g.x, w_a, *d, *t, hidden, R, max_len)
     plain = torch.full((T, R), 7.0, dtype=g.tdt, device=gpu)
     lora_get_qkvo_fwd_shrink(g.x, w_a, plain, *t, hidden, 2, R, max_len, plan=False)
+    lora_get_qkvo_fwd_shrink_qkv(g.x, w_a, *d, *t, hidden, R, max_len)    # (the last shrink: its plan serves the expands)
     assert torch.equal(plain, d[2])
     for p in (0, 2):
         d_ref = O.ref_prefill_shrink(np.zeros((T, R), np.float32), c.x, c.key, c.a_loc, c.a_start, c.a_len, start_np, lens,
