@@ -97,7 +97,6 @@ constexpr int kShrWaves = kShrThreads / kWave;  // K is split over the 4 wavefro
 constexpr int kShrMF = 4;                       // 16-row A fragments per tile
 constexpr int kShrTM = 16 * kShrMF;             // token rows per tile
 constexpr int kShrNB = 64;                      // rank columns per pass
-static_assert(kShrNB == kWave, "shrink_tile looks up one column per lane");
 constexpr int kShrLd = kShrNB + 4;              // LDS row pitch (floats) -> conflict-free C-tile stores
 
 // Element-wise fallback for layouts the vector path cannot read.
@@ -454,7 +453,6 @@ __device__ __forceinline__ void shrink_part_lds_pass(const SegShrinkArgs& p, uns
   const int crow = lane >> 3, piece = (lane & 7) ^ crow;
   const uint16_t* src_w[R::kLpw];  // entries 0, 1 unused
   int chunk[R::kLpw];
-  uint32_t have = 0;  // bit ui: the rank row of this lane's column in unit wn * NU + ui is the adapter's and has a page
   {
     int64_t pg[R::kLpw];
 #pragma unroll
@@ -465,13 +463,6 @@ __device__ __forceinline__ void shrink_part_lds_pass(const SegShrinkArgs& p, uns
       const int a = l - 8, u = a >> 1, pj = u / NT, t = u - pj * NT;
       const int j = nb0 + t * 16 + (a & 1) * 8 + crow;  // rank row (weight chunks)
       pg[q] = seg_page_nobranch(p.t, base_li + (int64_t)pj * rank + j, q >= 2 && j < r_eff && p.t.n_loc > 0);
-    }
-#pragma unroll
-    for (int ui = 0; ui < NU; ++ui) {
-      int u = wn * NU + ui;
-      if (u >= U) u = U - 1;
-      const int pj = u / NT, j = nb0 + (u - pj * NT) * 16 + (lane & 15);
-      have |= (uint32_t)(seg_page_nobranch(p.t, base_li + (int64_t)pj * rank + j, j < r_eff && p.t.n_loc > 0) >= 0) << ui;
     }
 #pragma unroll
     for (int q = 0; q < R::kLpw; ++q)  // a row that does not exist reads pool page 0: its products only reach columns that are zeroed
@@ -575,7 +566,7 @@ __device__ __forceinline__ void shrink_part_lds_pass(const SegShrinkArgs& p, uns
 #pragma unroll
             for (int i = 0; i < 4; ++i)
               s_out[((2 * wm + fi) * 16 + 4 * lg + i) * kShrOutPitch + c] =
-                  T::from_float((have >> ui) & 1 ? acc[fi][ui][i] : 0.f);
+                  T::from_float(nb0 + c < r_eff ? acc[fi][ui][i] : 0.f);
         }
       }
       lds_barrier();
@@ -640,7 +631,6 @@ __device__ __forceinline__ void shrink_part_lds(const SegShrinkArgs& p, unsigned
 template <typename T, int NPROJ, bool DEEP>
 __device__ __forceinline__ void shrink_tile(const SegShrinkArgs& p, float* s_part, int64_t row_first, int m_cnt,
                                             int r_eff, int64_t base_li, int rank, int cg) {
-  __shared__ bool s_have[NPROJ][kShrNB];  // rank column c of the pass has a page
   const int cs = p.col_split;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -670,8 +660,12 @@ __device__ __forceinline__ void shrink_tile(const SegShrinkArgs& p, float* s_par
     if (n_own > 0) {
       // weight rows of the lane's two loads per B fragment, for every projection of the
       // launch (projection pj's rows start rank entries of a_loc behind the one before):
-      // the page lookups go out together; a row that does not exist (j >= r_eff, bad page
-      // id) reads pool page 0 -- its products only reach output columns that are zeroed below
+      // the page lookups go out together; a row that does not exist (j >= r_eff) reads pool page 0
+      // -- its products only reach output columns that are zeroed below -- and so does one whose
+      // page id is outside the pool, whose column then holds that product: to look at it behind
+      // the K loops, even in a branch never taken, changes how the compiler schedules the loop of
+      // the q/k/v kernel, which fills the register file (2000 tokens of rank 128 in f16: 60 -> 74
+      // us; in bf16 it takes 75 as it is)
       const uint16_t* wline[NPROJ][4][2];
       {
         int64_t pg[NPROJ][4][2];
@@ -685,19 +679,12 @@ __device__ __forceinline__ void shrink_tile(const SegShrinkArgs& p, float* s_par
               pg[pj][t][g] = seg_page_nobranch(p.t, base_li + (int64_t)pj * rank + j,
                                                t < n_own && j < r_eff && p.t.n_loc > 0);
             }
-        int64_t pg_col[NPROJ];  // of the column this lane sums (every wavefront the same)
-#pragma unroll
-        for (int pj = 0; pj < NPROJ; ++pj)
-          pg_col[pj] = seg_page_nobranch(p.t, base_li + (int64_t)pj * rank + nb0 + lane,
-                                         nb0 + lane < r_eff && p.t.n_loc > 0);
 #pragma unroll
         for (int pj = 0; pj < NPROJ; ++pj)
 #pragma unroll
           for (int t = 0; t < 4; ++t)
 #pragma unroll
             for (int g = 0; g < 2; ++g) wline[pj][t][g] = wg + (pg[pj][t][g] >= 0 ? pg[pj][t][g] : 0) * p.w_stride;
-#pragma unroll
-        for (int pj = 0; pj < NPROJ; ++pj) s_have[pj][lane] = pg_col[pj] >= 0;  // (waits in LDS: the K loop fills the registers)
       }
 #pragma unroll
       for (int pj = 0; pj < NPROJ; ++pj)
@@ -763,7 +750,7 @@ __device__ __forceinline__ void shrink_tile(const SegShrinkArgs& p, float* s_par
         const int m = idx / kShrNB, c = idx - m * kShrNB;
         if (m < m_cnt && c < nb_cnt && ((c >> 4) & (cs - 1)) == cg) {
           float v = 0.f;
-          if (nb0 + c < r_eff && s_have[pj][c]) {
+          if (nb0 + c < r_eff) {
 #pragma unroll
             for (int wv = 0; wv < kShrWaves; ++wv) v += s_part[wv * (kShrTM * kShrLd) + m * kShrLd + c];
           }
