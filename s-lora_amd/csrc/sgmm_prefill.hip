@@ -2110,11 +2110,17 @@ bool shrink_plan_usable(int64_t n_requests, int64_t m_tiles, int64_t grid, int c
 // Which batches take sgmm_shrink_split_kernel.  It reads a request's weight rows once per 16 token rows, the
 // other kernels once per 64, so the line falls with the rank.  us per launch (one projection / q, k and v; hidden
 // 4096, f16, rank 64), split kernel against the register-fed ones: 512 tokens 7.1 / 9.8 against 14.2 / 30, 1024 9.5 /
-// 13.6 against 14.3 / 31.7, 2311 14.0 / 27.8 against 19 / 37; 4096 29 / 55 against 23.2 / 42.1.  A whole layer at rank
-// 32: 2311 tokens 87 against 100.7 us, 4096 137 against 135; at rank 16 4096 tokens 121 against 128.
+// 13.6 against 14.3 / 31.7, 2304 in 9 prompts 14.2 / 26.5 against 22.5 / 36.4; 4096 29 / 55 against 23.2 / 42.1.  A
+// whole layer at rank 32: 2311 tokens 87 against 100.7 us, 4096 137 against 135; at rank 16 4096 tokens 121 against 128.
+// Ranks 33 .. 64 put 64 columns into a workgroup of the q/k/v launch, one per part and projection: within two
+// rounds of them on 256 compute units.  The third costs what the launch had gained -- 2304 / 2682 tokens in 9 prompts
+// at hidden 5120 39.2 / 53.6 us against 42.7 / 42.3, at 8192 50.1 / 68.5 against 59.4 / 58.9, at 4096 26.5 / 36.6
+// against 36.4 / 36.5 -- and one projection, faster still (19.3 against 26.3, 28.0 against 36.3, 14.4 against 22.5), has to
+// take the kernel that q, k and v take: their results are the same bits.
 bool small_batch(int64_t n_tokens, int64_t n_requests, int64_t max_rank) {
-  return n_tokens > 0 && n_tokens <= (max_rank <= 16 ? 4096 : 3584) && n_requests > 0 && n_requests <= kSegMaxReqs && max_rank > 0 &&
-         n_tokens * ((max_rank + 31) / 32) <= 6144;
+  if (n_tokens <= 0 || n_requests <= 0 || n_requests > kSegMaxReqs || max_rank <= 0) return false;
+  if (max_rank > 32 && max_rank <= 64 && n_tokens + kSplitRows * n_requests > 2 * kShrMaxGrid / 3 * kSplitRows) return false;
+  return n_tokens <= (max_rank <= 16 ? 4096 : 3584) && n_tokens * ((max_rank + 31) / 32) <= 6144;
 }
 
 struct SmallGeometry {

@@ -362,7 +362,7 @@ def _random_bits(seed, shape, dtype):
     (4096, [64, 24], [250] * 5, 2, 4),                    # chunks of 512; rows that end inside a part
     (576, [64, 8], [256] * 5, 2, 4),                      # a last chunk of 64 elements; wavefronts with nothing to do
     (8192, [128, 32], [300, 300], 2, 4),                  # two chunks of 512 per wavefront; four groups of 32 columns
-    (512, [64, 32, 16, 8], [70] * 40, 4, 4),              # more workgroups than compute units
+    (512, [64, 32, 16, 8], [65] * 30, 4, 4),              # more workgroups than compute units
     (512, [16, 8], [3] * 256, 1, 1),                      # as many requests as a plan describes
 ])
 def test_small_prefill_batches_through_the_c_abi(hip, dtype, H, ranks, lens, one, three):
@@ -454,3 +454,12 @@ def test_expand_with_the_plan_of_another_batch_does_nothing_and_says_so(hip):
     big.plan = other.plan
     y0, d = _random_bits(12, (big.T, H), "f16"), _random_bits(13, (big.T, R), "f16")
     assert np.array_equal(big.expand(y0, [d], True, 0)[0], big.expand(y0, [d], False, 0)[0]) and big.status() == 0
+
+
+@pytest.mark.parametrize("R,lens,small", [
+    (64, [84] * 32, False), (64, [2736], False), (64, [2688], True), (64, [210] * 10, True),   # two rounds of q/k/v workgroups
+    (40, [341] * 8, False), (32, [84] * 32, True), (72, [62] * 33, True), (72, [2064], False),
+])
+def test_the_plan_says_which_batches_are_small(hip, R, lens, small):
+    c = _sgmm_case(hip, 31, 64, [R], lens)
+    assert (_Segmented(hip, c, R, "f16").build()[2] == -16) == small

@@ -489,7 +489,7 @@ def test_prefill_shrink_above_4096_tokens(gpu, dtype, hidden, ranks, n_req, lo, 
     (576, [24, 8], [40, 3]),                       # a last chunk of 64; wavefronts with nothing to do
     (8192, [128, 32], [20, 9]),                    # two chunks of 512 per wavefront; eight groups of 16 columns
     (5120, [64, 16], [256] * 5),                   # 32 columns per workgroup, 64 of q, k and v
-    (512, [64, 32, 16, 8], [70] * 40),             # more workgroups than compute units
+    (512, [64, 32, 16, 8], [65] * 30),             # more workgroups than compute units
     (512, [8, 16], [3] * 256),                     # as many requests as a plan describes
 ])
 def test_prefill_small_batches(gpu, dtype, hidden, ranks, lens):
