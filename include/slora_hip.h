@@ -292,8 +292,9 @@ SLORA_API int slora_sgmm_expand_qkv(void* o_q, void* o_k, void* o_v, const void*
 
 /* slora_sgmm_expand (nproj = 1: o0, x0, feat_out0, o_row_stride0, any qkvo) or slora_sgmm_expand_qkv (nproj = 3,
  * qkvo = 0; k and v share feat_out12 and o_row_stride12) with a plan of slora_sgmm_plan_build for this batch: same
- * results bit for bit.  Small batches (tokens times rank up to 32768) read their row spans from the plan
- * instead of looking the requests up in every workgroup; larger ones leave the plan alone.  The sizes must
+ * results bit for bit.  Small batches (tokens times rank up to 32768, less for very few or very many outputs)
+ * read their row spans from the plan instead of looking the requests up in every workgroup; larger ones
+ * leave the plan alone.  The sizes must
  * be those of the build call, as for slora_sgmm_shrink_planned. */
 SLORA_API int slora_sgmm_expand_planned(const void* plan, int nproj, void* o0, void* o1, void* o2, const void* x0,
                           const void* x1, const void* x2, const void* w, const slora_tables* tables, const void* scales,

@@ -2167,13 +2167,18 @@ int launch_small_shrink(const SegShrinkArgs& p, const int* plan, int64_t max_inp
   return launch_split<T, 4, 64>(p, plan, g.parts, stream);
 }
 
-// Which of those batches expand from the plan's spans.  A span reads its B^T pages for 32 rows, the walking kernel
-// for all rows of a request that it owns: us per launch (one projection / q, k and v), spans against walk, hidden 4096:
-// 64 tokens of rank 8 4.8 / 6.1 against 5.4 / 6.0, 1024 tokens of rank 8 8.1 / 14.7 against 8.7 / 15.7, of rank 32
-// 8.6 / 15.8 against 8.7 / 16.7, 512 of rank 64 6.7 / 12.2 against 7.4 / 13.0; beyond the line 1024 of rank 64 11.1 / 21.8
-// against 11.7 / 18.6.
-bool small_expand(int64_t n_tokens, int64_t n_requests, int64_t max_rank) {
-  return small_batch(n_tokens, n_requests, max_rank) && n_tokens * max_rank <= 32 * 1024;
+// Which of those batches expand from the plan's spans; `outputs`: columns of all projections of the launch.  A span
+// reads its B^T pages for 32 rows, the walking kernel for all rows of a request that it owns: us per launch
+// (one projection / q, k and v), spans against walk, hidden 4096: 64 tokens of rank 8 4.8 / 6.1 against 5.4 / 6.0, 1024
+// tokens of rank 8 8.1 / 14.7 against 8.7 / 15.7, of rank 32 8.6 / 15.8 against 8.7 / 16.7, 512 of rank 64 6.7 / 12.2
+// against 7.4 / 13.0; beyond the line 1024 of rank 64 11.1 / 21.8 against 11.7 / 18.6.  What is read again grows with the
+// outputs too: at hidden 8192 512 tokens of rank 64 in one prompt are 1.28 of the walk for q, k and v (24576 outputs; 256
+// tokens 0.98) and 1.00 for one projection.  And where a launch has few outputs, many tokens are many workgroups with
+// little to do: one projection of 512, 2048 / 3072 / 4096 tokens of rank 8 1.02 / 1.26 / 1.37 of the walk, of 1024 1.02 /
+// 1.10 / 1.18, q, k and v of 1024 1.06 / 1.08 / 1.13; of 4096 0.94 / 0.87 / 1.03.
+bool small_expand(int64_t n_tokens, int64_t n_requests, int64_t max_rank, int64_t outputs) {
+  return small_batch(n_tokens, n_requests, max_rank) && n_tokens * max_rank <= 32 * 1024 &&
+         n_tokens * max_rank * outputs <= 512 * 1024 * 1024 && (n_tokens <= 2048 || outputs >= 4096);
 }
 
 template <typename T, int KS>
@@ -2383,7 +2388,8 @@ int seg_expand_common(const int* plan, void* const o[3], const void* const x[3],
   p.row_cap = max_input_len > (1 << 30) ? (1 << 30) : (int)((max_input_len + kExpTMW - 1) / kExpTMW * kExpTMW);
   p.m_tiles = (int)((max_input_len + p.m_span - 1) / p.m_span);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (plan != nullptr && small_expand(n_tokens, n_requests, max_rank))
+  const int64_t outputs = nproj == 3 ? feat_out[0] + feat_out[1] + feat_out[2] : feat_out[0];
+  if (plan != nullptr && small_expand(n_tokens, n_requests, max_rank, outputs))
     return dtype == SLORA_DTYPE_F16 ? launch_small_expand<F16>(p, plan, max_input_len, s)
                                     : launch_small_expand<BF16>(p, plan, max_input_len, s);
   return dtype == SLORA_DTYPE_F16 ? launch_seg_expand<F16>(p, s) : launch_seg_expand<BF16>(p, s);

@@ -463,3 +463,21 @@ def test_expand_with_the_plan_of_another_batch_does_nothing_and_says_so(hip):
 def test_the_plan_says_which_batches_are_small(hip, R, lens, small):
     c = _sgmm_case(hip, 31, 64, [R], lens)
     assert (_Segmented(hip, c, R, "f16").build()[2] == -16) == small
+
+
+@pytest.mark.parametrize("H,R,T,nproj,spans", [
+    (512, 8, 2048, 1, True), (512, 8, 2064, 1, False), (1024, 8, 2064, 3, False),   # many tokens, few outputs
+    (2048, 8, 2064, 3, True), (4096, 8, 2064, 1, True),
+    (8192, 64, 320, 3, True), (8192, 64, 352, 3, False), (8192, 64, 512, 1, True),  # wide q, k and v
+])
+def test_which_expands_read_the_plans_spans(hip, H, R, T, nproj, spans):
+    """An expand that reads spans leaves its output alone when the plan is another batch's; one that looks its
+    rows up itself does not look at the plan."""
+    g = _Segmented(hip, _sgmm_case(hip, 32, H, [R], [T // 2, T - T // 2]), R, "f16")
+    other = _Segmented(hip, _sgmm_case(hip, 33, 64, [R], [30, 41]), R, "f16")
+    assert other.build()[2] == -16
+    g.plan = other.plan
+    y0, d = _random_bits(14, (T, H), "f16"), _random_bits(15, (T, R), "f16")
+    print(f"c-abi expand of {T} tokens of rank {R} at hidden {H}", flush=True)
+    y = g.expand(y0, [d] * nproj, True, None if nproj == 3 else 0)
+    assert all(np.array_equal(q, y0) == spans for q in y) and g.status() == int(spans)
