@@ -1057,7 +1057,7 @@ constexpr int kSegPartWords = 8;
 enum SegPlanHeader {
   SP_MAGIC = 0, SP_PARTS, SP_SPLIT, SP_NREQ, SP_NTOKENS, SP_MAXRANK, SP_ROWCAP,
   SP_STATUS,  // as PH_STATUS of the decode plan (word 7)
-  SP_SPANS    // small batches: records of the expand behind the SP_PARTS of the shrink (0: none)
+  SP_SPANS    // records of the expand behind the SP_PARTS of the shrink; 0 in the plan of a large batch
 };
 enum SegPart { PT_ROW = 0, PT_ROWS, PT_RANK, PT_START_LO, PT_START_HI, PT_ADAPTER };
 
