@@ -153,8 +153,8 @@ SLORA_API int slora_bgmv_plan_build(void* plan, int64_t plan_bytes, const slora_
  * WAITS for the work queued on `stream`.  0 after a build.  Bit 0: a launch was given this plan
  * with another batch size, rank cap or launch shape than the plan was built for -- such a launch
  * does nothing (the outputs keep their values) and leaves this mark instead of an error code,
- * because only the device can tell.  Bit 1: a hand-over inside slora_bgmv_lora_planned was
- * abandoned after its poll limit.  The mark covers a wrong plan in a large enough buffer only: a
+ * because only the device can tell.  Bit 1: a hand-over inside slora_bgmv_lora_planned took
+ * longer than its poll limit and its rows were computed a second time (the results are right).  The mark covers a wrong plan in a large enough buffer only: a
  * planned launch reads its item records before it has seen the header, so the buffer it is given
  * must hold slora_bgmv_plan_bytes(batch, rank_cap) bytes for the batch and rank cap OF THE LAUNCH,
  * whatever the plan in it was built for.  Not to be called on a stream that is being captured
@@ -183,21 +183,22 @@ SLORA_API int slora_bgmv_expand_planned(const void* plan, int64_t rank_cap, int6
                                         int64_t h_out1, int64_t h_out2, int64_t page_elems,
                                         int64_t n_pages, int qkvo, int dtype, void* stream);
 
-/* Shrink and expand of a projection (nproj = 1) or of q, k and v (nproj = 3, qkvo = 0) in ONE
- * launch, with a plan.  The reference issues the two back to back for every projection
- * (slora/models/peft/lora_unordered_batch_infer.py:267-273, 287-293, 307-313, 438-444); here one
- * workgroup per plan item computes its 8 rows of delta = x A, hands them to the other
- * workgroups of its run through counters behind the plan (device-scope stores and loads, no
- * second launch), and then updates y with its 8 pages of B^T:
+/* Shrink and expand of a projection (nproj = 1) or of q, k and v (nproj = 3, qkvo = 0), with a plan.  The
+ * reference issues the two back to back for every projection
+ * (slora/models/peft/lora_unordered_batch_infer.py:267-273, 287-293, 307-313, 438-444); here both are ONE
+ * launch where that is the faster form (pages of one pass -- 4096, 5120, 6144 or 8192 elements -- and
+ * launches of few or of enough workgroups; at most 4096 tokens and tokens * rank_cap <= 2^18): the
+ * shrink's workgroups hand the rows of delta = x A to the expand's through tagged words behind the plan
+ * (device-scope stores and loads).  Elsewhere it is the two planned launches.
  *   delta_i[b, j] = T(sum_k w_a[page(a,p,j), k] * x[b, k])                    as slora_bgmv_shrink
  *   y_i[b, n]     = T(y_i[b, n] + T(scales[a] * sum_d Bt[n*r+d] * delta_i[b, d]))  as slora_bgmv_expand
  * bit for bit what the two calls give.  delta_i ([batch, delta_cols], delta_cols a multiple of 8
  * and at least every rank in the batch for the usual result) is left filled as after the
  * shrink call.  w_a / w_b are the pools of the A side and the B side (key_buffer[l],
- * value_buffer[l]), which share page ids.  `plan` is written to (its counters): launches that
- * use one plan must not overlap, e.g. stay on one stream.  A hand-over that is not complete
- * after 65536 polls is abandoned (the workgroup goes on and a flag is set behind the plan)
- * rather than waited for for ever; it never is unless workgroups are not handed out in order. */
+ * value_buffer[l]), which share page ids.  `plan` is written to (its hand-over area): launches that
+ * use one plan must not overlap, e.g. stay on one stream.  A wait for rows that have not come after 16384
+ * polls ends: the waiting wavefront computes them itself and marks the plan's status word; it never
+ * happens unless workgroups are not handed out in order. */
 SLORA_API int slora_bgmv_lora_planned(void* plan, int64_t rank_cap, int64_t n_items, int nproj, void* y0, void* y1,
                                       void* y2, void* delta0, void* delta1, void* delta2, const void* x,
                                       const void* w_a, const void* w_b, const slora_tables* tables,

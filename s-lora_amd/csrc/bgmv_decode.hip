@@ -24,7 +24,7 @@
 //
 // Replaces slora/csrc/bgmv/bgmv_impl.cuh:14-241 of the reference.
 
-#include "bgmv_device.hpp"
+#include "bgmv_pages.hpp"
 
 namespace slora {
 namespace {
@@ -86,15 +86,15 @@ constexpr int kMaxLdsRuns = 2048;  // run descriptors kept in LDS
 // single L2.  Queues are padded to the longest with empty items.
 __global__ __launch_bounds__(kPlanThreads) void bgmv_plan_kernel(int* __restrict__ plan, Tables t, int batch,
                                                                  int rank_cap, int max_items,
-                                                                 int* __restrict__ scratch, int* __restrict__ sync,
-                                                                 int sync_words) {
+                                                                 int* __restrict__ scratch, int4* __restrict__ hand,
+                                                                 int hand_vecs) {
   __shared__ int s_bins[kMaxLdsBins];
   __shared__ int s_ra[kMaxLdsRuns], s_rb[kMaxLdsRuns], s_rn[kMaxLdsRuns];
   __shared__ int s_wave[kPlanWaves];
   __shared__ int s_max_rank, s_total;
   __shared__ int s_qstart[kXcds], s_qlen[kXcds];
   const int tid = threadIdx.x;
-  for (int i = tid; i < sync_words; i += kPlanThreads) sync[i] = 0;
+  for (int i = tid; i < hand_vecs; i += kPlanThreads) hand[i] = make_int4(0, 0, 0, 0);
   if (tid == 0) {
     s_max_rank = 0;
     s_total = 0;
@@ -252,7 +252,7 @@ constexpr int kFastPlanBatch = 1024;
 
 __global__ __launch_bounds__(kPlanThreads) void bgmv_plan_fast_kernel(int* __restrict__ plan, Tables t, int batch,
                                                                       int rank_cap, int max_items,
-                                                                      int* __restrict__ sync, int sync_words) {
+                                                                      int4* __restrict__ hand, int hand_vecs) {
   __shared__ int s_bins[kFastPlanBatch];    // adapter of a token, -1: none
   __shared__ int s_run[kFastPlanBatch];     // token -> run, valid at a run's first token
   __shared__ int s_ra[kFastPlanBatch], s_rr[kFastPlanBatch], s_rn[kFastPlanBatch];  // run: adapter, rank, items
@@ -265,7 +265,8 @@ __global__ __launch_bounds__(kPlanThreads) void bgmv_plan_fast_kernel(int* __res
   __shared__ int s_max_rank, s_total;
   __shared__ int s_qstart[kXcds], s_qlen[kXcds];
   const int tid = threadIdx.x;
-  for (int i = (int)blockIdx.x * kPlanThreads + tid; i < sync_words; i += (int)gridDim.x * kPlanThreads) sync[i] = 0;
+  for (int i = (int)blockIdx.x * kPlanThreads + tid; i < hand_vecs; i += (int)gridDim.x * kPlanThreads)
+    hand[i] = make_int4(0, 0, 0, 0);
   if (tid == 0) {
     s_max_rank = 0;
     s_total = 0;
@@ -442,7 +443,7 @@ __device__ __forceinline__ int block_exclusive_max(int v, int* s_wave) {
 
 __global__ __launch_bounds__(kPlanThreads) void bgmv_plan_sort_kernel(int* __restrict__ plan, Tables t, int batch,
                                                                       int rank_cap, int max_items, int n,
-                                                                      int* __restrict__ sync, int sync_words) {
+                                                                      int4* __restrict__ hand, int hand_vecs) {
   extern __shared__ __align__(16) unsigned char s_dyn[];
   uint32_t* s_key = reinterpret_cast<uint32_t*>(s_dyn);                // sorted: adapter << 13 | token, ~0: no member
   int* s_before = reinterpret_cast<int*>(s_key + n);                   // run -> items in front of it
@@ -452,7 +453,8 @@ __global__ __launch_bounds__(kPlanThreads) void bgmv_plan_sort_kernel(int* __res
   __shared__ int s_qstart[kXcds], s_qlen[kXcds];
   constexpr uint32_t kNone = 0xffffffffu;
   const int tid = threadIdx.x;
-  for (int i = (int)blockIdx.x * kPlanThreads + tid; i < sync_words; i += (int)gridDim.x * kPlanThreads) sync[i] = 0;
+  for (int i = (int)blockIdx.x * kPlanThreads + tid; i < hand_vecs; i += (int)gridDim.x * kPlanThreads)
+    hand[i] = make_int4(0, 0, 0, 0);
   if (tid == 0) s_max_rank = 0;
   if (tid < kXcds) {
     s_qstart[tid] = 0x7fffffff;
@@ -710,6 +712,68 @@ int launch_expand(ExpandArgs p, int64_t items, hipStream_t stream) {
   return launch_expand_nv<T, NPROJ, PLANNED, 8>(p, items, stream);
 }
 
+// Planned launches over whole one-pass pages (see bgmv_pages.hpp); grids as for the kernels above.
+template <typename T, int NV>
+__global__ __launch_bounds__(256, NV > 12 ? 2 : (NV > 8 ? 3 : 4)) void bgmv_shrink_pages_kernel(const PageArgs) {
+  extern __shared__ u32x4 s_x[];  // [kTT][NV * 64]
+  const PageArgs& p = page_args();
+  int unit = (int)blockIdx.x;
+  for (;;) {
+    const int n_items = pages_shrink<T, NV, false>(p, unit, (int)blockIdx.y, s_x);
+    unit += (int)gridDim.x;
+    if (!p.strided || unit >= n_items) return;
+    __syncthreads();  // the staging area of the item before is free
+  }
+}
+
+template <typename T, int NV, bool INTERLEAVE>
+__global__ __launch_bounds__(256, NV > 12 ? 3 : 4) void bgmv_expand_pages_kernel(const PageArgs) {
+  __shared__ __align__(16) uint16_t s_out[4][kTT * ExpandPass<NV>::kStrip];
+  const PageArgs& p = page_args();
+  int unit = (int)blockIdx.x, sub = (int)blockIdx.y;
+  if (INTERLEAVE) {
+    const int S = 2 * p.nproj, g = unit >> 3;
+    unit = (g / S) * 8 + (unit & 7);
+    sub = g % S;
+    if (unit >= p.n_units) return;
+  }
+  for (;;) {
+    const int n_items = pages_expand<T, NV, false>(p, unit, sub, s_out[threadIdx.x >> 6], nullptr);
+    unit += INTERLEAVE ? (int)gridDim.x / (2 * p.nproj) : (int)gridDim.x;
+    if (!p.strided || unit >= n_items) return;
+  }
+}
+
+template <typename T, int NV>
+int launch_shrink_pages(const PageArgs& p, hipStream_t stream) {
+  auto kernel = bgmv_shrink_pages_kernel<T, NV>;
+  constexpr int lds = kTT * ExpandPass<NV>::kElems * 2;
+  static PerDeviceOnce once;
+  if (!raise_dynamic_lds(reinterpret_cast<const void*>(kernel), lds, once)) return SLORA_ERR_LAUNCH;
+  hipLaunchKernelGGL(kernel, dim3((uint32_t)p.n_units, (uint32_t)p.nproj), dim3(256), lds, stream, p);
+  return hipGetLastError() == hipSuccess ? SLORA_OK : SLORA_ERR_LAUNCH;
+}
+
+template <typename T, int NV>
+int launch_expand_pages(const PageArgs& p, hipStream_t stream) {
+  const uint32_t wgs = 2 * p.nproj, units = (uint32_t)p.n_units;
+  if (p.interleave)
+    hipLaunchKernelGGL((bgmv_expand_pages_kernel<T, NV, true>), dim3((units + 7) / 8 * 8 * wgs), dim3(256), 0, stream, p);
+  else
+    hipLaunchKernelGGL((bgmv_expand_pages_kernel<T, NV, false>), dim3(units, wgs), dim3(256), 0, stream, p);
+  return hipGetLastError() == hipSuccess ? SLORA_OK : SLORA_ERR_LAUNCH;
+}
+
+template <typename T>
+int dispatch_pages(const PageArgs& p, int64_t page_elems, bool expand, hipStream_t s) {
+  switch (page_elems / (8 * kWave)) {
+    case 8: return expand ? launch_expand_pages<T, 8>(p, s) : launch_shrink_pages<T, 8>(p, s);
+    case 10: return expand ? launch_expand_pages<T, 10>(p, s) : launch_shrink_pages<T, 10>(p, s);
+    case 12: return expand ? launch_expand_pages<T, 12>(p, s) : launch_shrink_pages<T, 12>(p, s);
+    default: return expand ? launch_expand_pages<T, 16>(p, s) : launch_shrink_pages<T, 16>(p, s);
+  }
+}
+
 template <typename T>
 int dispatch_shrink(const ShrinkArgs& p, int nproj, bool planned, int64_t units, hipStream_t s) {
   return planned ? launch_shrink<T, true>(p, nproj, units, s) : launch_shrink<T, false>(p, nproj, units, s);
@@ -732,6 +796,13 @@ int shrink_common(const void* plan, int64_t n_items, int64_t rank_cap, void* con
   if (rc != SLORA_OK) return rc == kNothingToDo ? SLORA_OK : rc;
   const bool planned = plan != nullptr;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  // whole one-pass pages, and every row of delta listed by the plan
+  if (planned && h_in == page_elems && whole_pages(page_elems) && y_cols <= rank_cap && grid <= 0x7fffffffLL / 6) {
+    PageArgs q{};
+    fill_pages_shrink(q, p, nproj);
+    q.n_units = (int)grid;
+    return dtype == SLORA_DTYPE_F16 ? dispatch_pages<F16>(q, page_elems, false, s) : dispatch_pages<BF16>(q, page_elems, false, s);
+  }
   return dtype == SLORA_DTYPE_F16 ? dispatch_shrink<F16>(p, nproj, planned, grid, s)
                                   : dispatch_shrink<BF16>(p, nproj, planned, grid, s);
 }
@@ -747,6 +818,13 @@ int expand_common(const void* plan, int64_t n_items, int64_t rank_cap, void* con
   if (rc != SLORA_OK) return rc == kNothingToDo ? SLORA_OK : rc;
   const bool planned = plan != nullptr;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  if (planned && pages_serve(p, nproj, rank_cap) && grid <= 0x7fffffffLL / 7) {
+    PageArgs q{};
+    fill_pages_expand(q, p, nproj);
+    q.n_units = (int)grid;
+    q.e.n_units = (int)grid;
+    return dtype == SLORA_DTYPE_F16 ? dispatch_pages<F16>(q, page_elems, true, s) : dispatch_pages<BF16>(q, page_elems, true, s);
+  }
   return dtype == SLORA_DTYPE_F16 ? dispatch_expand<F16>(p, nproj, planned, grid, s)
                                   : dispatch_expand<BF16>(p, nproj, planned, grid, s);
 }
@@ -813,8 +891,8 @@ int slora_bgmv_plan_build(void* plan, int64_t plan_bytes, const slora_tables* ta
   if (rc != SLORA_OK) return rc;
   const int64_t max_items = plan_max_items(batch, rank_cap);
   if (max_items > 0x7fffffffLL) return SLORA_ERR_UNSUPPORTED;
-  int* sync = static_cast<int*>(plan) + plan_sync_offset(batch, rank_cap);
-  const int sync_words = (int)plan_sync_words(batch);
+  int4* hand = reinterpret_cast<int4*>(static_cast<int*>(plan) + plan_hand_offset(batch, rank_cap));
+  const int hand_vecs = (int)(plan_hand_words(batch, rank_cap) / 4);
   // Three builders, one plan (word for word): counting in LDS with a token per thread is the quickest
   // up to a few dozen tokens (4 us for one token, 10 us for 32), sorting from there on (15 us for 256
   // tokens, 23 us for 1024, 90 us for 8192: the counting builder takes 27 and 86 us for the first
@@ -825,7 +903,7 @@ int slora_bgmv_plan_build(void* plan, int64_t plan_bytes, const slora_tables* ta
     grid = grid < 1 ? 1 : (grid > 16 ? 16 : grid);
     hipLaunchKernelGGL(bgmv_plan_fast_kernel, dim3((uint32_t)grid), dim3(kPlanThreads), 0,
                        reinterpret_cast<hipStream_t>(stream), static_cast<int*>(plan), t, (int)batch, (int)rank_cap,
-                       (int)max_items, sync, sync_words);
+                       (int)max_items, hand, hand_vecs);
     return hipGetLastError() == hipSuccess ? SLORA_OK : SLORA_ERR_LAUNCH;
   }
   if (sortable) {
@@ -839,12 +917,12 @@ int slora_bgmv_plan_build(void* plan, int64_t plan_bytes, const slora_tables* ta
     grid = grid < 1 ? 1 : (grid > 16 ? 16 : grid);
     hipLaunchKernelGGL(bgmv_plan_sort_kernel, dim3((uint32_t)grid), dim3(kPlanThreads), lds,
                        reinterpret_cast<hipStream_t>(stream), static_cast<int*>(plan), t, (int)batch, (int)rank_cap,
-                       (int)max_items, n, sync, sync_words);
+                       (int)max_items, n, hand, hand_vecs);
     return hipGetLastError() == hipSuccess ? SLORA_OK : SLORA_ERR_LAUNCH;
   }
   int* scratch = static_cast<int*>(plan) + kPlanHeaderWords + max_items * kItemWords;
   hipLaunchKernelGGL(bgmv_plan_kernel, dim3(1), dim3(kPlanThreads), 0, reinterpret_cast<hipStream_t>(stream),
-                     static_cast<int*>(plan), t, (int)batch, (int)rank_cap, (int)max_items, scratch, sync, sync_words);
+                     static_cast<int*>(plan), t, (int)batch, (int)rank_cap, (int)max_items, scratch, hand, hand_vecs);
   return hipGetLastError() == hipSuccess ? SLORA_OK : SLORA_ERR_LAUNCH;
 }
 

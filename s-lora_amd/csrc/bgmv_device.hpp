@@ -38,17 +38,21 @@ __device__ __forceinline__ int64_t lookup_page(const Tables& t, int64_t li) {
 //   [8..40)  page id of a_loc entry p*rank + j0 + i at [8 + p*8 + i]  (p = q,k,v,o; -1 = none)
 //   [40..42) a_start[adapter] (int64)
 //   [42]     1 if this is the run's last stored item and rank > rank_cap (rows the plan does not list)
-// Behind the records: the one-workgroup builder's scratch (6 words per token), then the
-// hand-over counters of the one-launch LoRA (kSyncHeader words, then 4 per token: entry
-// [first token of a run][projection], see lora_handover), zeroed by every build.
+// Behind the records: the one-workgroup builder's scratch (6 words per token), then, zeroed by every
+// build, the hand-over area of the one-launch LoRA (bgmv_lora.hip; plans of more than kHandTokens
+// tokens or kHandEntries rows have none):
+//   kEpochWords words per item: [projection * 3 + s] = launches that workgroup s of the item (0: shrink,
+//   1, 2: the two halves of the expand) has taken part in;
+//   4 x rank_cap (rounded up to 8) words per token: [projection][row] = delta value | (launch << 16).
 constexpr int kPlanMagic = 0x534c5033;  // "SLP3"
-constexpr int kSyncHeader = 4;          // [0]: set when a hand-over gave up waiting (never expected)
-enum { SY_TIMEOUT = 0 };
+constexpr int kEpochWords = 16;
+constexpr int64_t kHandTokens = 4096, kHandEntries = 1 << 18;
 constexpr int kPlanHeaderWords = 16;
 constexpr int kItemWords = 48;
 enum { PH_MAGIC = 0, PH_NITEMS = 1, PH_MAXRANK = 2, PH_BATCH = 3, PH_TT = 4, PH_RANKCAP = 5, PH_NRUNS = 6, PH_STATUS = 7 };
 // PH_STATUS (0 after a build; read back with slora_plan_status): bit 0 = a launch named another batch size
-// or rank cap than the plan was built for and did nothing; bit 1 = a hand-over of the one-launch LoRA gave up
+// or rank cap than the plan was built for and did nothing; bit 1 = a hand-over of the one-launch LoRA gave up (and
+// computed what it had waited for)
 enum { kPlanStatusMismatch = 1, kPlanStatusTimeout = 2 };
 enum { IT_ADAPTER = 0, IT_RANK = 1, IT_NTOK = 2, IT_J0 = 3, IT_TOK = 4, IT_PAGES = 8, IT_BASE = 40, IT_MORE = 42 };
 
@@ -147,6 +151,7 @@ __device__ __forceinline__ void discover_run(const Tables& t, int batch, int b, 
 // read up front and pinned in scalar registers before the first branch, so the
 // compiler cannot sink the loads below the early exits: header check, record
 // and page ids are ONE round trip of independent scalar loads.
+template <bool ONE_GROUP = false>
 __device__ __forceinline__ void load_item(const int* __restrict__ plan, int idx, int pp, int jr0, int jr1, int batch,
                                           int rank_cap, Item& it, int& page0, int& page1) {
   // The header and the records do not change while a kernel that reads them runs
@@ -155,6 +160,7 @@ __device__ __forceinline__ void load_item(const int* __restrict__ plan, int idx,
   // stores.
   typedef const int __attribute__((address_space(4))) * ConstWords;
   ConstWords head = (ConstWords)plan;
+  if (ONE_GROUP) asm volatile("" : "+s"(head));  // in a loop over items: the header too is read here, not in front of the loop
   ConstWords rec = head + kPlanHeaderWords + (int64_t)idx * kItemWords;
   int magic = head[PH_MAGIC], n_items = head[PH_NITEMS], plan_batch = head[PH_BATCH], plan_cap = head[PH_RANKCAP];
   int a = rec[IT_ADAPTER], r = rec[IT_RANK], n_tok = rec[IT_NTOK], j0 = rec[IT_J0];
@@ -215,8 +221,7 @@ struct ShrinkArgs {
 // and are discarded) so that no branch separates the loads: first the activations, then
 // both weight pages; the LDS stores wait for the activations only.
 // NV: 16-byte vectors a lane holds of a page (8 = hidden up to 4096).
-// COH: the results are read by other workgroups of the same launch (st16_coherent).
-template <typename T, int NV, bool COH>
+template <typename T, int NV>
 __device__ __forceinline__ void shrink_fast(const ShrinkArgs& p, const Item& it, int proj, int r_eff,
                                             const int64_t (&page)[2], u32x4* s_x) {
   constexpr int XS = (NV + 3) / 4;  // activation vectors a thread stages per token
@@ -286,8 +291,7 @@ __device__ __forceinline__ void shrink_fast(const ShrinkArgs& p, const Item& it,
       if (t < it.n_tok) {
         const float sum = wave_sum(acc[i][t]);
         if (lane == 0 && page[i] >= 0 && row < r_eff) {
-          uint16_t* dst = y + (int64_t)it.tok[t] * p.y_cols + row;
-          if (COH) st16_coherent(dst, T::from_float(sum)); else *dst = T::from_float(sum);
+          y[(int64_t)it.tok[t] * p.y_cols + row] = T::from_float(sum);
         }
       }
     }
@@ -301,7 +305,7 @@ __device__ __forceinline__ void shrink_fast(const ShrinkArgs& p, const Item& it,
 // Grid: x = item (planned) or token * blocks + block (stateless), y = projection of the
 // launch.  s_x: [lds_tt][h_in / 8] LDS words.
 // `it` receives the item (n_tok = 0: nothing was done).
-template <typename T, bool PLANNED, int NV, bool COH = false>
+template <typename T, bool PLANNED, int NV>
 __device__ __forceinline__ int shrink_body(const ShrinkArgs& p, int unit, int proj, u32x4* s_x, Item& it) {
   constexpr int NW = 4;
   constexpr int NTASK = 2;
@@ -339,7 +343,7 @@ __device__ __forceinline__ int shrink_body(const ShrinkArgs& p, int unit, int pr
 #pragma unroll
     for (int i = 0; i < 2; ++i)
       if (it.j0 + wave + 4 * i >= r_eff) page2[i] = -1;
-    shrink_fast<T, NV, COH>(p, it, proj, r_eff, page2, s_x);
+    shrink_fast<T, NV>(p, it, proj, r_eff, page2, s_x);
     return it.plan_items;
   }
   const uint16_t* wbase = reinterpret_cast<const uint16_t*>(p.w);
@@ -445,8 +449,7 @@ __device__ __forceinline__ int shrink_body(const ShrinkArgs& p, int unit, int pr
           if (t < nt) {
             const float s = wave_sum(acc[i][t]);
             if (lane == 0 && wrow[i] != nullptr) {
-              uint16_t* dst = y + (int64_t)item_token(it, t0 + t) * p.y_cols + row[i];
-              if (COH) st16_coherent(dst, T::from_float(s)); else *dst = T::from_float(s);
+              y[(int64_t)item_token(it, t0 + t) * p.y_cols + row[i]] = T::from_float(s);
             }
           }
         }
@@ -615,8 +618,7 @@ __device__ __forceinline__ void expand_update(const ExpandArgs& p, int proj, con
 // FULL: every element of the page belongs to an output inside h_out and every rank
 // column is used (the caller checks: whole passes, page inside the output, delta as wide
 // as the rank) -- then no load needs its result masked.
-// COH: the delta rows were written by other workgroups of the same launch (ldg16_coherent).
-template <typename T, bool FULL, int NV, bool COH>
+template <typename T, bool FULL, int NV>
 __device__ __forceinline__ void expand_page(const ExpandArgs& p, int proj, const Item& it, int r_eff,
                                             const uint16_t* wpage, int64_t flat0, float scale, uint16_t* s_strip) {
   constexpr int kPass = ExpandPass<NV>::kElems;
@@ -654,9 +656,9 @@ __device__ __forceinline__ void expand_page(const ExpandArgs& p, int proj, const
     const uint16_t* xp = x + (int64_t)(t < it.n_tok ? it.tok[t] : it.tok[0]) * p.x_cols + (d_ok ? d0 : 0);
     // (FULL: a token the run does not have re-reads the first one's row; its sums are never used)
     if (FULL)
-      xv[t] = COH ? ldg16_coherent(xp) : ldg16(xp);
+      xv[t] = ldg16(xp);
     else
-      xv[t] = (t < it.n_tok && d_ok) ? (COH ? ldg16_coherent(xp) : ldg16(xp)) : zero16();
+      xv[t] = (t < it.n_tok && d_ok) ? ldg16(xp) : zero16();
   }
 
   for (int e0 = 0; e0 < page_elems; e0 += kPass) {
@@ -694,7 +696,7 @@ __device__ __forceinline__ void expand_page(const ExpandArgs& p, int proj, const
 
 // Any rank, any alignment: one lane per output whose first element lies in this
 // page, element-wise loads through a_loc (an output's r elements may continue
-// on the next page).
+// on the next page).  COH: the delta rows were written by other workgroups of the same launch.
 template <typename T, bool COH>
 __device__ __forceinline__ void expand_scalar(const ExpandArgs& p, int proj, const Item& it, int r_eff, int k,
                                               int64_t base_li, float scale) {
@@ -728,12 +730,12 @@ __device__ __forceinline__ void expand_scalar(const ExpandArgs& p, int proj, con
 
 // Page kk of projection `proj` for the item's run; `page` is its pool page id
 // or -2 to look it up in a_loc.
-template <typename T, int NV, bool COH>
+template <typename T, int NV>
 __device__ __forceinline__ void expand_one(const ExpandArgs& p, int proj, const Item& it, int r_eff, int kk,
                                            int64_t page, bool vec_ok, uint16_t* s_strip) {
   const int64_t base_li = it.base + (int64_t)it.r * (p.qkvo0 + proj);
   if (!vec_ok) {
-    expand_scalar<T, COH>(p, proj, it, r_eff, kk, base_li, load_scale(p.scales, p.scales_dtype, it.a));
+    expand_scalar<T, false>(p, proj, it, r_eff, kk, base_li, load_scale(p.scales, p.scales_dtype, it.a));
     return;
   }
   if (page == -2) page = lookup_page(p.t, base_li + kk);
@@ -745,9 +747,22 @@ __device__ __forceinline__ void expand_one(const ExpandArgs& p, int proj, const 
   const bool full = r_eff == it.r && p.page_elems % ExpandPass<NV>::kElems == 0 &&
                     flat0 + p.page_elems <= (int64_t)p.h_out[proj] * it.r;
   if (full)
-    expand_page<T, true, NV, COH>(p, proj, it, r_eff, wpage, flat0, scale, s_strip);
+    expand_page<T, true, NV>(p, proj, it, r_eff, wpage, flat0, scale, s_strip);
   else
-    expand_page<T, false, NV, COH>(p, proj, it, r_eff, wpage, flat0, scale, s_strip);
+    expand_page<T, false, NV>(p, proj, it, r_eff, wpage, flat0, scale, s_strip);
+}
+
+// pages that hold a projection's h_out * r elements (at most r)
+__device__ __forceinline__ int expand_pages(const ExpandArgs& p, int proj, int r) {
+  const int sh = p.pages_shift[proj];
+  int n_pg = r;
+  if (sh >= 0)
+    n_pg = (r + (1 << sh) - 1) >> sh;
+  else if (sh == -2)
+    n_pg = r > 512 ? (int)(((int64_t)p.h_out[proj] * r + p.page_elems - 1) / p.page_elems)
+                   : (int)(((uint32_t)p.h_out[proj] * (uint32_t)r + (uint32_t)p.page_elems - 1u) /
+                           (uint32_t)p.page_elems);
+  return n_pg > r ? r : n_pg;
 }
 
 // Expand has nothing to share between wavefronts (the delta row is 16 bytes per
@@ -757,7 +772,7 @@ __device__ __forceinline__ void expand_one(const ExpandArgs& p, int proj, const 
 // Grid: x = item (planned) or token * blocks + block (stateless), y = projection * 2 +
 // half: workgroup ids run item-fastest, so with a multiple of 8 items every workgroup of
 // an item lands on XCD item % 8.
-template <typename T, int NPROJ, bool PLANNED, int NV, bool COH = false>
+template <typename T, int NPROJ, bool PLANNED, int NV>
 __device__ __forceinline__ int expand_body(const ExpandArgs& p, int unit, int sub, uint16_t* s_strip) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int proj = sub >> 1;
@@ -777,16 +792,7 @@ __device__ __forceinline__ int expand_body(const ExpandArgs& p, int unit, int su
   const int r_eff = r < p.x_cols ? r : p.x_cols;
   if (r_eff <= 0) return it.plan_items;
   const int k = it.j0 + jr;
-  // pages that hold this projection's h_out * r elements
-  const int sh = p.pages_shift[proj];
-  int n_pg = r;
-  if (sh >= 0)
-    n_pg = (r + (1 << sh) - 1) >> sh;
-  else if (sh == -2)
-    n_pg = r > 512 ? (int)(((int64_t)p.h_out[proj] * r + p.page_elems - 1) / p.page_elems)
-                   : (int)(((uint32_t)p.h_out[proj] * (uint32_t)r + (uint32_t)p.page_elems - 1u) /
-                           (uint32_t)p.page_elems);
-  if (n_pg > r) n_pg = r;
+  const int n_pg = expand_pages(p, proj, r);
   // Pages the launch does not enumerate: the stateless grid stops at the delta
   // width and a plan at rank_cap; an adapter of larger rank has more, which
   // the wavefronts of the last enumerated block take in further rounds.
@@ -803,12 +809,12 @@ __device__ __forceinline__ int expand_body(const ExpandArgs& p, int unit, int su
                       (p.page_elems & (8 * r - 1)) == 0 && (p.h_out[proj] & 7) == 0 && p.y_aligned != 0;
   if (k < n_pg) {
     const int64_t page = PLANNED ? (int64_t)plan_pg : (int64_t)-2;
-    expand_one<T, NV, COH>(p, proj, it, r_eff, k, page, vec_ok, s_strip);
+    expand_one<T, NV>(p, proj, it, r_eff, k, page, vec_ok, s_strip);
   }
   if (extra) {
 #pragma unroll 1
     for (int kk = k + kRB; kk < n_pg; kk += kRB)
-      expand_one<T, NV, COH>(p, proj, it, r_eff, kk, -2, vec_ok, s_strip);
+      expand_one<T, NV>(p, proj, it, r_eff, kk, -2, vec_ok, s_strip);
   }
   return it.plan_items;
 }
@@ -844,13 +850,21 @@ int64_t plan_max_items(int64_t batch, int64_t rank_cap) {
 }
 // int32 words of the builder's scratch area behind the items
 int64_t plan_scratch_words(int64_t batch) { return batch * SC_WORDS; }
-// int32 words of the hand-over counters behind the scratch area, and where they start
-int64_t plan_sync_words(int64_t batch) { return kSyncHeader + 4 * batch; }
-int64_t plan_sync_offset(int64_t batch, int64_t rank_cap) {
-  return kPlanHeaderWords + plan_max_items(batch, rank_cap) * kItemWords + plan_scratch_words(batch);
+// The hand-over area behind the scratch area: where it starts (16-byte aligned), the row pitch of its
+// tagged values, its size (a multiple of 4 words; 0: the plan has none)
+int64_t plan_hand_offset(int64_t batch, int64_t rank_cap) {
+  return (kPlanHeaderWords + plan_max_items(batch, rank_cap) * kItemWords + plan_scratch_words(batch) + 3) / 4 * 4;
+}
+int64_t plan_hand_pitch(int64_t rank_cap) { return (rank_cap + 7) / 8 * 8; }
+bool plan_hand_over(int64_t batch, int64_t rank_cap) {
+  return batch <= kHandTokens && batch * plan_hand_pitch(rank_cap) <= kHandEntries;
+}
+int64_t plan_hand_words(int64_t batch, int64_t rank_cap) {
+  if (!plan_hand_over(batch, rank_cap)) return 0;
+  return plan_max_items(batch, rank_cap) * kEpochWords + batch * 4 * plan_hand_pitch(rank_cap);
 }
 int64_t plan_words(int64_t batch, int64_t rank_cap) {
-  return plan_sync_offset(batch, rank_cap) + plan_sync_words(batch);
+  return plan_hand_offset(batch, rank_cap) + plan_hand_words(batch, rank_cap);
 }
 
 // Grid of a planned launch: the items the caller read back.  Without that count (a plan rebuilt

@@ -1,11 +1,10 @@
-// Decode shrink and expand of the same projections in one launch (see the comment in front
-// of LoraArgs).  A file of its own so that it compiles next to bgmv_decode.hip, whose device
-// code it shares through bgmv_device.hpp.
+// Decode shrink and expand of the same projections in one launch.  A file of its own so that it
+// compiles next to bgmv_decode.hip, whose device code it shares through bgmv_pages.hpp.
 //
 // Replaces the back-to-back dispatch_bgmv pairs of
 // slora/models/peft/lora_unordered_batch_infer.py:267-273, 287-293, 307-313, 438-444.
 
-#include "bgmv_device.hpp"
+#include "bgmv_pages.hpp"
 
 namespace slora {
 namespace {
@@ -14,207 +13,147 @@ namespace {
 // shrink and expand of the same projections in ONE launch
 // ---------------------------------------------------------------------------
 // The reference issues shrink and expand of a projection back to back
-// (slora/models/peft/lora_unordered_batch_infer.py:267-273): two launches, the second of
-// which cannot start before the first has drained.  Here one workgroup per item does both
-// halves of its item: the shrink of its 8 rows (shrink_body, unchanged), then the 8 pages of
-// B^T with the same page ids (expand_body, unchanged: wavefront w takes pages w and w + 4).
-// An expand page needs the whole delta row of its run, i.e. the rows of ALL items of the run
-// (rank / 8 workgroups): the hand-over between them is one counter per (run, projection)
-// behind the plan.  A workgroup stores its rows with device-scope stores, waits for them,
-// counts itself in and polls until the run's `need` workgroups of this launch have done so;
-// then it reads the rows with device-scope loads.  The counter is never reset: it grows by
-// `need` per launch, launches on one plan do not overlap, so the value a workgroup's own
-// increment returns tells which launch this is ((old / need + 1) * need is the count to wait
-// for).  Producers and consumers are the same workgroups, and the items of a run are
-// neighbours in their XCD's queue: workgroups are handed out in index order, so whoever a
-// workgroup waits for is resident or about to be as soon as anything finishes.  The wait is
-// bounded all the same (spin_limit polls, then a sticky flag in the counters' header and the
-// workgroup goes on) so that no wavefront can wait for ever.
-struct LoraArgs {
-  ShrinkArgs s;
-  ExpandArgs e;
-  int* sync;       // the plan's counters
-  int rank_cap;    // of the plan: a run has ceil(min(rank, rank_cap) / 8) items
-  int spin_limit;  // polls after which a waiting workgroup gives up
-};
-
-// First half of the hand-over, called by all threads of the workgroup after its shrink rows
-// are stored: waits for the stores, meets, counts the workgroup in.  Returns (in wavefront 0)
-// the count to wait for; 0 if the run has no other workgroup.
-__device__ __forceinline__ int lora_arrive(const LoraArgs& p, const Item& it, int proj_abs) {
-  const int listed = it.r < p.rank_cap ? it.r : p.rank_cap;
-  const int need = (listed + kRB - 1) / kRB;
-  // wait until the stores of this wavefront are acknowledged (vmcnt(0); a workgroup-scope fence
-  // alone need not wait for global stores), i.e. have reached the level the other workgroups read from
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  __builtin_amdgcn_s_waitcnt(0x0F70);
-  __syncthreads();
-  int target = 0;
-  if (need > 1 && threadIdx.x == 0) {
-    int* cnt = p.sync + kSyncHeader + ((int64_t)it.tok[0] * 4 + proj_abs);
-    const int old = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    target = (old / need + 1) * need;
-  }
-  return target;
-}
-
-// Second half: wavefront 0 polls until the run's workgroups of this launch have all counted
-// in (bounded), then the workgroup meets again.
-__device__ __forceinline__ void lora_wait(const LoraArgs& p, const Item& it, int proj_abs, int target) {
-  if (threadIdx.x < kWave) {
-    target = __builtin_amdgcn_readfirstlane(target);
-    if (target != 0) {
-      const int* cnt = p.sync + kSyncHeader + ((int64_t)it.tok[0] * 4 + proj_abs);
-      int spins = 0;
-      while (__hip_atomic_load(cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - target < 0) {
-        if (++spins > p.spin_limit) {  // never expected; leaves a mark instead of waiting for ever
-          if (threadIdx.x == 0) {
-            p.sync[SY_TIMEOUT] = 1;
-            __hip_atomic_fetch_or(const_cast<int*>(p.s.plan) + PH_STATUS, kPlanStatusTimeout, __ATOMIC_RELAXED,
-                                  __HIP_MEMORY_SCOPE_AGENT);
-          }
-          break;
-        }
-        __builtin_amdgcn_s_sleep(4);
-      }
+// (slora/models/peft/lora_unordered_batch_infer.py:267-273): two launches, the second of which cannot
+// start before the first has drained, and both pay a launch, a record and the way of the first data.
+// Here the grid holds the workgroups of both: first those of the shrink (an item's 8 rows of one
+// projection each), then those of the expand (half of an item's 8 pages of
+// B^T each).  Workgroups are handed out in that order and the first kind waits for nobody, so whatever a
+// workgroup of the second kind waits for is running or done.  It has its pages and its y values on
+// the way before it looks for the delta rows of its run.
+//
+// Hand-over: the value of a delta row's column travels in a word of its own behind the plan, (value | launch
+// << 16), written with a device-scope store and read with device-scope loads; a reader repeats its loads until
+// every word names this launch.  No counter, no wait for a store to be acknowledged and no second
+// round trip stand between a producer's last product and the reader's arithmetic.  Which launch this is
+// every workgroup knows from a word that nobody else writes (the launches it has taken part in), so the
+// area is cleared by the plan build only and launches may be replayed.  Launches on one plan must not overlap.
+//
+// The wait is bounded: after spin_limit polls a wavefront computes the rows of its run itself (pages_general)
+// and leaves a mark in the plan's status word.
+//
+// What it took: a form whose every workgroup did both halves ran 44 us for q, k and v of S2's 256 tokens; this
+// arrangement with the general paths inlined 62, without them 36, with one polling load per token and workgroup
+// instead of every lane reading all its columns (the polls kept the shrink's own loads waiting) 33.
+//
+// Grid, two forms (see bgmv_expand_kernel): two-dimensional, x = item, y < nproj: shrink of projection y, else expand
+// half y - nproj; one-dimensional (INTERLEAVE): the shrinks projection by projection, then the expand
+// workgroups of an item one after the other.  LDS: the shrink's staging area, or a strip per wavefront
+// and token and the delta rows.
+template <typename T, int NV, bool INTERLEAVE>
+__global__ __launch_bounds__(256, NV > 12 ? 2 : (NV > 8 ? 3 : 4)) void bgmv_lora_kernel(const PageArgs) {
+  extern __shared__ u32x4 s_x[];  // [kTT][h_in / 8]
+  const PageArgs& p = page_args();
+  int unit = (int)blockIdx.x, sub = (int)blockIdx.y;
+  if (INTERLEAVE) {
+    if (unit < p.n_units * p.nproj) {
+      sub = unit / p.n_units;
+      unit -= sub * p.n_units;
+    } else {
+      const int S = 2 * p.nproj, id = unit - p.n_units * p.nproj, g = id >> 3;
+      unit = (g / S) * 8 + (id & 7);
+      sub = p.nproj + g % S;
     }
   }
-  __syncthreads();
-  // the rows are read with device-scope loads; keep them behind the wait
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-}
-
-template <typename T, int NV>
-__device__ __forceinline__ int lora_body(const LoraArgs& p, int unit, int proj, u32x4* s_x, uint16_t* s_strip) {
-  Item it;
-  const int n_items = shrink_body<T, true, NV, true>(p.s, unit, proj, s_x, it);
-  if (it.n_tok <= 0) return n_items;  // no such item (uniform over the workgroup)
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int proj_abs = p.s.qkvo0 + proj;
-  const int r = it.r;
-  const ExpandArgs& e = p.e;
-  // The usual case in straight-line code: both pages of this wavefront (w and w + 4 of the item's
-  // block) are whole one-pass pages inside the output, on the vector path.  Their loads and the y
-  // values go out between the two halves of the hand-over, so they are in flight while it completes.
-  const bool fast = (r & (r - 1)) == 0 && r >= 8 && r <= 128 && r <= e.x_cols && it.more == 0 && (e.x_cols & 7) == 0 &&
-                    e.page_elems == ExpandPass<NV>::kElems && e.pages_shift[proj] == -1 && (e.h_out[proj] & 7) == 0 &&
-                    e.y_aligned != 0;
-  const int target = lora_arrive(p, it, proj_abs);
-  if (!fast) {
-    lora_wait(p, it, proj_abs, target);
-    expand_body<T, 1, true, NV, true>(e, unit, proj * 2, s_strip);
-    expand_body<T, 1, true, NV, true>(e, unit, proj * 2 + 1, s_strip);
-    return n_items;
-  }
-  const int lg_r = __builtin_ctz((unsigned)r);
-  const int h_stride = e.h_out[proj];
-  const uint16_t* y = reinterpret_cast<const uint16_t*>(e.y[proj]);
-  typedef const int __attribute__((address_space(4))) * ConstWords;
-  ConstWords rec = (ConstWords)p.s.plan + kPlanHeaderWords + (int64_t)unit * kItemWords;
-  int pg[2];
-  u32x4 wv[2][NV], yv[2][kTT];
-  int n_page0[2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    pg[i] = rec[IT_PAGES + proj_abs * kRB + wave + 4 * i];
-    const uint16_t* wpage = reinterpret_cast<const uint16_t*>(e.w) + (int64_t)(pg[i] >= 0 ? pg[i] : 0) * e.page_elems;
-#pragma unroll
-    for (int c = 0; c < NV; ++c) wv[i][c] = ldg16_stream(wpage + (c * kWave + lane) * 8);
-  }
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int k = it.j0 + wave + 4 * i;
-    n_page0[i] = (int)(((int64_t)k * e.page_elems) >> lg_r);
-    const bool y_ok = lane * 8 < (ExpandPass<NV>::kElems >> lg_r);
-#pragma unroll
-    for (int t = 0; t < kTT; ++t)  // lanes with no outputs re-read the page's first ones; the values are not used
-      yv[i][t] = ldg16_stream(y + (int64_t)(t < it.n_tok ? it.tok[t] : it.tok[0]) * h_stride +
-                              (y_ok ? n_page0[i] + lane * 8 : n_page0[i]));
-  }
-  const float scale = load_scale(e.scales, e.scales_dtype, it.a);
-  lora_wait(p, it, proj_abs, target);
-  const int d0 = (lane & ((r >> 3) - 1)) * 8;
-  const uint16_t* x = reinterpret_cast<const uint16_t*>(e.x[proj]);
-  u32x4 xv[kTT];
-#pragma unroll
-  for (int t = 0; t < kTT; ++t)
-    xv[t] = ldg16_coherent(x + (int64_t)(t < it.n_tok ? it.tok[t] : it.tok[0]) * e.x_cols + d0);
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    if (pg[i] >= 0)
-      expand_update<T, NV>(e, proj, it, lg_r, wv[i], xv, yv[i], n_page0[i], h_stride, scale, s_strip);
-  }
-  return n_items;
-}
-
-// Grid: x = item, y = projection of the launch.  LDS: the shrink's staging area (dynamic) and a
-// strip per wavefront for the expand.
-template <typename T, int NV>
-__global__ __launch_bounds__(256, NV > 8 ? 3 : 4) void bgmv_lora_kernel(const LoraArgs p) {
-  extern __shared__ u32x4 s_x[];  // [lds_tt][h_in / 8]
-  __shared__ __align__(16) uint16_t s_out[4][ExpandPass<NV>::kStrip];
-  int unit = (int)blockIdx.x;
-  const int n_items = lora_body<T, NV>(p, unit, (int)blockIdx.y, s_x, s_out[threadIdx.x >> 6]);
-  if (p.s.strided) {  // the items beyond the grid, if the batch has that many
-    for (unit += (int)gridDim.x; unit < n_items; unit += (int)gridDim.x) {
+  if (sub < p.nproj) {
+    for (;;) {
+      const int n_items = pages_shrink<T, NV, true>(p, unit, sub, s_x);
+      // a launch sized for a fraction of the plan's capacity: the items beyond the grid, if the batch has that many
+      unit += p.n_units;
+      if (!p.strided || unit >= n_items) return;
       __syncthreads();  // the staging area of the item before is free
-      lora_body<T, NV>(p, unit, (int)blockIdx.y, s_x, s_out[threadIdx.x >> 6]);
     }
+  }
+  sub -= p.nproj;
+  uint16_t* s_strip = reinterpret_cast<uint16_t*>(s_x) + (threadIdx.x >> 6) * (kTT * ExpandPass<NV>::kStrip);
+  uint32_t* s_delta = reinterpret_cast<uint32_t*>(reinterpret_cast<uint16_t*>(s_x) + 4 * kTT * ExpandPass<NV>::kStrip);
+  for (;;) {
+    const int n_items = pages_expand<T, NV, true>(p, unit, sub, s_strip, s_delta);
+    unit += p.n_units;
+    if (!p.strided || unit >= n_items) return;
+    __syncthreads();  // the delta rows of the item before have been read
   }
 }
 
 template <typename T, int NV>
-int launch_lora_nv(const LoraArgs& p, int64_t grid, int nproj, size_t lds, hipStream_t stream) {
-  auto kernel = bgmv_lora_kernel<T, NV>;
-  static PerDeviceOnce once;
-  if (lds > 48 * 1024 && !raise_dynamic_lds(reinterpret_cast<const void*>(kernel), 128 * 1024, once))
-    return SLORA_ERR_LAUNCH;
-  hipLaunchKernelGGL(kernel, dim3((uint32_t)grid, (uint32_t)nproj), dim3(256), lds, stream, p);
+int launch_lora(const PageArgs& p, hipStream_t stream) {
+  auto kernel = p.interleave ? bgmv_lora_kernel<T, NV, true> : bgmv_lora_kernel<T, NV, false>;
+  constexpr size_t strips = 4 * kTT * ExpandPass<NV>::kStrip * sizeof(uint16_t) + kDeltaBytes;
+  constexpr size_t staging = (size_t)kTT * ExpandPass<NV>::kElems * 2, lds = strips > staging ? strips : staging;
+  static PerDeviceOnce once[2];
+  if (!raise_dynamic_lds(reinterpret_cast<const void*>(kernel), (int)lds, once[p.interleave])) return SLORA_ERR_LAUNCH;
+  dim3 grid((uint32_t)p.n_units, 3 * p.nproj);
+  if (p.interleave) grid = dim3((uint32_t)(p.n_units * 3 * p.nproj), 1);
+  hipLaunchKernelGGL(kernel, grid, dim3(256), lds, stream, p);
   return hipGetLastError() == hipSuccess ? SLORA_OK : SLORA_ERR_LAUNCH;
 }
 
 template <typename T>
-int launch_lora(LoraArgs p, int64_t grid, int nproj, hipStream_t stream) {
-  if (grid <= 0) return SLORA_OK;
-  if (grid > 0x7fffffffLL / 8) return SLORA_ERR_UNSUPPORTED;
-  const size_t row_bytes = (size_t)p.s.h_in * 2;
-  int tt = kTT;
-  while (tt > 1 && tt * row_bytes > 64 * 1024) --tt;
-  const size_t lds = tt * row_bytes;
-  if (lds > 128 * 1024 - 8 * 1024) return SLORA_ERR_UNSUPPORTED;
-  p.s.lds_tt = tt;
-  p.e.n_units = (int)grid;
-  p.e.interleave = 0;
-  // Only the 4096-element pass is instantiated: wider pages take the same kernel's general paths
-  // (several passes per page), correct and slower.
-  return launch_lora_nv<T, 8>(p, grid, nproj, lds, stream);
+int dispatch_lora(const PageArgs& p, int64_t page_elems, hipStream_t stream) {
+  switch (page_elems / (8 * kWave)) {
+    case 8: return launch_lora<T, 8>(p, stream);
+    case 10: return launch_lora<T, 10>(p, stream);
+    case 12: return launch_lora<T, 12>(p, stream);
+    default: return launch_lora<T, 16>(p, stream);
+  }
+}
+
+// Whether one launch serves the call (whole one-pass pages, and a plan with a hand-over area whose launches put the
+// workgroups of an item on its XCD), and is the faster form.  us, one launch against two, shrink + expand of q, k and v
+// and in brackets of o; `units` items each:
+//   rank 8, hidden 4096: 1 item 4.7 / 6.4 (4.6 / 6.6), 40 9.0 / 9.6 (7.1 / 9.1), 79 10.0 / 11.1 (7.4 / 9.2), 218 20.6 / 22.8 (9.5 / 11.8);
+//   5120: 62 13.4 / 14.4 (9.9 / 11.8); 8192: 67 13.7 / 15.3 (11.3 / 13.2);
+//   ranks 8 to 64, 4096: 37 8.6 / 8.7 (7.3 / 7.3), 60 14.5 / 13.1 (8.6 / 9.0), 108 14.5 / 13.7 (9.2 / 9.0), 147 17.0 / 17.1 (10.7 / 10.0),
+//   231 20.3 / 21.9 (13.6 / 12.7), 480 32.7 / 33.8 (14.7 / 15.5), 623 41.5 / 41.9 (20.2 / 19.1), 1093 74.5 / 72.4 (27.4 / 28.8);
+//   5120: 33 9.7 / 10.0 (7.4 / 8.2), 86 20.8 / 16.1 (11.3 / 12.0), 1214 103 / 98.5 (37.3 / 37.7);
+//   8192, k and v 1024 wide: 24 10.1 / 11.2 (7.9 / 9.2), 51 11.9 / 14.6 (8.7 / 10.1), 150 22.2 / 24.4 (13.4 / 14.3), 263 31.4 / 31.3
+//   (18.4 / 20.1), 607 63.3 / 60.2 (31.8 / 32.6).
+// A small launch saves the second launch, record and first data.  With every workgroup resident at once the expand's pages
+// compete with the shrink's, and a run of rank 64 waits for the slowest of eight workgroups: in the middle range
+// the two launches are level or better where ranks go beyond 16.  Where the shrink alone fills the chip the expand's
+// workgroups follow it in order and find their rows ready; several rounds of either hide the boundary anyway.
+bool lora_one_launch(const ExpandArgs& e, int64_t h_in, int64_t batch, int64_t rank_cap, int64_t units, int nproj) {
+  if (h_in != e.page_elems || !pages_serve(e, nproj, rank_cap) || !plan_hand_over(batch, rank_cap) || units % kXcds != 0)
+    return false;
+  const int64_t shrinks = units * nproj;  // workgroups
+  if (shrinks <= 128 || e.x_cols <= 16) return shrinks <= 1536;
+  if (e.page_elems == ExpandPass<8>::kElems) return shrinks >= 448 && shrinks <= 1536;
+  return e.page_elems == ExpandPass<16>::kElems && shrinks <= 512;
 }
 
 int lora_common(const void* plan, int64_t n_items, int64_t rank_cap, void* const y[3], void* const delta[3],
                 const int64_t h_out[3], int nproj, int qkvo0, const void* x, const void* wa, const void* wb,
                 const slora_tables* tables, const int64_t* bins, const void* scales, int scales_dtype, int64_t batch,
                 int64_t h_in, int64_t delta_cols, int64_t page_elems, int64_t n_pages, int dtype, void* stream) {
-  LoraArgs p{};
+  ShrinkArgs s{};
+  PageArgs p{};
   int64_t grid_s = 0, grid_e = 0;
   int rc = shrink_prepare(plan, n_items, rank_cap, delta, nproj, qkvo0, x, wa, tables, bins, batch, h_in, delta_cols,
-                          page_elems, n_pages, dtype, p.s, grid_s);
+                          page_elems, n_pages, dtype, s, grid_s);
   if (rc != SLORA_OK) return rc == kNothingToDo ? SLORA_OK : rc;
   const void* xs[3] = {delta[0], delta[1], delta[2]};
   rc = expand_prepare(plan, n_items, rank_cap, y, xs, h_out, nproj, qkvo0, wb, tables, bins, scales, scales_dtype,
                       batch, delta_cols, page_elems, n_pages, dtype, p.e, grid_e);
-  if (rc == kNothingToDo)  // no output to update: the shrink half alone
-    return slora_bgmv_shrink_planned(plan, rank_cap, n_items, nproj, delta[0], delta[1], delta[2], x, wa, tables, bins,
-                                     batch, h_in, delta_cols, page_elems, n_pages, qkvo0, dtype, stream);
-  if (rc != SLORA_OK) return rc;
-  if (grid_s != grid_e) return SLORA_ERR_BAD_SHAPE;
+  const bool expands = rc != kNothingToDo;
+  if (expands && rc != SLORA_OK) return rc;
   // the delta rows are read 8 bytes at a time by device-scope loads
   if ((delta_cols & 7) != 0) return SLORA_ERR_UNSUPPORTED;
-  p.sync = const_cast<int*>(static_cast<const int*>(plan)) + plan_sync_offset(batch, rank_cap);
-  p.rank_cap = (int)rank_cap;
-  p.spin_limit = 1 << 16;
-  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  return dtype == SLORA_DTYPE_F16 ? launch_lora<F16>(p, grid_s, nproj, s) : launch_lora<BF16>(p, grid_s, nproj, s);
+  if (!expands || !lora_one_launch(p.e, h_in, batch, rank_cap, grid_s, nproj)) {
+    rc = slora_bgmv_shrink_planned(plan, rank_cap, n_items, nproj, delta[0], delta[1], delta[2], x, wa, tables, bins, batch,
+                                   h_in, delta_cols, page_elems, n_pages, qkvo0, dtype, stream);
+    if (rc != SLORA_OK || !expands) return rc;
+    return slora_bgmv_expand_planned(plan, rank_cap, n_items, nproj, y[0], y[1], y[2], xs[0], xs[1], xs[2], wb, tables, bins,
+                                     scales, scales_dtype, batch, delta_cols, h_out[0], h_out[1], h_out[2], page_elems,
+                                     n_pages, qkvo0, dtype, stream);
+  }
+  fill_pages_shrink(p, s, nproj);
+  fill_pages_expand(p, p.e, nproj);
+  p.epochs = const_cast<int*>(p.plan) + plan_hand_offset(batch, rank_cap);
+  p.words = reinterpret_cast<uint32_t*>(p.epochs + plan_max_items(batch, rank_cap) * kEpochWords);
+  p.pitch = (int)plan_hand_pitch(rank_cap);
+  p.spin_limit = 1 << 14;
+  p.n_units = (int)grid_s;
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  return dtype == SLORA_DTYPE_F16 ? dispatch_lora<F16>(p, page_elems, st) : dispatch_lora<BF16>(p, page_elems, st);
 }
 
 }  // namespace

@@ -501,7 +501,7 @@ void dispatch_bgmv_qkv_expand(const Tensor& y_q, const Tensor& y_k, const Tensor
   check_rc(rc, "dispatch_bgmv_qkv_expand");
 }
 
-// Shrink and expand of one projection in one launch: delta = x A (left in `delta`), y += scale * delta B.
+// Shrink and expand of one projection in one call (one launch where that is faster): delta = x A (left in `delta`), y += scale * delta B.
 // With plan=False (or no plan for the batch) the two stateless launches are issued instead.
 void dispatch_bgmv_lora(const Tensor& y, const Tensor& delta, const Tensor& x, const Tensor& w_a, const Tensor& w_b,
                         const Tensor& start_indicies, const Tensor& lora_ranks, const Tensor& loc_indicies,
@@ -1169,7 +1169,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
       .def_readonly("n_runs", &BgmvPlan::n_runs)
       .def("status", [](const BgmvPlan& pl) { return plan_status_of(pl.buf); },
            "status word of the plan (waits for the current stream): 0, or bit 0 = a launch named another batch "
-           "size or rank cap and did nothing, bit 1 = a hand-over of the one-launch LoRA was abandoned");
+           "size or rank cap and did nothing, bit 1 = a hand-over of the one-launch LoRA took too long and its rows were "
+           "computed a second time");
   py::class_<SgmmPlan, std::shared_ptr<SgmmPlan>>(m, "SgmmPlan")
       .def_readonly("buf", &SgmmPlan::buf)
       .def_readonly("usable", &SgmmPlan::usable)

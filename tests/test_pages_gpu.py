@@ -1,0 +1,104 @@
+"""The decode kernels for pages of exactly one pass (hidden 4096, 5120, 6144 or 8192): planned shrink and expand, and
+both in one launch, bit for bit against the calls without a plan (kernels of their own) over the forms the launches
+accept: run lengths 1 to 4, ranks on and off the vector path, grouped-query outputs, pages that do not exist, delta
+narrower than the rank, an output that is not 16-byte aligned, launches with and without an item count."""
+import numpy as np
+import pytest
+import torch
+
+from lora_cases import make_case
+from test_bgmv_gpu import GpuCase
+
+pytestmark = pytest.mark.gpu
+
+
+def _outputs(c, g, gpu, aligned):
+    gen = torch.Generator(device=gpu)
+    gen.manual_seed(7)
+    out = []
+    for h in c.h_out:
+        flat = torch.empty(c.batch * h + 8, dtype=g.tdt, device=gpu).normal_(generator=gen)
+        out.append(flat[0 if aligned else 4:][: c.batch * h].view(c.batch, h))
+    return out
+
+
+def _fresh(c, g, gpu, y0, R, aligned):
+    y = _outputs(c, g, gpu, aligned)
+    for a, b in zip(y, y0):
+        a.copy_(b)
+    return y, [torch.full((c.batch, R), 0.5, dtype=g.tdt, device=gpu) for _ in range(4)]
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("hidden,ranks,batch,h_out,R,aligned", [
+    (4096, [64, 8, 16, 32, 128], 11, None, 128, True),
+    (4096, [8], 4, None, 8, True),                             # one run of four tokens, one item
+    (4096, [16, 8], 41, [4096, 512, 512, 4096], 16, True),     # one launch at any size; k and v an eighth of a page
+    (4096, [64, 24, 4, 12, 8], 9, None, 64, True),             # ranks off the vector path
+    (4096, [64, 32, 8], 9, None, 16, True),                    # delta narrower than the rank
+    (4096, [64, 8], 7, None, 64, False),
+    (5120, [64, 8, 16], 7, None, 64, True),
+    (6144, [8, 16], 13, None, 16, True),
+    (8192, [64, 8, 32], 10, [8192, 1024, 1024, 8192], 64, True),
+    (8192, [16, 8], 130, None, 16, True),                      # workgroups that walk several items
+])
+def test_whole_page_launches_equal_the_calls_without_a_plan(gpu, dtype, hidden, ranks, batch, h_out, R, aligned):
+    import slora_hip
+    from slora_hip import (dispatch_bgmv, dispatch_bgmv_lora, dispatch_bgmv_qkv_expand, dispatch_bgmv_qkv_lora,
+                           dispatch_bgmv_qkv_shrink)
+    c = make_case(500 + hidden + batch + R, hidden, ranks, batch, dtype=dtype, h_out=h_out, zipf_alpha=1.0)
+    c.bins[batch // 2] = -1                                     # a token without an adapter
+    c.a_loc[int(c.a_start[0]) + 1] = c.n_pages + 3              # a page outside the pool
+    g = GpuCase(c, gpu)
+    t = (g.a_start, g.a_len, g.a_loc, g.bins)
+    y0 = [v.clone() for v in _outputs(c, g, gpu, True)]
+    y_s, d_s = _fresh(c, g, gpu, y0, R, aligned)
+    for p in range(4):
+        dispatch_bgmv(d_s[p], g.x, g.key, *t, p, g.scales, plan=False)
+        dispatch_bgmv(y_s[p], d_s[p], g.value, *t, p, g.scales, plan=False)
+    for readback in (True, False):
+        plan = slora_hip.make_plan(*t, R, c.n_pages, readback=readback)
+        for rep in range(3):
+            print(f"{dtype} hidden {hidden} batch {batch} R {R} readback {readback} rep {rep}", flush=True)
+            y, d = _fresh(c, g, gpu, y0, R, aligned)
+            dispatch_bgmv_qkv_shrink(*d[:3], g.x, g.key, *t, plan=plan)
+            dispatch_bgmv_qkv_expand(*y[:3], *d[:3], g.value, *t, g.scales, plan=plan)
+            dispatch_bgmv(d[3], g.x, g.key, *t, 3, g.scales, plan=plan)
+            dispatch_bgmv(y[3], d[3], g.value, *t, 3, g.scales, plan=plan)
+            for p in range(4):
+                assert torch.equal(d[p], d_s[p]) and torch.equal(y[p], y_s[p]), (p, "two launches")
+            y, d = _fresh(c, g, gpu, y0, R, aligned)
+            dispatch_bgmv_qkv_lora(*y[:3], *d[:3], g.x, g.key, g.value, *t, g.scales, plan=plan)
+            dispatch_bgmv_lora(y[3], d[3], g.x, g.key, g.value, *t, 3, g.scales, plan=plan)
+            for p in range(4):
+                assert torch.equal(d[p], d_s[p]) and torch.equal(y[p], y_s[p]), (p, "one launch")
+        assert plan.status() == 0
+
+
+def test_a_hand_over_that_never_comes_is_computed(gpu):
+    """The word that counts a shrink workgroup's launches is changed in the plan, so that its rows name a launch nobody
+    waits for: the readers give up after their poll limit, compute the rows themselves and mark the plan."""
+    import slora_hip
+    from slora_hip import dispatch_bgmv, dispatch_bgmv_lora
+    c = make_case(9, 4096, [16, 8], 6, dtype="f16", bins=[0, 0, 1, 0, 0, 0])
+    g = GpuCase(c, gpu)
+    t = (g.a_start, g.a_len, g.a_loc, g.bins)
+    R = 16
+    gen = torch.Generator(device=gpu)
+    gen.manual_seed(3)
+    y0 = torch.empty((c.batch, 4096), dtype=g.tdt, device=gpu).normal_(generator=gen)
+    d_s, y_s = torch.zeros((c.batch, R), dtype=g.tdt, device=gpu), y0.clone()
+    dispatch_bgmv(d_s, g.x, g.key, *t, 3, g.scales, plan=False)
+    dispatch_bgmv(y_s, d_s, g.value, *t, 3, g.scales, plan=False)
+    plan = slora_hip.make_plan(*t, R, c.n_pages)
+    per_run = R // 8
+    items = (c.batch * per_run + 7) // 8 * 8 + 8 * (per_run + 1)
+    area = (16 + items * 48 + c.batch * 6 + 3) // 4 * 4         # behind header, records and scratch
+    words = plan.buf.cpu().numpy()
+    unit = next(u for u in range(plan.n_items) if words[16 + u * 48 + 2] > 0)   # an item with tokens
+    plan.buf[area + unit * 16 + 3 * 3] = 7                      # projection o, workgroup of the shrink
+    d, y = torch.zeros_like(d_s), y0.clone()
+    dispatch_bgmv_lora(y, d, g.x, g.key, g.value, *t, 3, g.scales, plan=plan)
+    torch.cuda.synchronize()
+    assert torch.equal(y, y_s) and torch.equal(d, d_s)
+    assert plan.status() == 2
