@@ -28,8 +28,9 @@ from typing import List, Optional, Sequence
 
 import torch
 
-from ._kernels import (dispatch_bgmv, dispatch_bgmv_qkv_expand, dispatch_bgmv_qkv_shrink, lora_get_qkvo_fwd_expand,
-                       lora_get_qkvo_fwd_expand_qkv, lora_get_qkvo_fwd_shrink, lora_get_qkvo_fwd_shrink_qkv)
+from ._kernels import (dispatch_bgmv, dispatch_bgmv_lora, dispatch_bgmv_qkv_expand, dispatch_bgmv_qkv_lora,
+                       dispatch_bgmv_qkv_shrink, lora_get_qkvo_fwd_expand, lora_get_qkvo_fwd_expand_qkv,
+                       lora_get_qkvo_fwd_shrink, lora_get_qkvo_fwd_shrink_qkv)
 
 # lora_unordered_batch_infer.py:334: in the reference the segmented kernels serve batches with a long
 # request, adapters of rank >= 64 and at least two requests, and everything else is BGMV
@@ -199,6 +200,11 @@ class LoraUnorderedBatchInfer:
             return None
         return (ia.a_loc, ia.a_start, ia.a_len, *self._prompts, self.req_bins), self._longest
 
+    def _one_call(self, key: torch.Tensor, val: torch.Tensor) -> bool:
+        """Whether the per-token shrink and expand of a layer go out as one call (which wants whole 16-byte pieces of
+        delta and pools of one shape): the same bits as the two."""
+        return self.fused and self.max_lora_dim % 8 == 0 and key.shape == val.shape
+
     # ---- q, k, v of one layer (:254-318 decode, :321-408 prefill) --------------------------
     def lora_get_qkv(self, layer_id: int, input_embs: torch.Tensor, q: torch.Tensor, cache_k: torch.Tensor,
                      cache_v: torch.Tensor) -> None:
@@ -234,7 +240,9 @@ class LoraUnorderedBatchInfer:
                                          self.max_lora_dim, longest)
             return
         tabs = (ia.a_start, ia.a_len, ia.a_loc, self._bins)
-        if self.fused:
+        if self._one_call(key, val):
+            dispatch_bgmv_qkv_lora(q, cache_k, cache_v, d[0], d[1], d[2], input_embs, key, val, *tabs, ia.a_scaling)
+        elif self.fused:
             dispatch_bgmv_qkv_shrink(d[0], d[1], d[2], input_embs, key, *tabs)
             dispatch_bgmv_qkv_expand(q, cache_k, cache_v, d[0], d[1], d[2], val, *tabs, ia.a_scaling)
         else:
@@ -260,5 +268,8 @@ class LoraUnorderedBatchInfer:
                                      longest)
             return
         tabs = (ia.a_start, ia.a_len, ia.a_loc, self._bins)
+        if self._one_call(key, val) and self.max_lora_dim < min(input.shape[1], o.shape[1]):
+            dispatch_bgmv_lora(o, d, input, key, val, *tabs, 3, ia.a_scaling)
+            return
         dispatch_bgmv(d, input, key, *tabs, 3, ia.a_scaling)
         dispatch_bgmv(o, d, val, *tabs, 3, ia.a_scaling)
