@@ -91,20 +91,6 @@ struct ExpandHot {
   }
 };
 
-// The word of the scale table that holds adapter a's entry, read without a branch, and the entry itself out of it: the
-// type is looked at where the value is needed, not in front of the weights.  (The word may hold a neighbour; it is
-// part of the table's allocation, which starts on four bytes.)
-__device__ __forceinline__ uint32_t scale_word(const void* scales, int dtype, int64_t a) {
-  const uint64_t at = (uint64_t)scales + (uint64_t)a * (dtype == SLORA_DTYPE_F32 ? 4u : 2u);
-  return *(const uint32_t __attribute__((address_space(4)))*)(at & ~(uint64_t)3);
-}
-__device__ __forceinline__ float scale_of(uint32_t word, const void* scales, int dtype, int64_t a) {
-  if (dtype == SLORA_DTYPE_F32) return __uint_as_float(word);
-  const uint64_t at = (uint64_t)scales + (uint64_t)a * 2u;
-  const uint16_t v = (uint16_t)(word >> ((at & 2) * 8));
-  return dtype == SLORA_DTYPE_F16 ? F16::to_float(v) : BF16::to_float(v);
-}
-
 // Runs whose pages are all whole one-pass pages inside the output, on the vector path.  In a one-launch LoRA (HAND) their
 // readers take delta from the tagged words; the others read delta itself, which their producers store, and wait for, in
 // front of the words.  (Both sides of the hand-over decide this from the run alone.)
