@@ -946,6 +946,27 @@ void lora_get_qkvo_fwd_expand_qkv(const Tensor& x_q, const Tensor& x_k, const Te
                  " max_rank=" + std::to_string(max_rank) + ")");
 }
 
+// Whether the segmented kernels serve a call of a prefill step whose tokens the reference gives to the per-token operator:
+// pools of the shape of the step's first one, 1-D tables, contiguous 16-byte aligned rows of at most a page.  What they
+// refuse (strided rows or pools, another row count) the per-token kernels still refuse, and what only those take (tables
+// that are not 1-D, pools of two page widths) they still take.
+bool segments_ok(const Tensor& first, const Tensor& key, const Tensor& val, const Tensor& a_loc, const Tensor& a_start,
+                 const Tensor& a_len, int64_t n_tok, int64_t width, const Tensor& x, const Tensor& out0,
+                 const c10::optional<Tensor>& out1, const c10::optional<Tensor>& out2) {
+  if (first.dim() != 3 || key.sizes() != first.sizes() || val.sizes() != first.sizes() || !key.is_contiguous() ||
+      !val.is_contiguous() || a_loc.dim() != 1 || a_start.dim() != 1 || a_len.dim() != 1)
+    return false;
+  const Tensor* rows[4] = {&x, &out0, out1.has_value() ? &*out1 : nullptr, out2.has_value() ? &*out2 : nullptr};
+  for (const Tensor* t : rows) {
+    if (t == nullptr) continue;
+    if (t->dim() != 2 || t->size(0) != n_tok || t->size(1) % 8 != 0 || t->size(1) > width ||
+        t->scalar_type() != first.scalar_type() || t->device() != first.device() || !t->is_contiguous() ||
+        (reinterpret_cast<uintptr_t>(t->data_ptr()) & 15) != 0)
+      return false;
+  }
+  return x.size(1) % 64 == 0;
+}
+
 // ---------------------------------------------------------------------------
 // pool helpers (slora/server/router/model_infer/infer_adapter.py, slora/common/mem_allocator.py)
 // ---------------------------------------------------------------------------
@@ -1239,6 +1260,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("make_prefill_plan", &make_prefill_plan, py::arg("b_lora_start"), py::arg("b_lora_ranks"), py::arg("b_start_loc"),
         py::arg("b_seq_len"), py::arg("b_indicies"), py::arg("n_tokens"), py::arg("max_rank"), py::arg("max_input_len"));
 
+  m.def("segments_ok", &segments_ok, py::arg("first"), py::arg("key"), py::arg("val"), py::arg("a_loc"), py::arg("a_start"),
+        py::arg("a_len"), py::arg("n_tok"), py::arg("width"), py::arg("x"), py::arg("out0"), py::arg("out1") = py::none(),
+        py::arg("out2") = py::none());
   m.def("load_rows_into_pool", &load_rows_into_pool, py::arg("buffers"), py::arg("rows"), py::arg("loc"));
   m.def("pack_transposed_into_pool", &pack_transposed_into_pool, py::arg("buffers"), py::arg("mats"), py::arg("first"),
         py::arg("dst_pitch"), py::arg("n_slot"), py::arg("loc"));
