@@ -31,8 +31,8 @@ HBM_PEAK_GBS = 8000.0
 # a plain 256 MiB copy: 2.000 and 1.000); keyed by (workload, batch, mode, kernel).
 # None where not measured.
 TRAFFIC_BYTES = {
-    ("s2", 256, "planned-fused", "bgmv_expand_kernel<F16, 3, true, 8>"): 81465122,  # 75173666 read + 6291456 written
-    ("s2", 256, "planned-fused", "bgmv_shrink_kernel<F16, true, 8>"): 70979806,  # the q/k/v launch
+    ("s2", 256, "planned-fused", "bgmv_expand_pages_kernel<F16, 8, false>"): 81347884,  # 75056428 read + 6291456 written
+    ("s2", 256, "planned-fused", "bgmv_shrink_pages_kernel<F16, 8>"): 70791311,  # the q/k/v launch
     ("c3", "sgmm_expand_walk_kernel<BF16, 2, 1>"): 281689745,  # 155663826 read + 126025919 written
     ("c3", "sgmm_expand_walk_kernel<BF16, 2, 3>"): 860943997,  # 482866722 read + 378077275 written
     ("c3", "sgmm_shrink_planned_kernel<BF16, 1, false, true>"): 142557796,  # 140588644 read + 1969152 written
@@ -155,24 +155,27 @@ def make_step(w, bufs, mode, keep_plan=False):
 
     nv = next((n for n in (8, 10, 12, 16) if w.hidden <= 512 * n), 8)  # the instantiation the library picks
     nv_e = nv if planned else 8   # the stateless expand keeps the 4096-element pass
-    sk, ek = f"bgmv_shrink_kernel<{ty}, {pl}, {nv}>", f"bgmv_expand_kernel<{ty}, %d, {pl}, {nv_e}>"
+    sk, eks = f"bgmv_shrink_kernel<{ty}, {pl}, {nv}>", {n: f"bgmv_expand_kernel<{ty}, {n}, {pl}, {nv_e}>" for n in (1, 3)}
+    if planned and w.hidden == 512 * nv:  # whole pages: kernels of their own
+        narrow = {n: str(min(w.h_out[:3] if n == 3 else w.h_out[3:]) < w.hidden).lower() for n in (1, 3)}
+        sk, eks = f"bgmv_shrink_pages_kernel<{ty}, {nv}>", {n: f"bgmv_expand_pages_kernel<{ty}, {nv}, {narrow[n]}>" for n in (1, 3)}
     if one_launch:
-        lk = f"bgmv_lora_kernel<{ty}, %d, {nv}>"
+        lk = f"bgmv_lora_kernel<{ty}, {nv}> (or the two kernels, where the library takes two launches)"
         families = {
-            "qkv_lora": (over_layers(qkv_lora), lk % 3, L, w.qkv_shrink_bytes() + w.qkv_expand_bytes()),
-            "o_lora": (over_layers(o_lora), lk % 1, L, w.shrink_bytes() + w.expand_bytes(w.h_out[3])),
+            "qkv_lora": (over_layers(qkv_lora), lk, L, w.qkv_shrink_bytes() + w.qkv_expand_bytes()),
+            "o_lora": (over_layers(o_lora), lk, L, w.shrink_bytes() + w.expand_bytes(w.h_out[3])),
         }
     elif fused:
         families = {
             "qkv_shrink": (over_layers(qkv_shrink), sk, L, w.qkv_shrink_bytes()),
             "o_shrink": (over_layers(shrink, 3), sk, L, w.shrink_bytes()),
-            "qkv_expand": (over_layers(qkv_expand), ek % 3, L, w.qkv_expand_bytes()),
-            "o_expand": (over_layers(expand, 3), ek % 1, L, w.expand_bytes(w.h_out[3])),
+            "qkv_expand": (over_layers(qkv_expand), eks[3], L, w.qkv_expand_bytes()),
+            "o_expand": (over_layers(expand, 3), eks[1], L, w.expand_bytes(w.h_out[3])),
         }
     else:
         families = {
             "shrink": (all_proj(shrink), sk, 4 * L, w.shrink_bytes()),
-            "expand": (all_proj(expand), ek % 1, 4 * L, sum(w.expand_bytes(h) for h in w.h_out) / 4),
+            "expand": (all_proj(expand), eks[1], 4 * L, sum(w.expand_bytes(h) for h in w.h_out) / 4),
         }
 
     def step():
