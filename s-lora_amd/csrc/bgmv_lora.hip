@@ -25,8 +25,9 @@ namespace {
 // << 16), written with a device-scope store and read with device-scope loads; a reader repeats its loads until
 // every word names this launch.  No counter, no wait for a store to be acknowledged and no second
 // round trip stand between a producer's last product and the reader's arithmetic.  Which launch this is
-// every workgroup knows from a word that nobody else writes (the launches it has taken part in), so the
-// area is cleared by the plan build only and launches may be replayed.  Launches on one plan must not overlap.
+// every workgroup knows from a word that nobody else writes (the launches it has taken part in; all of a run's take part
+// in every one-launch call on the plan, so they agree), so the area is cleared by the plan build only and launches may be
+// replayed.  Launches on one plan must not overlap.
 //
 // The wait is bounded: after spin_limit polls a wavefront computes the rows of its run itself (pages_general)
 // and leaves a mark in the plan's status word.
@@ -97,8 +98,8 @@ int dispatch_lora(const PageArgs& p, int64_t page_elems, hipStream_t stream) {
   }
 }
 
-// Whether one launch serves the call (whole one-pass pages, and a plan with a hand-over area whose launches put the
-// workgroups of an item on its XCD), and is the faster form.  us, one launch against two, shrink + expand of q, k and v
+// Whether one launch serves the call (whole one-pass pages, delta as wide as the plan, and a plan with a hand-over area whose
+// launches put the workgroups of an item on its XCD), and is the faster form.  us, one launch against two, shrink + expand of q, k and v
 // and in brackets of o; `units` items each:
 //   rank 8, hidden 4096: 1 item 4.7 / 6.4 (4.6 / 6.6), 40 9.0 / 9.6 (7.1 / 9.1), 79 10.0 / 11.1 (7.4 / 9.2), 218 20.6 / 22.8 (9.5 / 11.8);
 //   5120: 62 13.4 / 14.4 (9.9 / 11.8); 8192: 67 13.7 / 15.3 (11.3 / 13.2);
@@ -112,7 +113,10 @@ int dispatch_lora(const PageArgs& p, int64_t page_elems, hipStream_t stream) {
 // the two launches are level or better where ranks go beyond 16.  Where the shrink alone fills the chip the expand's
 // workgroups follow it in order and find their rows ready; several rounds of either hide the boundary anyway.
 bool lora_one_launch(const ExpandArgs& e, int64_t h_in, int64_t batch, int64_t rank_cap, int64_t units, int nproj) {
-  if (h_in != e.page_elems || !pages_serve(e, nproj, rank_cap) || !plan_hand_over(batch, rank_cap) || units % kXcds != 0)
+  // (delta as wide as the plan lists: a launch over fewer columns would leave the words and counters of the others behind,
+  // and a later one over all of them would wait for rows that name an older launch)
+  if (h_in != e.page_elems || e.x_cols != rank_cap || !pages_serve(e, nproj, rank_cap) || !plan_hand_over(batch, rank_cap) ||
+      units % kXcds != 0)
     return false;
   const int64_t shrinks = units * nproj;  // workgroups
   if (shrinks <= 128 || e.x_cols <= 16) return shrinks <= 1536;

@@ -102,3 +102,29 @@ def test_a_hand_over_that_never_comes_is_computed(gpu):
     torch.cuda.synchronize()
     assert torch.equal(y, y_s) and torch.equal(d, d_s)
     assert plan.status() == 2
+
+
+def test_one_plan_takes_deltas_of_different_widths(gpu):
+    """Narrow and wide deltas in turn on one plan, each right and none late: a launch that skips the rows behind a narrow
+    delta must not leave readers of a later one waiting for them."""
+    import slora_hip
+    from slora_hip import dispatch_bgmv, dispatch_bgmv_lora, dispatch_bgmv_qkv_lora
+    c = make_case(21, 4096, [64, 32, 8, 64], 9, dtype="f16", zipf_alpha=1.0)
+    g = GpuCase(c, gpu)
+    t = (g.a_start, g.a_len, g.a_loc, g.bins)
+    y0 = _outputs(c, g, gpu, True)
+    want = {}
+    for R in (16, 64):
+        y, d = _fresh(c, g, gpu, y0, R, True)
+        for p in range(4):
+            dispatch_bgmv(d[p], g.x, g.key, *t, p, g.scales, plan=False)
+            dispatch_bgmv(y[p], d[p], g.value, *t, p, g.scales, plan=False)
+        want[R] = (y, d)
+    plan = slora_hip.make_plan(*t, 64, c.n_pages)
+    for i, R in enumerate((64, 16, 64, 16, 16, 64)):
+        y, d = _fresh(c, g, gpu, y0, R, True)
+        dispatch_bgmv_qkv_lora(*y[:3], *d[:3], g.x, g.key, g.value, *t, g.scales, plan=plan)
+        dispatch_bgmv_lora(y[3], d[3], g.x, g.key, g.value, *t, 3, g.scales, plan=plan)
+        for p in range(4):
+            assert torch.equal(d[p], want[R][1][p]) and torch.equal(y[p], want[R][0][p]), (i, R, p)
+        assert plan.status() == 0, (i, R)
