@@ -37,6 +37,8 @@ extern "C" {
 /* major * 100 + minor.  The major number changes when an entry point is removed or its
  * signature changes (callers built against an older major must be rebuilt), the minor one when
  * entry points are added.
+ *   2.2 (202): + slora_store_ids.  (Decode plans hold the tagged words of slora_bgmv_lora_planned
+ *              since before this number: slora_bgmv_plan_bytes differs from early builds of 2.1.)
  *   2.1 (201): + slora_sgmm_expand_planned; prefill plans hold spans for it (slora_sgmm_plan_bytes
  *              grew from 8 to 33 KB).
  *   2.0 (200): slora_bgmv_lora_planned (shrink and expand in one launch) has a new signature and a
@@ -46,7 +48,7 @@ extern "C" {
  *   1.2 (102): + slora_sgmm_expand_qkv.
  *   1.1 (101): + slora_sgmm_shrink_qkv, slora_pool_page_checksums, slora_pool_pack_transposed,
  *              slora_pool_alloc_contiguous_static; - slora_bgmv_lora_planned. */
-#define SLORA_VERSION 201
+#define SLORA_VERSION 202
 
 #define SLORA_API __attribute__((visibility("default")))
 
@@ -342,6 +344,11 @@ SLORA_API int slora_pool_pack_transposed(void* const* dst_bufs, const void* cons
                                          const int64_t* rows, const int64_t* cols, const int64_t* dst_pitch,
                                          const int64_t* n_slot, int n_mats, const int64_t* loc, int64_t n_loc,
                                          int64_t page_elems, int64_t n_pages, void* stream);
+
+/* out[i] = host_ids[i], i < n, for a HOST array (a batch's adapter indices): the values travel as
+ * kernel arguments, so host_ids may be changed or freed when the call returns, nothing waits for the
+ * stream, and a call recorded into a graph stores what it was given at every replay. */
+SLORA_API int slora_store_ids(int64_t* out, const int64_t* host_ids, int64_t n, void* stream);
 
 /* new_a_loc[new_a_start[i] + k] = old_a_loc[old_a_start[i] + k], k < old_a_len[i],
  * i < n_adapters.  Replaces launch_var_len_copy_triton

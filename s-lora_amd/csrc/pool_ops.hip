@@ -5,6 +5,7 @@
 //                             (slora/server/router/model_infer/infer_adapter.py:56-57,
 //                             81-82: `key_buffer[l][loc] = w_combined[0]`, one
 //                             index_put per layer and side in the reference)
+//   slora_store_ids           a batch's adapter indices from the host into a device array
 //   slora_var_len_copy        new_loc[new_start[i] + k] = old_loc[old_start[i] + k]
 //                             (infer_adapter.py:261-280, launch_var_len_copy_triton)
 //   slora_tables_compact      the index tables after some adapters are dropped, and the
@@ -20,6 +21,7 @@
 // All of it is plain byte/integer movement, bound by HBM bandwidth (the first) or
 // by a handful of dependent round trips (the rest).
 
+#include <cstring>
 #include <mutex>
 
 #include "common.hpp"
@@ -244,6 +246,25 @@ __global__ __launch_bounds__(256) void pool_pack_kernel(const PackArgs p) {
     if ((uint64_t)page >= (uint64_t)p.n_pages) continue;  // a page id outside the pool is skipped
     dst[page * p.page_elems + off] = s_t[tx][cc];
   }
+}
+
+// ---------------------------------------------------------------------------
+// a few integers of the host into device memory
+// ---------------------------------------------------------------------------
+// The values travel in the launch's argument segment: nothing of the host is read after the launch call returns, no
+// transfer waits for the stream, and a recorded launch keeps them.  Bound: the launch.
+constexpr int kStoreIds = 448;  // of the 4096 bytes an argument segment may have
+struct StoreArgs {
+  int64_t v[kStoreIds];
+  int64_t* out;
+  int n;
+};
+
+__global__ __launch_bounds__(kStoreIds) void store_ids_kernel(const StoreArgs) {
+  typedef const StoreArgs __attribute__((address_space(4))) * Args;
+  const Args p = (Args)__builtin_amdgcn_kernarg_segment_ptr();  // (an array indexed by the lane: read where it lies)
+  const int i = threadIdx.x;
+  if (i < p->n) p->out[i] = p->v[i];
 }
 
 // ---------------------------------------------------------------------------
@@ -795,6 +816,22 @@ int slora_pool_pack_transposed(void* const* dst_bufs, const void* const* src_mat
       hipLaunchKernelGGL(pool_pack_vec_kernel, dim3((uint32_t)max_tiles, (uint32_t)p.n_mats), dim3(256), 0, s, p);
     else
       hipLaunchKernelGGL(pool_pack_kernel, dim3((uint32_t)max_tiles, (uint32_t)p.n_mats), dim3(256), 0, s, p);
+    if (hipGetLastError() != hipSuccess) return SLORA_ERR_LAUNCH;
+  }
+  return SLORA_OK;
+}
+
+int slora_store_ids(int64_t* out, const int64_t* host_ids, int64_t n, void* stream) {
+  using namespace slora;
+  if (n < 0) return SLORA_ERR_BAD_SHAPE;
+  if (n == 0) return SLORA_OK;
+  if (out == nullptr || host_ids == nullptr) return SLORA_ERR_NULL_POINTER;
+  for (int64_t i = 0; i < n; i += kStoreIds) {
+    StoreArgs p;
+    p.n = (int)(n - i < kStoreIds ? n - i : kStoreIds);
+    p.out = out + i;
+    std::memcpy(p.v, host_ids + i, (size_t)p.n * sizeof(int64_t));
+    hipLaunchKernelGGL(store_ids_kernel, dim3(1), dim3(kStoreIds), 0, reinterpret_cast<hipStream_t>(stream), p);
     if (hipGetLastError() != hipSuccess) return SLORA_ERR_LAUNCH;
   }
   return SLORA_OK;

@@ -967,6 +967,15 @@ bool segments_ok(const Tensor& first, const Tensor& key, const Tensor& val, cons
   return x.size(1) % 64 == 0;
 }
 
+// Adapter indices of the host in a tensor on like's device, without a transfer (see slora_store_ids)
+Tensor store_ids(const std::vector<int64_t>& ids, const Tensor& like) {
+  TORCH_CHECK(like.is_cuda(), "like must be a CUDA tensor");
+  const Tensor out = at::empty({(int64_t)ids.size()}, like.options().dtype(at::kLong));
+  check_rc(slora_store_ids(out.numel() > 0 ? out.data_ptr<int64_t>() : nullptr, ids.data(), out.numel(), stream_of(like)),
+           "store_ids");
+  return out;
+}
+
 // ---------------------------------------------------------------------------
 // pool helpers (slora/server/router/model_infer/infer_adapter.py, slora/common/mem_allocator.py)
 // ---------------------------------------------------------------------------
@@ -1263,6 +1272,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("segments_ok", &segments_ok, py::arg("first"), py::arg("key"), py::arg("val"), py::arg("a_loc"), py::arg("a_start"),
         py::arg("a_len"), py::arg("n_tok"), py::arg("width"), py::arg("x"), py::arg("out0"), py::arg("out1") = py::none(),
         py::arg("out2") = py::none());
+  m.def("store_ids", &store_ids, py::arg("ids"), py::arg("like"));
   m.def("load_rows_into_pool", &load_rows_into_pool, py::arg("buffers"), py::arg("rows"), py::arg("loc"));
   m.def("pack_transposed_into_pool", &pack_transposed_into_pool, py::arg("buffers"), py::arg("mats"), py::arg("first"),
         py::arg("dst_pitch"), py::arg("n_slot"), py::arg("loc"));

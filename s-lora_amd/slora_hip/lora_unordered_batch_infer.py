@@ -30,7 +30,7 @@ import torch
 
 from ._kernels import (dispatch_bgmv, dispatch_bgmv_lora, dispatch_bgmv_qkv_expand, dispatch_bgmv_qkv_lora,
                        dispatch_bgmv_qkv_shrink, lora_get_qkvo_fwd_expand, lora_get_qkvo_fwd_expand_qkv,
-                       lora_get_qkvo_fwd_shrink, lora_get_qkvo_fwd_shrink_qkv, segments_ok)
+                       lora_get_qkvo_fwd_shrink, lora_get_qkvo_fwd_shrink_qkv, segments_ok, store_ids)
 
 # lora_unordered_batch_infer.py:334: in the reference the segmented kernels serve batches with a long
 # request, adapters of rank >= 64 and at least two requests, and everything else is BGMV
@@ -107,6 +107,9 @@ class LoraUnorderedBatchInfer:
             ids = [infer_adapter.adapter_dirs.index(a.lora_dir) for a in adapters]
         self._ids, self._device = ids, dev
         self._req_bins: Optional[torch.Tensor] = None
+        self._step_bins: Optional[torch.Tensor] = None  # the indices as the step that was begun last reads them
+        if self._recording():
+            self.req_bins = torch.tensor(ids, dtype=torch.long, device=dev)  # refused, with the runtime's own message
         kb = self.key_buffer[0]
         self.page_elems = int(kb.shape[1] * kb.shape[2])
         self.kv_embed_dim = int(kv_embed_dim) if kv_embed_dim is not None else self.page_elems
@@ -125,19 +128,28 @@ class LoraUnorderedBatchInfer:
 
     @property
     def req_bins(self) -> torch.Tensor:
-        """Adapter index of every request, on the device (:37).  Looked at before the first ``begin_step`` it is
-        uploaded there and then, as for a decode step; a prefill step's ``begin_step`` uploads it."""
+        """Adapter index of every request, on the device (:37).  Uploaded when first looked at, if a prefill step has not
+        done so.  While a graph is being recorded a tensor of that graph takes its place: what a capture
+        writes is not there before the first replay."""
         if self._req_bins is None:
+            if self._recording():
+                return store_ids(self._ids, self.key_buffer[0])
             self._req_bins = torch.tensor(self._ids, dtype=torch.long, device=self._device)
         return self._req_bins
+
+    @req_bins.setter
+    def req_bins(self, bins: torch.Tensor) -> None:
+        self._req_bins = bins
+
+    def _recording(self) -> bool:
+        return self._device.type == "cuda" and torch.cuda.is_current_stream_capturing()
 
     def _upload_bins(self) -> None:
         """The adapter indices of a prefill step through pinned memory on the stream of the step: a copy from pageable
         memory waits for everything that is queued on the stream, i.e. for the step before, while the next one is not
         even begun (9 prompts of 2311 tokens, 8 layers: 559 -> 531 us a step).  A decode step keeps that wait: its launches
         are sized by the plan's item count, which the host has in time only where the stream is nearly idle when the
-        plan is built (23 tokens, 32 layers: 830 us, without the wait 1064).  Inside a graph capture the copy is
-        refused, as it was: a replay would read the host's memory again."""
+        plan is built (23 tokens, 32 layers: 830 us, without the wait 1064)."""
         if self._req_bins is None and self._device.type == "cuda" and not torch.cuda.is_current_stream_capturing():
             n = len(self._ids)
             # (one size for all usual batches: the first block of a size costs an allocation of pinned memory)
@@ -154,15 +166,16 @@ class LoraUnorderedBatchInfer:
         and ``total_token_num`` (the sum of ``b_seq_len``, an argument of the reference's ``forward``)
         the one inside ``repeat_interleave``, when the caller knows them: the step then starts
         without waiting for the device."""
-        assert b_start_loc.shape[0] == b_seq_len.shape[0] == len(self._ids)
+        n_req = len(self._ids) if self._req_bins is None else self._req_bins.shape[0]
+        assert b_start_loc.shape[0] == b_seq_len.shape[0] == n_req
         if is_prefill:
             self._upload_bins()
+        bins = self._step_bins = self.req_bins
         self.is_prefill = bool(is_prefill)
         self.b_start_loc, self.b_seq_len = b_start_loc, b_seq_len
         self.max_b_seq_len = int(max_b_seq_len) if max_b_seq_len is not None else int(torch.max(b_seq_len).item())
-        n_req = int(b_seq_len.shape[0])
         if self.is_prefill:
-            self.batch_req_bins = torch.repeat_interleave(self.req_bins, b_seq_len.to(torch.long),
+            self.batch_req_bins = torch.repeat_interleave(bins, b_seq_len.to(torch.long),
                                                           output_size=total_token_num)
             n_tok = int(self.batch_req_bins.shape[0])
             self.use_segmented = (self.max_b_seq_len >= PREFILL_MIN_SEQ_LEN and
@@ -191,7 +204,7 @@ class LoraUnorderedBatchInfer:
             self.batch_req_bins = None
             n_tok = n_req
             self.use_segmented = False
-            self._bins = self.req_bins
+            self._bins = bins
         self._n_tok = n_tok
         dev = self._device
         # (one fill for all three where each starts on 16 bytes, as an allocation of its own would)
@@ -207,12 +220,12 @@ class LoraUnorderedBatchInfer:
         refuse, and what only they take (tables that are not 1-D, pools of two page widths) they still take."""
         ia = self.infer_adapter
         if self.use_segmented:
-            return (ia.a_loc, ia.a_start, ia.a_len, self.b_start_loc, self.b_seq_len, self.req_bins), self.max_b_seq_len
+            return (ia.a_loc, ia.a_start, ia.a_len, self.b_start_loc, self.b_seq_len, self._step_bins), self.max_b_seq_len
         if self._prompts is None:
             return None
         if not segments_ok(self.key_buffer[0], key, val, ia.a_loc, ia.a_start, ia.a_len, self._n_tok, self.page_elems, x, *outs):
             return None
-        return (ia.a_loc, ia.a_start, ia.a_len, *self._prompts, self.req_bins), self._longest
+        return (ia.a_loc, ia.a_start, ia.a_len, *self._prompts, self._step_bins), self._longest
 
     def _one_call(self, key: torch.Tensor, val: torch.Tensor) -> bool:
         """Whether the per-token shrink and expand of a layer go out as one call (which wants whole 16-byte pieces of

@@ -63,6 +63,7 @@ SIGNATURES = {
     "slora_sgmm_expand_qkv": (_I, [_P, _P, _P, _P, _P, _P, _P, _TP, _P, _I, _P, _P, _P, _I64, _I64, _I64, _I64, _I64,
                                    _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I, _P]),
     "slora_pool_scatter_rows": (_I, [_P, _P, _I, _P, _I64, _I64, _I64, _I64, _I64, _P]),
+    "slora_store_ids": (_I, [_P, _P, _I64, _P]),
     "slora_pool_pack_transposed": (_I, [_P, _P, _P, _P, _P, _P, _P, _I, _P, _I64, _I64, _I64, _P]),
     "slora_var_len_copy": (_I, [_P, _P, _P, _P, _P, _I64, _I64, _I64, _P]),
     "slora_tables_compact": (_I, [_TP, _P, _I, _P, _P, _P, _P, _P, _P, _P, _P, _P]),

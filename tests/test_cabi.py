@@ -39,7 +39,7 @@ def test_header_and_binding_agree(lib):
 
 def test_version_and_strerror(lib):
     import cabi_ctypes as _cabi
-    assert lib.slora_version() == 201
+    assert lib.slora_version() == 202
     assert _cabi.strerror(0) == "ok"
     assert "No suitable kernel" in _cabi.strerror(_cabi.ERR_UNSUPPORTED)
     for code in range(-7, 0):
@@ -134,6 +134,15 @@ def test_planned_expand_argument_checks(lib):
     assert call(nproj=3, o12=512) == A.ERR_BAD_SHAPE                         # o1 rows narrower than feat_out12
     assert call(x_stride=32) == A.ERR_BAD_SHAPE                              # x rows narrower than max_rank
     assert call(dtype=7) == A.ERR_BAD_DTYPE
+
+
+def test_store_ids_argument_checks(lib):
+    import cabi_ctypes as A
+    P = 0x10000
+    assert lib.slora_store_ids(None, None, 0, None) == A.OK
+    assert lib.slora_store_ids(P, P, -1, None) == A.ERR_BAD_SHAPE
+    assert lib.slora_store_ids(None, P, 4, None) == A.ERR_NULL_POINTER
+    assert lib.slora_store_ids(P, None, 4, None) == A.ERR_NULL_POINTER
 
 
 def test_python_mirror_rejects_cpu_tensors():

@@ -1,0 +1,75 @@
+"""LoraUnorderedBatchInfer recorded into a HIP graph: an object that was built outside records its steps, the first one
+included, and stays usable outside the graph and on other streams."""
+import numpy as np
+import pytest
+import torch
+
+from test_engine_gpu import _Model
+
+pytestmark = pytest.mark.gpu
+
+
+def _engine(gpu, is_prefill, hidden=4096):
+    """An engine that has run no step, its arguments of begin_step and one layer's tensors."""
+    from slora_hip import LoraUnorderedBatchInfer
+    m = _Model(gpu, "f16", hidden, hidden, 1, {"a": 8, "b": 16, "c": 8}, heads=hidden // 128)
+    rng = np.random.default_rng(4)
+    req = [m.names[i] for i in rng.integers(0, 3, size=7)]
+    lens = np.asarray([40, 70, 3, 55, 64, 90, 21] if is_prefill else [9] * 7, np.int32)
+    n_tok = int(lens.sum()) if is_prefill else len(req)
+    step = dict(b_start_loc=torch.from_numpy(np.concatenate([[0], np.cumsum(lens)[:-1]]).astype(np.int32)).to(gpu),
+                b_seq_len=torch.from_numpy(lens).to(gpu), is_prefill=is_prefill, max_b_seq_len=int(lens.max()),
+                total_token_num=n_tok)
+    gen = torch.Generator(device=gpu)
+    gen.manual_seed(8)
+    t = [torch.empty((n_tok, hidden), dtype=m.tdt, device=gpu).normal_(generator=gen) for _ in range(6)]
+    return m, (lambda: LoraUnorderedBatchInfer(m.ia, [m.adapters[n] for n in req])), step, t
+
+
+def _layer(eng, step, t, y):
+    for a, b in zip(y, t[2:]):
+        a.copy_(b)
+    eng.begin_step(**step)
+    eng.lora_get_qkv(0, t[0], *y[:3])
+    eng.lora_get_o(0, t[1], y[3])
+
+
+@pytest.mark.parametrize("is_prefill", [False, True], ids=["decode", "prefill"])
+def test_the_first_step_of_an_engine_is_recorded(gpu, is_prefill):
+    """Built outside, first stepped inside a capture: every replay gives the eager bits, the object steps eagerly after the
+    capture (before and between replays), and a step recorded a second time by the same object is right as well."""
+    m, new, step, t = _engine(gpu, is_prefill)
+    want = [torch.empty_like(v) for v in t[2:]]
+    _layer(new(), step, t, want)              # (another object; also loads the kernels)
+    torch.cuda.synchronize()
+    eng = new()
+    graphs = []
+    for _ in range(2):
+        y = [torch.zeros_like(v) for v in t[2:]]
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            _layer(eng, step, t, y)
+        graphs.append((g, y))
+        late = [torch.zeros_like(v) for v in t[2:]]
+        _layer(eng, step, t, late)            # nothing of the recorded step has run yet
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(late, want))
+    for rep in range(3):
+        for g, y in graphs:
+            for v in y:
+                v.zero_()
+            g.replay()
+            torch.cuda.synchronize()
+            for a, b in zip(y, want):
+                assert torch.equal(a, b), rep
+
+
+@pytest.mark.parametrize("n", [1, 447, 448, 449, 1000])
+def test_store_ids(gpu, n):
+    """Indices of the host in a device tensor, around the number one launch carries; the list may change at once."""
+    from slora_hip._kernels import store_ids
+    ids = np.random.default_rng(n).integers(-2**40, 2**40, size=n).tolist()
+    want = list(ids)
+    got = store_ids(ids, torch.zeros(1, dtype=torch.float16, device=gpu))
+    ids[:] = [0] * n
+    assert got.dtype == torch.long and got.cpu().tolist() == want
