@@ -128,9 +128,9 @@ class LoraUnorderedBatchInfer:
 
     @property
     def req_bins(self) -> torch.Tensor:
-        """Adapter index of every request, on the device (:37).  Uploaded when first looked at, if a prefill step has not
-        done so.  While a graph is being recorded a tensor of that graph takes its place: what a capture
-        writes is not there before the first replay."""
+        """Adapter index of every request, on the device (:37).  Uploaded when first looked at, with a wait, so that any
+        stream may read it from then on.  While a graph is being recorded a tensor of that graph takes its
+        place: what a capture writes is not there before the first replay."""
         if self._req_bins is None:
             if self._recording():
                 return store_ids(self._ids, self.key_buffer[0])
@@ -144,18 +144,17 @@ class LoraUnorderedBatchInfer:
     def _recording(self) -> bool:
         return self._device.type == "cuda" and torch.cuda.is_current_stream_capturing()
 
-    def _upload_bins(self) -> None:
-        """The adapter indices of a prefill step through pinned memory on the stream of the step: a copy from pageable
-        memory waits for everything that is queued on the stream, i.e. for the step before, while the next one is not
-        even begun (9 prompts of 2311 tokens, 8 layers: 559 -> 531 us a step).  A decode step keeps that wait: its launches
-        are sized by the plan's item count, which the host has in time only where the stream is nearly idle when the
+    def _bins_of_step(self, is_prefill: bool) -> torch.Tensor:
+        """The adapter indices as a step reads them.  A prefill step has a tensor of its own, written on the step's stream by
+        a kernel out of the launch's arguments: a copy from pageable memory waits for everything that is queued on the
+        stream, i.e. for the step before, while the next one is not even begun, and a copy from pinned memory needs a new
+        block for every step that is in flight (9 prompts of 2311 tokens, 8 layers, us a step: 559, 531 and 521 in this
+        form; the first pass on new inputs 688 -> 665 against pinned memory).  A decode step keeps that wait: its launches are sized by
+        the plan's item count, which the host has in time only where the stream is nearly idle when the
         plan is built (23 tokens, 32 layers: 830 us, without the wait 1064)."""
-        if self._req_bins is None and self._device.type == "cuda" and not torch.cuda.is_current_stream_capturing():
-            n = len(self._ids)
-            # (one size for all usual batches: the first block of a size costs an allocation of pinned memory)
-            stage = torch.empty(max(n, 1024), dtype=torch.long, pin_memory=True)[:n]
-            stage.copy_(torch.tensor(self._ids, dtype=torch.long))
-            self._req_bins = stage.to(self._device, non_blocking=True)
+        if is_prefill and self._req_bins is None and self._device.type == "cuda":
+            return store_ids(self._ids, self.key_buffer[0])
+        return self.req_bins
 
     # ---- per step (forward(), :44-80) -----------------------------------------------------
     def begin_step(self, b_start_loc: torch.Tensor, b_seq_len: torch.Tensor, is_prefill: bool,
@@ -168,9 +167,7 @@ class LoraUnorderedBatchInfer:
         without waiting for the device."""
         n_req = len(self._ids) if self._req_bins is None else self._req_bins.shape[0]
         assert b_start_loc.shape[0] == b_seq_len.shape[0] == n_req
-        if is_prefill:
-            self._upload_bins()
-        bins = self._step_bins = self.req_bins
+        bins = self._step_bins = self._bins_of_step(is_prefill)
         self.is_prefill = bool(is_prefill)
         self.b_start_loc, self.b_seq_len = b_start_loc, b_seq_len
         self.max_b_seq_len = int(max_b_seq_len) if max_b_seq_len is not None else int(torch.max(b_seq_len).item())

@@ -1,5 +1,5 @@
-"""LoraUnorderedBatchInfer recorded into a HIP graph: an object that was built outside records its steps, the first one
-included, and stays usable outside the graph and on other streams."""
+"""LoraUnorderedBatchInfer recorded into a HIP graph (an object that was built outside records its steps, the first one
+included, and stays usable outside the graph), begun ahead of the device and on several streams."""
 import numpy as np
 import pytest
 import torch
@@ -73,3 +73,41 @@ def test_store_ids(gpu, n):
     got = store_ids(ids, torch.zeros(1, dtype=torch.float16, device=gpu))
     ids[:] = [0] * n
     assert got.dtype == torch.long and got.cpu().tolist() == want
+
+
+def test_prefill_steps_begun_ahead_of_the_device(gpu):
+    """Many prefill steps begun while the device is busy with the first: none takes a block of pinned memory (a block whose
+    copy is still to come cannot be used again, so each of them would be a new allocation)."""
+    m, new, step, t = _engine(gpu, True, hidden=512)
+    y = [torch.zeros_like(v) for v in t[2:]]
+    _layer(new(), step, t, y)
+    torch.cuda.synchronize()
+    before = torch.cuda.host_memory_stats()
+    torch.cuda._sleep(20_000_000)
+    engines = [new() for _ in range(8)]
+    for eng in engines:
+        eng.begin_step(**step)
+    after = torch.cuda.host_memory_stats()
+    torch.cuda.synchronize()
+    for key in ("num_host_alloc", "active_bytes.allocated"):
+        assert after.get(key, 0) == before.get(key, 0), key
+    assert all(eng.req_bins.tolist() == engines[0].req_bins.tolist() for eng in engines)
+
+
+def test_steps_of_one_engine_on_two_streams(gpu):
+    """A decode step on a stream that knows nothing of the busy one on which the object's prefill step was begun."""
+    m, new, step, t = _engine(gpu, True)
+    rows = [v[:7].clone() for v in t]
+    decode = dict(step, is_prefill=False)
+    want = [torch.empty_like(v) for v in rows[2:]]
+    _layer(new(), decode, rows, want)
+    torch.cuda.synchronize()
+    eng, y = new(), [torch.zeros_like(v) for v in rows[2:]]
+    busy, other = torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.cuda.stream(busy):
+        torch.cuda._sleep(20_000_000)
+        eng.begin_step(**step)
+    with torch.cuda.stream(other):
+        _layer(eng, decode, rows, y)
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(y, want))
