@@ -201,7 +201,8 @@ SLORA_API int slora_bgmv_expand_planned(const void* plan, int64_t rank_cap, int6
  * value_buffer[l]), which share page ids.  `plan` is written to (its hand-over area): launches that
  * use one plan must not overlap, e.g. stay on one stream.  A wait for rows that have not come after 16384
  * polls ends: the waiting wavefront computes them itself and marks the plan's status word; it never
- * happens unless workgroups are not handed out in order. */
+ * happens unless workgroups are not handed out in order.  Outputs may share memory with x (such calls take the
+ * two launches). */
 SLORA_API int slora_bgmv_lora_planned(void* plan, int64_t rank_cap, int64_t n_items, int nproj, void* y0, void* y1,
                                       void* y2, void* delta0, void* delta1, void* delta2, const void* x,
                                       const void* w_a, const void* w_b, const slora_tables* tables,

@@ -124,6 +124,11 @@ bool lora_one_launch(const ExpandArgs& e, int64_t h_in, int64_t batch, int64_t r
   return e.page_elems == ExpandPass<16>::kElems && shrinks <= 512;
 }
 
+bool overlap(const void* a, int64_t a_bytes, const void* b, int64_t b_bytes) {
+  const uintptr_t pa = reinterpret_cast<uintptr_t>(a), pb = reinterpret_cast<uintptr_t>(b);
+  return pa < pb + (uint64_t)b_bytes && pb < pa + (uint64_t)a_bytes;
+}
+
 int lora_common(const void* plan, int64_t n_items, int64_t rank_cap, void* const y[3], void* const delta[3],
                 const int64_t h_out[3], int nproj, int qkvo0, const void* x, const void* wa, const void* wb,
                 const slora_tables* tables, const int64_t* bins, const void* scales, int scales_dtype, int64_t batch,
@@ -141,7 +146,10 @@ int lora_common(const void* plan, int64_t n_items, int64_t rank_cap, void* const
   if (expands && rc != SLORA_OK) return rc;
   // the delta rows are read 8 bytes at a time by device-scope loads
   if ((delta_cols & 7) != 0) return SLORA_ERR_UNSUPPORTED;
-  if (!expands || !lora_one_launch(p.e, h_in, batch, rank_cap, grid_s, nproj)) {
+  // an output that shares memory with the activations: two launches read all of those before the first output is written
+  bool in_place = false;
+  for (int i = 0; i < nproj; ++i) in_place = in_place || overlap(x, batch * h_in * 2, y[i], batch * h_out[i] * 2);
+  if (!expands || in_place || !lora_one_launch(p.e, h_in, batch, rank_cap, grid_s, nproj)) {
     rc = slora_bgmv_shrink_planned(plan, rank_cap, n_items, nproj, delta[0], delta[1], delta[2], x, wa, tables, bins, batch,
                                    h_in, delta_cols, page_elems, n_pages, qkvo0, dtype, stream);
     if (rc != SLORA_OK || !expands) return rc;

@@ -29,6 +29,20 @@ def _fresh(c, g, gpu, y0, R, aligned):
     return y, [torch.full((c.batch, R), 0.5, dtype=g.tdt, device=gpu) for _ in range(4)]
 
 
+def _hand_over_area(batch, R):
+    """Where a plan's hand-over area starts (behind header, records and scratch) and its items: a plan is 16 words, 48 per item
+    and 6 per token; 16 words of launch counts per item follow."""
+    per_run = (R + 7) // 8
+    items = (batch * per_run + 7) // 8 * 8 + 8 * (per_run + 1)
+    return (16 + items * 48 + batch * 6 + 3) // 4 * 4, items
+
+
+def _launches_counted(plan, batch, R, first=0):
+    """Sum of the launch counts of a plan's items from `first` on: 0 unless a call took the one launch."""
+    area, items = _hand_over_area(batch, R)
+    return int(plan.buf[area + 16 * first:area + 16 * items].view(-1, 16)[:, :12].sum())
+
+
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
 @pytest.mark.parametrize("hidden,ranks,batch,h_out,R,aligned", [
     (4096, [64, 8, 16, 32, 128], 11, None, 128, True),
@@ -91,9 +105,7 @@ def test_a_hand_over_that_never_comes_is_computed(gpu):
     dispatch_bgmv(d_s, g.x, g.key, *t, 3, g.scales, plan=False)
     dispatch_bgmv(y_s, d_s, g.value, *t, 3, g.scales, plan=False)
     plan = slora_hip.make_plan(*t, R, c.n_pages)
-    per_run = R // 8
-    items = (c.batch * per_run + 7) // 8 * 8 + 8 * (per_run + 1)
-    area = (16 + items * 48 + c.batch * 6 + 3) // 4 * 4         # behind header, records and scratch
+    area, _ = _hand_over_area(c.batch, R)
     words = plan.buf.cpu().numpy()
     unit = next(u for u in range(plan.n_items) if words[16 + u * 48 + 2] > 0)   # an item with tokens
     plan.buf[area + unit * 16 + 3 * 3] = 7                      # projection o, workgroup of the shrink
@@ -128,3 +140,41 @@ def test_one_plan_takes_deltas_of_different_widths(gpu):
         for p in range(4):
             assert torch.equal(d[p], want[R][1][p]) and torch.equal(y[p], want[R][0][p]), (i, R, p)
         assert plan.status() == 0, (i, R)
+
+
+@pytest.mark.parametrize("shift", [0, 1])
+def test_outputs_that_share_memory_with_the_activations(gpu, shift):
+    """The o projection added in place to its own activations, and k written over those of q, k and v (whole, and one row
+    further down): every row of x is read before the first output is written, as with two calls."""
+    import slora_hip
+    from slora_hip import (dispatch_bgmv, dispatch_bgmv_lora, dispatch_bgmv_qkv_expand, dispatch_bgmv_qkv_lora,
+                           dispatch_bgmv_qkv_shrink)
+    c = make_case(33, 4096, [8, 16, 8], 40, dtype="bf16", zipf_alpha=1.0)
+    g = GpuCase(c, gpu)
+    t = (g.a_start, g.a_len, g.a_loc, g.bins)
+    plan = slora_hip.make_plan(*t, 16, c.n_pages)
+
+    def tensors():
+        rows = torch.zeros((c.batch + shift, 4096), dtype=g.tdt, device=gpu)
+        rows[:c.batch].copy_(g.x)
+        y, d = _fresh(c, g, gpu, _outputs(c, g, gpu, True), 16, True)
+        return rows[:c.batch], rows[shift:], y, d
+
+    x, over, y, d = tensors()
+    dispatch_bgmv_qkv_shrink(*d[:3], x, g.key, *t, plan=False)
+    dispatch_bgmv_qkv_expand(y[0], over, y[2], *d[:3], g.value, *t, g.scales, plan=False)
+    want = [over.clone(), y[0], y[2], *d[:3]]
+    x, over, y, d = tensors()
+    dispatch_bgmv_qkv_lora(y[0], over, y[2], *d[:3], x, g.key, g.value, *t, g.scales, plan=plan)
+    assert all(torch.equal(a, b) for a, b in zip([over, y[0], y[2], *d[:3]], want))
+    x, over, y, d = tensors()
+    dispatch_bgmv(d[3], x, g.key, *t, 3, g.scales, plan=False)
+    dispatch_bgmv(over, d[3], g.value, *t, 3, g.scales, plan=False)
+    want = [over.clone(), d[3]]
+    x, over, y, d = tensors()
+    dispatch_bgmv_lora(over, d[3], x, g.key, g.value, *t, 3, g.scales, plan=plan)
+    assert torch.equal(over, want[0]) and torch.equal(d[3], want[1])
+    # (the calls above had to take two launches to be right; others on this plan take one)
+    assert _launches_counted(plan, c.batch, 16) == 0
+    dispatch_bgmv_lora(y[3], d[3], x, g.key, g.value, *t, 3, g.scales, plan=plan)
+    assert _launches_counted(plan, c.batch, 16) > 0 and plan.status() == 0
