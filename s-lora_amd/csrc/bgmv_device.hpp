@@ -844,9 +844,10 @@ constexpr size_t kLdsHardLimit = 160 * 1024 - 256;
 
 // item capacity of a plan: every run's items plus the padding that evens out the 8 queues
 // (a whole number of groups of 8, so that a launch sized for the capacity keeps item i on XCD i % 8)
+int64_t plan_padding_items(int64_t rank_cap) { return kXcds * ((rank_cap + kRB - 1) / kRB + 1); }
 int64_t plan_max_items(int64_t batch, int64_t rank_cap) {
   const int64_t per_run = (rank_cap + kRB - 1) / kRB;
-  return (batch * per_run + kXcds - 1) / kXcds * kXcds + kXcds * (per_run + 1);
+  return (batch * per_run + kXcds - 1) / kXcds * kXcds + plan_padding_items(rank_cap);
 }
 // int32 words of the builder's scratch area behind the items
 int64_t plan_scratch_words(int64_t batch) { return batch * SC_WORDS; }

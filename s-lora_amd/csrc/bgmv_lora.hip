@@ -99,29 +99,37 @@ int dispatch_lora(const PageArgs& p, int64_t page_elems, hipStream_t stream) {
 }
 
 // Whether one launch serves the call (whole one-pass pages, delta as wide as the plan, and a plan with a hand-over area whose
-// launches put the workgroups of an item on its XCD), and is the faster form.  us, one launch against two, shrink + expand of q, k and v
-// and in brackets of o; `units` items each:
-//   rank 8, hidden 4096: 1 item 4.7 / 6.4 (4.6 / 6.6), 40 9.0 / 9.6 (7.1 / 9.1), 79 10.0 / 11.1 (7.4 / 9.2), 218 20.6 / 22.8 (9.5 / 11.8);
-//   5120: 62 13.4 / 14.4 (9.9 / 11.8); 8192: 67 13.7 / 15.3 (11.3 / 13.2);
-//   ranks 8 to 64, 4096: 37 8.6 / 8.7 (7.3 / 7.3), 60 14.5 / 13.1 (8.6 / 9.0), 108 14.5 / 13.7 (9.2 / 9.0), 147 17.0 / 17.1 (10.7 / 10.0),
-//   231 20.3 / 21.9 (13.6 / 12.7), 480 32.7 / 33.8 (14.7 / 15.5), 623 41.5 / 41.9 (20.2 / 19.1), 1093 74.5 / 72.4 (27.4 / 28.8);
-//   5120: 33 9.7 / 10.0 (7.4 / 8.2), 86 20.8 / 16.1 (11.3 / 12.0), 1214 103 / 98.5 (37.3 / 37.7);
-//   8192, k and v 1024 wide: 24 10.1 / 11.2 (7.9 / 9.2), 51 11.9 / 14.6 (8.7 / 10.1), 150 22.2 / 24.4 (13.4 / 14.3), 263 31.4 / 31.3
-//   (18.4 / 20.1), 607 63.3 / 60.2 (31.8 / 32.6).
-// A small launch saves the second launch, record and first data.  With every workgroup resident at once the expand's pages
-// compete with the shrink's, and a run of rank 64 waits for the slowest of eight workgroups: in the middle range
-// the two launches are level or better where ranks go beyond 16.  Where the shrink alone fills the chip the expand's
-// workgroups follow it in order and find their rows ready; several rounds of either hide the boundary anyway.
-bool lora_one_launch(const ExpandArgs& e, int64_t h_in, int64_t batch, int64_t rank_cap, int64_t units, int nproj) {
+// launches put the workgroups of an item on its XCD), and is the faster form.  `units`: items the grid is sized for, which
+// is the batch's own number only if the caller knows it (`counted`), else the plan's capacity or a quarter of it.
+//
+// Both sides measured in graphs of cold layers, us one launch / two, shrink + expand of q, k and v and in brackets of o:
+//   ranks up to 16, hidden 4096: 8 items 4.6 / 5.6 (4.4 / 6.0), 80 10.7 / 11.9 (7.4 / 9.0), 232 22.4 / 22.5 (10.0 / 12.2), 296 27.0 / 26.8
+//   (13.1 / 15.0), 528 38.9 / 36.6 (16.4 / 18.1); 5120: 272 34.8 / 36.1 (17.1 / 19.6), 336 42.3 / 40.1; 8192: 128 20.4 / 20.9 (13.7 /
+//   15.8), 216 29.9 / 27.8 (17.2 / 18.2), 448 57.8 / 48.0 (28.2 / 27.2);
+//   rank 32, 4096: 32 5.7 / 7.1 (5.0 / 6.9), 64 8.4 / 9.0 (6.5 / 7.6), 160 15.8 / 15.5 (9.1 / 10.2), 256 19.7 / 20.4 (10.0 / 11.0), 416 29.1 /
+//   28.1 (14.3 / 14.8), 896 56.8 / 51.0 (22.2 / 22.9);
+//   ranks to 64, 4096: 16 5.1 / 6.6 (5.0 / 6.5), 80 9.0 / 8.3 (6.8 / 6.9), 96 13.6 / 11.9 (8.2 / 8.1), 128 13.4 / 12.2 (7.9 / 8.3), 224 18.7 /
+//   18.6 (10.0 / 10.1), 368 27.0 / 25.5 (14.3 / 12.8), 512 33.3 / 31.9 (15.6 / 15.1), 832 51.3 / 46.6 (20.8 / 21.2); 5120: 80 11.2 / 10.3
+//   (7.3 / 8.5), 256 24.3 / 24.2 (12.3 / 12.4), 464 43.2 / 40.2 (19.8 / 18.3); 8192: 80 14.0 / 13.2 (9.0 / 9.9), 328 45.0 / 41.5 (20.5 / 20.5);
+//   k and v a quarter or an eighth of a page, 4096: 80 7.3 / 8.3, 144 11.2 / 12.5, 280 17.9 / 17.8, 512 27.7 / 26.4; 8192: 88 11.8 / 14.0,
+//   128 16.1 / 17.2, 192 22.7 / 23.2, 328 35.7 / 32.9.
+// A launch whose shrink workgroups fit the chip at once saves the second launch, record and first data.  From there on the
+// expand's pages compete with the shrink's loads, and already from about forty items where ranks go beyond 32 and all of q, k and v
+// have outputs as wide as a page: there a run waits for the slowest of eight workgroups.  Of a capacity-sized grid most
+// workgroups find no item, and the items are at most what the capacity holds beside the padding of the eight queues:
+// 23 tokens, grid of 256 for 96 items, 18.0 / 14.0 (8.1 / 8.8); 8 tokens, 136, 10.5 / 9.9 (6.9 / 6.9); 4 tokens, 104, 5.5 / 7.2 (4.9 / 6.6); rank 8, 512
+// tokens, 136 for 168, 20.7 / 22.6 (13.2 / 15.8).
+bool lora_one_launch(const ExpandArgs& e, int64_t h_in, int64_t batch, int64_t rank_cap, int64_t units, bool counted, int nproj) {
   // (delta as wide as the plan lists: a launch over fewer columns would leave the words and counters of the others behind,
   // and a later one over all of them would wait for rows that name an older launch)
   if (h_in != e.page_elems || e.x_cols != rank_cap || !pages_serve(e, nproj, rank_cap) || !plan_hand_over(batch, rank_cap) ||
       units % kXcds != 0)
     return false;
-  const int64_t shrinks = units * nproj;  // workgroups
-  if (shrinks <= 128 || e.x_cols <= 16) return shrinks <= 1536;
-  if (e.page_elems == ExpandPass<8>::kElems) return shrinks >= 448 && shrinks <= 1536;
-  return e.page_elems == ExpandPass<16>::kElems && shrinks <= 512;
+  const int64_t resident = 256 * (e.page_elems <= ExpandPass<8>::kElems ? 4 : (e.page_elems <= ExpandPass<12>::kElems ? 3 : 2));
+  const bool narrow = nproj == 3 && e.pages_shift[1] >= 2 && e.pages_shift[2] >= 2;
+  if (e.x_cols <= 32 || narrow) return units * nproj <= resident;
+  const int64_t items = counted ? units : plan_max_items(batch, rank_cap) - plan_padding_items(rank_cap);
+  return items * nproj <= (nproj == 3 ? 128 : 256);
 }
 
 bool overlap(const void* a, int64_t a_bytes, const void* b, int64_t b_bytes) {
@@ -149,7 +157,7 @@ int lora_common(const void* plan, int64_t n_items, int64_t rank_cap, void* const
   // an output that shares memory with the activations: two launches read all of those before the first output is written
   bool in_place = false;
   for (int i = 0; i < nproj; ++i) in_place = in_place || overlap(x, batch * h_in * 2, y[i], batch * h_out[i] * 2);
-  if (!expands || in_place || !lora_one_launch(p.e, h_in, batch, rank_cap, grid_s, nproj)) {
+  if (!expands || in_place || !lora_one_launch(p.e, h_in, batch, rank_cap, grid_s, grid_s == n_items, nproj)) {
     rc = slora_bgmv_shrink_planned(plan, rank_cap, n_items, nproj, delta[0], delta[1], delta[2], x, wa, tables, bins, batch,
                                    h_in, delta_cols, page_elems, n_pages, qkvo0, dtype, stream);
     if (rc != SLORA_OK || !expands) return rc;

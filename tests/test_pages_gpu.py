@@ -37,10 +37,10 @@ def _hand_over_area(batch, R):
     return (16 + items * 48 + batch * 6 + 3) // 4 * 4, items
 
 
-def _launches_counted(plan, batch, R, first=0):
+def _launches_counted(plan, batch, R, first=0, proj=slice(0, 4)):
     """Sum of the launch counts of a plan's items from `first` on: 0 unless a call took the one launch."""
     area, items = _hand_over_area(batch, R)
-    return int(plan.buf[area + 16 * first:area + 16 * items].view(-1, 16)[:, :12].sum())
+    return int(plan.buf[area + 16 * first:area + 16 * items].view(-1, 16)[:, :12].view(-1, 4, 3)[:, proj].sum())
 
 
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
@@ -178,3 +178,41 @@ def test_outputs_that_share_memory_with_the_activations(gpu, shift):
     assert _launches_counted(plan, c.batch, 16) == 0
     dispatch_bgmv_lora(y[3], d[3], x, g.key, g.value, *t, 3, g.scales, plan=plan)
     assert _launches_counted(plan, c.batch, 16) > 0 and plan.status() == 0
+
+
+@pytest.mark.parametrize("hidden,kv,ranks,batch,R,counted,qkv,o", [
+    (4096, 4096, [8], 1, 64, True, True, True),                     # 8 items
+    (4096, 4096, [64], 1, 64, True, False, True),                   # 8 items of one queue: 64
+    (4096, 4096, [64, 32, 64, 32], 23, 64, True, False, True),      # forty to 256 items
+    (4096, 4096, [64, 64, 64], 160, 64, True, False, False),        # more than 256
+    (4096, 4096, [64, 32, 16, 8], 4, 64, False, True, True),        # not counted: what the capacity can hold decides
+    (4096, 4096, [64, 32, 16, 8], 6, 64, False, False, True),
+    (4096, 4096, [8], 23, 64, False, False, True),
+    (4096, 4096, [8], 33, 64, False, False, False),
+    (4096, 4096, [16, 8], 150, 16, False, True, True),              # 3 * 328 shrink workgroups
+    (4096, 4096, [16, 8], 160, 16, False, False, True),             # 3 * 344
+    (4096, 1024, [64, 32, 16, 8], 23, 64, False, True, True),       # narrow k and v
+    (4096, 2048, [64, 32, 16, 8], 23, 64, False, False, True),
+    (8192, 8192, [16, 8], 64, 16, False, True, True),               # 3 * 152
+    (8192, 8192, [16, 8], 80, 16, False, False, True),              # 3 * 184
+])
+def test_one_launch_or_two(gpu, hidden, kv, ranks, batch, R, counted, qkv, o):
+    """On both sides of the lines between one launch and two, with the item count and without: which one a call took, and
+    the bits of the calls without a plan."""
+    import slora_hip
+    from slora_hip import dispatch_bgmv, dispatch_bgmv_lora, dispatch_bgmv_qkv_lora
+    c = make_case(600 + batch + R, hidden, ranks, batch, dtype="f16", h_out=[hidden, kv, kv, hidden])
+    g = GpuCase(c, gpu)
+    t = (g.a_start, g.a_len, g.a_loc, g.bins)
+    y0 = _outputs(c, g, gpu, True)
+    want_y, want_d = _fresh(c, g, gpu, y0, R, True)
+    for p in range(4):
+        dispatch_bgmv(want_d[p], g.x, g.key, *t, p, g.scales, plan=False)
+        dispatch_bgmv(want_y[p], want_d[p], g.value, *t, p, g.scales, plan=False)
+    plan = slora_hip.make_plan(*t, R, c.n_pages, readback=counted)
+    y, d = _fresh(c, g, gpu, y0, R, True)
+    dispatch_bgmv_qkv_lora(*y[:3], *d[:3], g.x, g.key, g.value, *t, g.scales, plan=plan)
+    dispatch_bgmv_lora(y[3], d[3], g.x, g.key, g.value, *t, 3, g.scales, plan=plan)
+    assert all(torch.equal(a, b) for a, b in zip(y + d, want_y + want_d))
+    got = [_launches_counted(plan, batch, R, proj=p) > 0 for p in (slice(0, 3), slice(3, 4))]
+    assert got == [qkv, o] and plan.status() == 0, (got, plan.n_items)
