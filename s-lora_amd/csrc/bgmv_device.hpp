@@ -40,13 +40,15 @@ __device__ __forceinline__ int64_t lookup_page(const Tables& t, int64_t li) {
 //   [42]     1 if this is the run's last stored item and rank > rank_cap (rows the plan does not list)
 // Behind the records: the one-workgroup builder's scratch (6 words per token), then, zeroed by every
 // build, the hand-over area of the one-launch LoRA (bgmv_lora.hip; plans of more than kHandTokens
-// tokens or kHandEntries rows have none):
+// tokens or kHandEntries rows have none: few of their calls would be one launch, and all their builds
+// would clear megabytes -- 4096 tokens of rank 64 50.5 us a build, 53.7 with an area, 2048 of rank
+// 128 33.3 and 36.6; at kHandEntries the clearing hides behind the rest, 512 of rank 64 17.3 and 17.3):
 //   kEpochWords words per item: [projection * 3 + s] = launches that workgroup s of the item (0: shrink,
 //   1, 2: the two halves of the expand) has taken part in;
 //   4 x rank_cap (rounded up to 8) words per token: [projection][row] = delta value | (launch << 16).
 constexpr int kPlanMagic = 0x534c5033;  // "SLP3"
 constexpr int kEpochWords = 16;
-constexpr int64_t kHandTokens = 4096, kHandEntries = 1 << 18;
+constexpr int64_t kHandTokens = 4096, kHandEntries = 1 << 15;
 constexpr int kPlanHeaderWords = 16;
 constexpr int kItemWords = 48;
 enum { PH_MAGIC = 0, PH_NITEMS = 1, PH_MAXRANK = 2, PH_BATCH = 3, PH_TT = 4, PH_RANKCAP = 5, PH_NRUNS = 6, PH_STATUS = 7 };

@@ -136,6 +136,17 @@ def test_planned_expand_argument_checks(lib):
     assert call(dtype=7) == A.ERR_BAD_DTYPE
 
 
+@pytest.mark.parametrize("batch,cap,area", [(1, 8, True), (512, 64, True), (513, 64, False), (256, 128, True), (257, 128, False),
+                                             (4096, 8, True), (4097, 8, False), (4096, 64, False), (2048, 12, True), (2049, 12, False)])
+def test_plans_that_no_launch_hands_over_in_have_no_area_for_it(lib, batch, cap, area):
+    """Header (16 words), records (48 per item) and scratch (6 per token), and behind them 16 words per item and 4 rows per
+    token only where slora_bgmv_lora_planned may use them: every build clears those."""
+    per_run, pitch = (cap + 7) // 8, (cap + 7) // 8 * 8
+    items = (batch * per_run + 7) // 8 * 8 + 8 * (per_run + 1)
+    words = (16 + items * 48 + batch * 6 + 3) // 4 * 4
+    assert lib.slora_bgmv_plan_bytes(batch, cap) == 4 * (words + (items * 16 + batch * 4 * pitch if area else 0))
+
+
 def test_store_ids_argument_checks(lib):
     import cabi_ctypes as A
     P = 0x10000
