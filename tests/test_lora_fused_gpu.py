@@ -53,9 +53,7 @@ def test_one_launch_lora_equals_the_two_calls(gpu, dtype, hidden, ranks, batch, 
             dispatch_bgmv_qkv_lora(*y3, *d3, g.x, g.key, g.value, *t, g.scales, plan=plan)
             for p in range(3):
                 assert torch.equal(d3[p], d_s[p]) and torch.equal(y3[p], y_s[p]), (p, rep)
-        # no hand-over was abandoned
-        words = plan.buf.cpu().numpy()
-        assert words[0] == 0x534c5033
+        assert plan.status() == 0   # no hand-over was abandoned (its results would be right all the same)
     # without a plan the same entry point issues the two stateless launches
     d = torch.zeros((batch, R), dtype=g.tdt, device=gpu)
     y = y0[3].clone()

@@ -54,7 +54,7 @@ def _launches_counted(plan, batch, R, first=0, proj=slice(0, 4)):
     (5120, [64, 8, 16], 7, None, 64, True),
     (6144, [8, 16], 13, None, 16, True),
     (8192, [64, 8, 32], 10, [8192, 1024, 1024, 8192], 64, True),
-    (8192, [16, 8], 130, None, 16, True),                      # workgroups that walk several items
+    (8192, [16, 8], 130, None, 16, True),
 ])
 def test_whole_page_launches_equal_the_calls_without_a_plan(gpu, dtype, hidden, ranks, batch, h_out, R, aligned):
     import slora_hip
@@ -89,31 +89,83 @@ def test_whole_page_launches_equal_the_calls_without_a_plan(gpu, dtype, hidden, 
         assert plan.status() == 0
 
 
-def test_a_hand_over_that_never_comes_is_computed(gpu):
+@pytest.mark.parametrize("ranks,R,aligned", [
+    ([16, 8], 16, True),
+    ([24, 8], 24, True),        # a rank off the vector path: delta itself is read
+    ([16, 8], 16, False),       # an output that is not 16-byte aligned: the same
+])
+def test_a_hand_over_that_never_comes_is_computed(gpu, ranks, R, aligned):
     """The word that counts a shrink workgroup's launches is changed in the plan, so that its rows name a launch nobody
     waits for: the readers give up after their poll limit, compute the rows themselves and mark the plan."""
     import slora_hip
     from slora_hip import dispatch_bgmv, dispatch_bgmv_lora
-    c = make_case(9, 4096, [16, 8], 6, dtype="f16", bins=[0, 0, 1, 0, 0, 0])
+    c = make_case(9, 4096, ranks, 6, dtype="f16", bins=[0, 0, 1, 0, 0, 0])
     g = GpuCase(c, gpu)
     t = (g.a_start, g.a_len, g.a_loc, g.bins)
-    R = 16
-    gen = torch.Generator(device=gpu)
-    gen.manual_seed(3)
-    y0 = torch.empty((c.batch, 4096), dtype=g.tdt, device=gpu).normal_(generator=gen)
-    d_s, y_s = torch.zeros((c.batch, R), dtype=g.tdt, device=gpu), y0.clone()
-    dispatch_bgmv(d_s, g.x, g.key, *t, 3, g.scales, plan=False)
-    dispatch_bgmv(y_s, d_s, g.value, *t, 3, g.scales, plan=False)
+    y0 = _outputs(c, g, gpu, True)
+    y_s, d_s = _fresh(c, g, gpu, y0, R, aligned)
+    dispatch_bgmv(d_s[3], g.x, g.key, *t, 3, g.scales, plan=False)
+    dispatch_bgmv(y_s[3], d_s[3], g.value, *t, 3, g.scales, plan=False)
     plan = slora_hip.make_plan(*t, R, c.n_pages)
     area, _ = _hand_over_area(c.batch, R)
     words = plan.buf.cpu().numpy()
-    unit = next(u for u in range(plan.n_items) if words[16 + u * 48 + 2] > 0)   # an item with tokens
+    unit = next(u for u in range(plan.n_items) if words[16 + u * 48 + 2] > 0 and words[16 + u * 48 + 1] == ranks[0])
     plan.buf[area + unit * 16 + 3 * 3] = 7                      # projection o, workgroup of the shrink
-    d, y = torch.zeros_like(d_s), y0.clone()
-    dispatch_bgmv_lora(y, d, g.x, g.key, g.value, *t, 3, g.scales, plan=plan)
+    y, d = _fresh(c, g, gpu, y0, R, aligned)
+    dispatch_bgmv_lora(y[3], d[3], g.x, g.key, g.value, *t, 3, g.scales, plan=plan)
     torch.cuda.synchronize()
-    assert torch.equal(y, y_s) and torch.equal(d, d_s)
+    assert torch.equal(y[3], y_s[3]) and torch.equal(d[3], d_s[3])
     assert plan.status() == 2
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("hidden,kv,ranks,adapters,batch,R,qkv,o", [
+    (4096, 4096, [16], 100, 245, 16, True, True),
+    (4096, 1024, [16, 24, 8], 90, 200, 24, True, True),     # the one-dimensional grid; ranks off the vector path
+    (5120, 5120, [16], 80, 245, 16, True, True),
+    (6144, 6144, [16], 80, 245, 16, True, True),
+    (8192, 1024, [16], 60, 245, 16, True, True),
+    (4096, 4096, [32, 64], 64, 64, 64, False, False),
+    (8192, 1024, [32], 60, 64, 64, True, False),
+])
+def test_workgroups_that_walk_several_items(gpu, dtype, hidden, kv, ranks, adapters, batch, R, qkv, o):
+    """A plan without an item count, a capacity above 512 (launches get a quarter of it) and a batch of more items than that, so
+    that workgroups take a second turn: two launches and, where it is one, one launch, three times on one plan, bit for bit
+    the calls without a plan."""
+    import slora_hip
+    from slora_hip import (dispatch_bgmv, dispatch_bgmv_lora, dispatch_bgmv_qkv_expand, dispatch_bgmv_qkv_lora,
+                           dispatch_bgmv_qkv_shrink)
+    rng = np.random.default_rng(batch + hidden)
+    mix = [ranks[i % len(ranks)] for i in range(adapters)]
+    bins = rng.permutation(np.concatenate([np.arange(adapters), rng.integers(0, adapters, size=batch)])[:batch])
+    need = 4 * sum(mix)
+    c = make_case(700 + hidden + R, hidden, mix, batch, dtype=dtype, h_out=[hidden, kv, kv, hidden], bins=bins, n_pages=need + 9)
+    g = GpuCase(c, gpu)
+    t = (g.a_start, g.a_len, g.a_loc, g.bins)
+    y0 = _outputs(c, g, gpu, True)
+    want_y, want_d = _fresh(c, g, gpu, y0, R, True)
+    for p in range(4):
+        dispatch_bgmv(want_d[p], g.x, g.key, *t, p, g.scales, plan=False)
+        dispatch_bgmv(want_y[p], want_d[p], g.value, *t, p, g.scales, plan=False)
+    plan = slora_hip.make_plan(*t, R, c.n_pages, readback=False)
+    _, capacity = _hand_over_area(batch, R)
+    grid = (capacity // 4 + 7) // 8 * 8
+    assert capacity > 512 and int(plan.buf[1]) > grid, (capacity, int(plan.buf[1]))
+    for rep in range(3):
+        print(f"walk {dtype} hidden {hidden} kv {kv} batch {batch} R {R} rep {rep}", flush=True)
+        y, d = _fresh(c, g, gpu, y0, R, True)
+        dispatch_bgmv_qkv_shrink(*d[:3], g.x, g.key, *t, plan=plan)
+        dispatch_bgmv_qkv_expand(*y[:3], *d[:3], g.value, *t, g.scales, plan=plan)
+        dispatch_bgmv(d[3], g.x, g.key, *t, 3, g.scales, plan=plan)
+        dispatch_bgmv(y[3], d[3], g.value, *t, 3, g.scales, plan=plan)
+        assert all(torch.equal(a, b) for a, b in zip(y + d, want_y + want_d)), (rep, "two launches")
+        y, d = _fresh(c, g, gpu, y0, R, True)
+        dispatch_bgmv_qkv_lora(*y[:3], *d[:3], g.x, g.key, g.value, *t, g.scales, plan=plan)
+        dispatch_bgmv_lora(y[3], d[3], g.x, g.key, g.value, *t, 3, g.scales, plan=plan)
+        assert all(torch.equal(a, b) for a, b in zip(y + d, want_y + want_d)), (rep, "one call")
+    # items behind the grid have been taken, and counted, by workgroups on their second turn
+    counted = [_launches_counted(plan, batch, R, first=grid, proj=p) > 0 for p in (slice(0, 3), slice(3, 4))]
+    assert counted == [qkv, o] and plan.status() == 0
 
 
 def test_one_plan_takes_deltas_of_different_widths(gpu):
