@@ -56,7 +56,8 @@ def parse_args():
                     help="dropin: 8 stateless dispatch_bgmv calls per layer exactly as the reference issues them; "
                          "fused: q/k/v shrink and q/k/v expand as one launch each (4 launches per layer); "
                          "planned*: the same with a per-step plan (built inside every timed step) passed as plan=; "
-                         "planned-lora: shrink and expand of q/k/v in one launch and of o in one launch (2 per layer)")
+                         "planned-lora: shrink and expand of q/k/v in one call and of o in one call (2 per layer), each one "
+                         "launch where the library finds that faster")
     ap.add_argument("--all-modes", action="store_true", help="also time the other modes and report them under 'modes'")
     ap.add_argument("--launch", choices=["graph", "direct"], default="graph",
                     help="graph: the step is captured once into a HIP graph and replayed; direct: Python calls")
@@ -202,6 +203,12 @@ def make_step(w, bufs, mode, keep_plan=False):
             expand(l, 3)
 
     return step, families
+
+
+def launches_per_step(mode, n_layers, plan=0):
+    """LoRA launches of a step and its plan build; None for planned-lora, whose two calls per layer are one launch or two
+    each, as the library finds faster for the batch."""
+    return None if mode == "planned-lora" else n_layers * (4 if mode.endswith("fused") else 8) + plan
 
 
 def graphed(fn, torch):
@@ -409,10 +416,11 @@ def measure_dropin_direct(w, bufs, torch, args):
 
     ms_eng = wall_ms(engine_step, max(5, args.steps // 2), 3)
     return {"engine-fused-direct": {
-        "what": "LoraUnorderedBatchInfer(fused=True) built anew every step: q/k/v in one shrink and one expand "
-                "launch per layer, direct launches from Python, plan built and reused by the library",
+        "what": "LoraUnorderedBatchInfer(fused=True) built anew every step: one call for q/k/v and one for o per layer, "
+                "one launch or two each as the library finds faster, issued directly from Python, plan built and "
+                "reused by the library",
         "ms_per_step": round(ms_eng, 4), "tokens_per_s": round(w.batch / (ms_eng * 1e-3), 1),
-        "launches_per_step": 4 * L + 2},
+        "calls_per_step": 2 * L},
         "dropin-direct-autoplan": {
         "what": "reference call pattern (8 dispatch_bgmv per layer, new req_bins per step), direct launches from "
                 "Python through the extension, plan built and reused by the library",
@@ -858,7 +866,7 @@ def main():
             fn = graphed(st, torch) if use_graph else st
             ms = time_steps(fn)
             other_modes[m] = {"ms_per_step": round(ms, 4), "tokens_per_s": round(w.batch / (ms * 1e-3), 1),
-                              "launches_per_step": w.n_layers * (2 if m == "planned-lora" else 4 if m.endswith("fused") else 8)}
+                              "launches_per_step": launches_per_step(m, w.n_layers)}
 
     # ---- launch duration of every kind of launch in the step: a sweep of that kind over
     # all layers, HIP events on the stream the kernels run on (back-to-back launches, so
@@ -954,8 +962,7 @@ def main():
             "pool_pages_per_layer": w.n_pages, "page_bytes": w.page_elems * 2, "placement": args.placement,
             "mode": args.mode,
             "launch": args.launch,
-            "launches_per_step": w.n_layers * (2 if args.mode == "planned-lora" else 4 if fused else 8) +
-                                 (1 if args.mode.startswith("planned") else 0),
+            "launches_per_step": launches_per_step(args.mode, w.n_layers, plan=1 if args.mode.startswith("planned") else 0),
         },
         "step_hbm": {
             "algorithmic_bytes_per_step": w.step_bytes(fused),

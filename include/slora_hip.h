@@ -98,7 +98,10 @@ SLORA_API int slora_bgmv_shrink(void* y, const void* x, const void* w, const slo
  *   y[b, n] = T( y[b, n] + T( sum_{d < min(r_a, x_cols)} f32(Bt[n*r_a + d]) * f32(x[b, d]) * f32(scales[a]) ) )
  * x is [batch, x_cols] contiguous, y is [batch, h_out] contiguous.  `scales`
  * is read in ITS OWN type scales_dtype (the reference reinterprets the fp16
- * scaling table as bf16 on the bf16 path, lora_ops.cc:118). */
+ * scaling table as bf16 on the bf16 path, lora_ops.cc:118).  Here and wherever
+ * scales are taken: one entry per adapter, aligned to its type.  A 16-bit entry
+ * may be read as part of the aligned 32-bit word it lies in, so the memory of a
+ * table begins and ends on four bytes, as every device allocation does. */
 SLORA_API int slora_bgmv_expand(void* y, const void* x, const void* w, const slora_tables* tables,
                       const int64_t* bins, const void* scales, int scales_dtype, int64_t batch,
                       int64_t x_cols, int64_t h_out, int64_t page_elems, int64_t n_pages,

@@ -306,7 +306,7 @@ __device__ __forceinline__ void shrink_fast(const ShrinkArgs& p, const Item& it,
 // and share its activations in that L2).
 // Grid: x = item (planned) or token * blocks + block (stateless), y = projection of the
 // launch.  s_x: [lds_tt][h_in / 8] LDS words.
-// `it` receives the item (n_tok = 0: nothing was done).
+// `it`: room for the item, the caller's, so that the turns of a workgroup that walks several share it.
 template <typename T, bool PLANNED, int NV>
 __device__ __forceinline__ int shrink_body(const ShrinkArgs& p, int unit, int proj, u32x4* s_x, Item& it) {
   constexpr int NW = 4;

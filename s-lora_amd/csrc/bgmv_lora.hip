@@ -29,8 +29,11 @@ namespace {
 // in every one-launch call on the plan, so they agree), so the area is cleared by the plan build only and launches may be
 // replayed.  Launches on one plan must not overlap.
 //
-// The wait is bounded: after spin_limit polls a wavefront computes the rows of its run itself (pages_general)
+// The wait is bounded: after spin_limit polls a wavefront computes the rows of its run itself (pages_recompute)
 // and leaves a mark in the plan's status word.
+//
+// Both halves in one kernel cost 28 to 45 spilled scalar registers, depending on type and page width (lanes of
+// vector registers, no memory); the shrink by itself spills none.
 //
 // What it took: a form whose every workgroup did both halves ran 44 us for q, k and v of S2's 256 tokens; this
 // arrangement with the general paths inlined 62, without them 36, with one polling load per token and workgroup

@@ -5,7 +5,9 @@
 // What a launch of a few tokens waits for is one wavefront's chain of round trips and instructions, so the code that a
 // wavefront runs through holds no test it could do without, and what only other runs need is kept out of its registers
 // (page_args_again): with the general paths inlined as they were, a one-token shrink took 7.5 us of a launch
-// that now takes 5.0 for both halves.
+// that now takes 5.0 for both halves.  The shrink kernels spill no register.  The expand kernels spill up to 4 scalar ones and,
+// at pages of 6144 elements, 2 or 3 vector ones (12 to 16 bytes of scratch; the f16 form over full-width outputs none: 128
+// registers are what four workgroups per compute unit allow).
 #pragma once
 
 #include "bgmv_device.hpp"

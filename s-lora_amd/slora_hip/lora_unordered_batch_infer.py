@@ -15,12 +15,16 @@ Two ways to issue the work, same results bit for bit:
 * ``fused=False``: the reference's call sequence, one ``dispatch_bgmv`` or
   ``lora_get_qkvo_fwd_*`` call per projection and direction (8 per layer),
   ``delta[0]`` shared by q and o as in the reference;
-* ``fused=True`` (default): q, k and v of a layer in one shrink launch (which reads
-  the activations once) and one expand launch, in decode and in prefill steps.
+* ``fused=True`` (default): q, k and v of a layer in one call, which reads the
+  activations once.  In decode steps shrink and expand are one call as well, which the
+  library turns into one launch where that is faster than two; in prefill steps
+  they are one launch each.
 
 Either way the first call of a step builds the batch's plan inside the library and
 the other calls of the step reuse it (the index tensors are the same objects in
-every call of a step); nothing here waits for the device.
+every call of a step).  Nothing here waits for the device, but for the upload of
+the adapter indices in front of an object's first decode step (``_bins_of_step``) and for
+what ``begin_step`` is not told (its docstring).
 """
 from __future__ import annotations
 
