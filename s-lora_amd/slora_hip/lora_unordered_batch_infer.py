@@ -28,6 +28,7 @@ what ``begin_step`` is not told (its docstring).
 """
 from __future__ import annotations
 
+from contextlib import nullcontext
 from typing import List, Optional, Sequence
 
 import torch
@@ -112,6 +113,7 @@ class LoraUnorderedBatchInfer:
         self._ids, self._device = ids, dev
         self._req_bins: Optional[torch.Tensor] = None
         self._step_bins: Optional[torch.Tensor] = None  # the indices as the step that was begun last reads them
+        self._inference = torch.is_inference_mode_enabled()
         if self._recording():
             self.req_bins = torch.tensor(ids, dtype=torch.long, device=dev)  # refused, with the runtime's own message
         kb = self.key_buffer[0]
@@ -136,14 +138,20 @@ class LoraUnorderedBatchInfer:
         stream may read it from then on.  While a graph is being recorded a tensor of that graph takes its
         place: what a capture writes is not there before the first replay."""
         if self._req_bins is None:
-            if self._recording():
-                return store_ids(self._ids, self.key_buffer[0])
-            self._req_bins = torch.tensor(self._ids, dtype=torch.long, device=self._device)
+            with self._own_mode():
+                if self._recording():
+                    return store_ids(self._ids, self.key_buffer[0])
+                self._req_bins = torch.tensor(self._ids, dtype=torch.long, device=self._device)
         return self._req_bins
 
     @req_bins.setter
     def req_bins(self, bins: torch.Tensor) -> None:
         self._req_bins = bins
+
+    def _own_mode(self):
+        """The inference mode that the object was built in, for tensors that are made later than the object but are its own:
+        plans are reused by tensor versions, which inference tensors lack."""
+        return nullcontext() if torch.is_inference_mode_enabled() == self._inference else torch.inference_mode(self._inference)
 
     def _recording(self) -> bool:
         return self._device.type == "cuda" and torch.cuda.is_current_stream_capturing()
@@ -157,7 +165,8 @@ class LoraUnorderedBatchInfer:
         the plan's item count, which the host has in time only where the stream is nearly idle when the
         plan is built (23 tokens, 32 layers: 830 us, without the wait 1064)."""
         if is_prefill and self._req_bins is None and self._device.type == "cuda":
-            return store_ids(self._ids, self.key_buffer[0])
+            with self._own_mode():
+                return store_ids(self._ids, self.key_buffer[0])
         return self.req_bins
 
     # ---- per step (forward(), :44-80) -----------------------------------------------------

@@ -111,3 +111,22 @@ def test_steps_of_one_engine_on_two_streams(gpu):
         _layer(eng, decode, rows, y)
     torch.cuda.synchronize()
     assert all(torch.equal(a, b) for a, b in zip(y, want))
+
+
+@pytest.mark.parametrize("is_prefill", [False, True], ids=["decode", "prefill"])
+def test_steps_under_inference_mode(gpu, is_prefill):
+    """An object built outside torch.inference_mode(), stepped inside: the indices are an ordinary tensor, and a decode step
+    builds its plan once."""
+    import slora_hip
+    m, new, step, t = _engine(gpu, is_prefill)
+    want, y = [torch.empty_like(v) for v in t[2:]], [torch.empty_like(v) for v in t[2:]]
+    _layer(new(), step, t, want)
+    eng = new()
+    slora_hip.clear_plan_cache()
+    slora_hip.plan_cache_stats(reset=True)
+    with torch.inference_mode():
+        _layer(eng, step, t, y)
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(y, want)) and not eng._step_bins.is_inference()
+    stats = slora_hip.plan_cache_stats()
+    assert is_prefill or (stats["builds"], stats["hits"]) == (1, 1)

@@ -42,6 +42,22 @@ def test_a_step_keeps_its_own_lengths(known):
     assert eng.batch_req_bins.tolist() == [0] * 300 + [1] * 200 + [0] * 500 + [1] * 600
 
 
+@pytest.mark.parametrize("is_prefill", [False, True])
+@pytest.mark.parametrize("built_inside", [False, True])
+def test_adapter_indices_are_of_the_mode_the_object_was_built_in(is_prefill, built_inside):
+    """A step begun under torch.inference_mode() by an object built outside reads ordinary tensors: those have the version
+    that the library's plan reuse goes by, inference tensors have none."""
+    from slora_hip import LoraUnorderedBatchInfer
+    with torch.inference_mode(built_inside):
+        eng = LoraUnorderedBatchInfer(_Table(32), [_Adapter("ab"[i % 2], 32) for i in range(4)])
+    b_seq_len = torch.tensor([30, 20, 50, 60], dtype=torch.int32)
+    with torch.inference_mode():
+        eng.begin_step(torch.cumsum(b_seq_len, 0, dtype=torch.int32) - b_seq_len, b_seq_len, is_prefill)
+        bins = eng._step_bins if is_prefill else eng._bins
+    assert bins.is_inference() == built_inside and eng.req_bins.is_inference() == built_inside
+    assert eng.req_bins.tolist() == bins.tolist() == [0, 1, 0, 1]
+
+
 def segments(eng, rows, layer=0):
     x, q, k, v = (torch.zeros((rows, eng.page_elems), dtype=eng.delta_dtype) for _ in range(4))
     return eng._segments(eng.key_buffer[layer], eng.value_buffer[layer], x, q, k, v)
