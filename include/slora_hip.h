@@ -192,7 +192,7 @@ SLORA_API int slora_bgmv_expand_planned(const void* plan, int64_t rank_cap, int6
  * reference issues the two back to back for every projection
  * (slora/models/peft/lora_unordered_batch_infer.py:267-273, 287-293, 307-313, 438-444); here both are ONE
  * launch where that is the faster form (pages of one pass -- 4096, 5120, 6144 or 8192 elements --,
- * delta_cols = rank_cap, and launches of few or of enough workgroups; at most 4096 tokens and
+ * delta_cols = rank_cap, and not too many workgroups; at most 4096 tokens and
  * tokens * rank_cap <= 2^15): the
  * shrink's workgroups hand the rows of delta = x A to the expand's through tagged words behind the plan
  * (device-scope stores and loads).  Elsewhere it is the two planned launches.

@@ -268,3 +268,25 @@ def test_one_launch_or_two(gpu, hidden, kv, ranks, batch, R, counted, qkv, o):
     assert all(torch.equal(a, b) for a, b in zip(y + d, want_y + want_d))
     got = [_launches_counted(plan, batch, R, proj=p) > 0 for p in (slice(0, 3), slice(3, 4))]
     assert got == [qkv, o] and plan.status() == 0, (got, plan.n_items)
+
+
+def test_launch_numbers_wrap(gpu):
+    """Launches are numbered in 16 bits: the four around the wrap, each on activations of its own, take no row of another."""
+    import slora_hip
+    from slora_hip import dispatch_bgmv, dispatch_bgmv_lora
+    c = make_case(44, 4096, [16, 12, 8], 11, dtype="f16")
+    g = GpuCase(c, gpu)
+    t = (g.a_start, g.a_len, g.a_loc, g.bins)
+    plan = slora_hip.make_plan(*t, 16, c.n_pages)
+    area, items = _hand_over_area(c.batch, 16)
+    plan.buf[area:area + 16 * items] = 65533
+    y0 = _outputs(c, g, gpu, True)
+    for rep in range(5):
+        x = torch.roll(g.x, rep, 1)
+        want_y, want_d = _fresh(c, g, gpu, y0, 16, True)
+        dispatch_bgmv(want_d[3], x, g.key, *t, 3, g.scales, plan=False)
+        dispatch_bgmv(want_y[3], want_d[3], g.value, *t, 3, g.scales, plan=False)
+        y, d = _fresh(c, g, gpu, y0, 16, True)
+        dispatch_bgmv_lora(y[3], d[3], x, g.key, g.value, *t, 3, g.scales, plan=plan)
+        assert torch.equal(y[3], want_y[3]) and torch.equal(d[3], want_d[3]), rep
+    assert plan.status() == 0 and int(plan.buf[area:area + 16 * items].max()) == 65538
