@@ -967,13 +967,52 @@ bool segments_ok(const Tensor& first, const Tensor& key, const Tensor& val, cons
   return x.size(1) % 64 == 0;
 }
 
-// Adapter indices of the host in a tensor on like's device, without a transfer (see slora_store_ids)
-Tensor store_ids(const std::vector<int64_t>& ids, const Tensor& like) {
+// Adapter indices of the host in a tensor on like's device (see slora_store_ids), and an event behind the store that other
+// streams and the host wait for.
+class StoredIds {
+ public:
+  StoredIds(const std::vector<int64_t>& ids, const Tensor& like, hipStream_t stream) {
+    ids_ = at::empty({(int64_t)ids.size()}, like.options().dtype(at::kLong));
+    check_rc(slora_store_ids(ids_.numel() > 0 ? ids_.data_ptr<int64_t>() : nullptr, ids.data(), ids_.numel(), stream), "store_ids");
+    check_hip(hipEventCreateWithFlags(&done_, hipEventDisableTiming));
+    const hipError_t rc = hipEventRecord(done_, stream);
+    if (rc != hipSuccess) (void)hipEventDestroy(done_);
+    check_hip(rc);
+  }
+  StoredIds(const StoredIds&) = delete;
+  StoredIds& operator=(const StoredIds&) = delete;
+  ~StoredIds() {
+    if (hipEventDestroy(done_) != hipSuccess) (void)hipGetLastError();
+  }
+  const Tensor& ids() const { return ids_; }
+  // work issued to the current stream from now on comes behind the store
+  void order() const { check_hip(hipStreamWaitEvent(static_cast<hipStream_t>(stream_of(ids_)), done_, 0)); }
+  // The host waits, also while this thread records a graph (waits are refused in a capture's own mode, because a captured
+  // event could never come; this one is outside any).
+  void wait() const {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    check_hip(hipThreadExchangeStreamCaptureMode(&mode));
+    hipError_t rc;
+    {
+      py::gil_scoped_release free;
+      rc = hipEventSynchronize(done_);
+    }
+    check_hip(hipThreadExchangeStreamCaptureMode(&mode));
+    check_hip(rc);
+  }
+
+ private:
+  static void check_hip(hipError_t rc) { TORCH_CHECK(rc == hipSuccess, "store_ids: ", hipGetErrorString(rc)); }
+  Tensor ids_;
+  hipEvent_t done_ = nullptr;
+};
+
+// On the default stream only, else nullptr: every other stream may be recorded into a graph later, and while it is the
+// runtime refuses to wait for an event on it, be it older than the recording (and the recording is lost).
+std::shared_ptr<StoredIds> store_ids(const std::vector<int64_t>& ids, const Tensor& like) {
   TORCH_CHECK(like.is_cuda(), "like must be a CUDA tensor");
-  const Tensor out = at::empty({(int64_t)ids.size()}, like.options().dtype(at::kLong));
-  check_rc(slora_store_ids(out.numel() > 0 ? out.data_ptr<int64_t>() : nullptr, ids.data(), out.numel(), stream_of(like)),
-           "store_ids");
-  return out;
+  hipStream_t stream = static_cast<hipStream_t>(stream_of(like));
+  return stream == nullptr ? std::make_shared<StoredIds>(ids, like, stream) : nullptr;
 }
 
 // ---------------------------------------------------------------------------
@@ -1201,6 +1240,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
            "status word of the plan (waits for the current stream): 0, or bit 0 = a launch named another batch "
            "size or rank cap and did nothing, bit 1 = a hand-over of the one-launch LoRA took too long and its rows were "
            "computed a second time");
+  py::class_<StoredIds, std::shared_ptr<StoredIds>>(m, "StoredIds")
+      .def_property_readonly("ids", &StoredIds::ids)
+      .def("order", &StoredIds::order)
+      .def("wait", &StoredIds::wait);
+  m.def("store_ids", &store_ids, py::arg("ids"), py::arg("like"));
   py::class_<SgmmPlan, std::shared_ptr<SgmmPlan>>(m, "SgmmPlan")
       .def_readonly("buf", &SgmmPlan::buf)
       .def_readonly("usable", &SgmmPlan::usable)
@@ -1272,7 +1316,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("segments_ok", &segments_ok, py::arg("first"), py::arg("key"), py::arg("val"), py::arg("a_loc"), py::arg("a_start"),
         py::arg("a_len"), py::arg("n_tok"), py::arg("width"), py::arg("x"), py::arg("out0"), py::arg("out1") = py::none(),
         py::arg("out2") = py::none());
-  m.def("store_ids", &store_ids, py::arg("ids"), py::arg("like"));
   m.def("load_rows_into_pool", &load_rows_into_pool, py::arg("buffers"), py::arg("rows"), py::arg("loc"));
   m.def("pack_transposed_into_pool", &pack_transposed_into_pool, py::arg("buffers"), py::arg("mats"), py::arg("first"),
         py::arg("dst_pitch"), py::arg("n_slot"), py::arg("loc"));

@@ -22,13 +22,11 @@ Two ways to issue the work, same results bit for bit:
 
 Either way the first call of a step builds the batch's plan inside the library and
 the other calls of the step reuse it (the index tensors are the same objects in
-every call of a step).  Nothing here waits for the device, but for the upload of
-the adapter indices in front of an object's first decode step (``_bins_of_step``) and for
-what ``begin_step`` is not told (its docstring).
+every call of a step).  Nothing here waits for the device, but an object's first decode
+step (``begin_step``) and what ``begin_step`` is not told (its docstring).
 """
 from __future__ import annotations
 
-from contextlib import nullcontext
 from typing import List, Optional, Sequence
 
 import torch
@@ -110,12 +108,13 @@ class LoraUnorderedBatchInfer:
             ids = [idx_map[a.lora_dir] for a in adapters]
         else:
             ids = [infer_adapter.adapter_dirs.index(a.lora_dir) for a in adapters]
-        self._ids, self._device = ids, dev
-        self._req_bins: Optional[torch.Tensor] = None
-        self._step_bins: Optional[torch.Tensor] = None  # the indices as the step that was begun last reads them
-        self._inference = torch.is_inference_mode_enabled()
-        if self._recording():
-            self.req_bins = torch.tensor(ids, dtype=torch.long, device=dev)  # refused, with the runtime's own message
+        # On the default stream the adapter indices go to the device as kernel arguments: a copy waits for everything
+        # queued on the stream, i.e. for the step before, while the next one is not even begun, and a copy from pinned memory
+        # needs a new block for every step that is in flight (9 prompts of 2311 tokens, 8 layers, us a step: 559, 531 and 526 in
+        # this form).  `_stored`: what steps wait for until the host has.  On other streams it is the copy, which
+        # is also what refuses an object that is built while a graph is being recorded.
+        self._stored = store_ids(ids, self.key_buffer[0]) if dev.type == "cuda" else None
+        self._req_bins = torch.tensor(ids, dtype=torch.long, device=dev) if self._stored is None else self._stored.ids
         kb = self.key_buffer[0]
         self.page_elems = int(kb.shape[1] * kb.shape[2])
         self.kv_embed_dim = int(kv_embed_dim) if kv_embed_dim is not None else self.page_elems
@@ -134,40 +133,20 @@ class LoraUnorderedBatchInfer:
 
     @property
     def req_bins(self) -> torch.Tensor:
-        """Adapter index of every request, on the device (:37).  Uploaded when first looked at, with a wait, so that any
-        stream may read it from then on.  While a graph is being recorded a tensor of that graph takes its
-        place: what a capture writes is not there before the first replay."""
-        if self._req_bins is None:
-            with self._own_mode():
-                if self._recording():
-                    return store_ids(self._ids, self.key_buffer[0])
-                self._req_bins = torch.tensor(self._ids, dtype=torch.long, device=self._device)
+        """Adapter index of every request, on the device (:37), there for every stream.  Steps read this tensor, recorded
+        ones at every replay."""
+        self._settle()
         return self._req_bins
 
     @req_bins.setter
     def req_bins(self, bins: torch.Tensor) -> None:
-        self._req_bins = bins
+        self._req_bins, self._stored = bins, None
 
-    def _own_mode(self):
-        """The inference mode that the object was built in, for tensors that are made later than the object but are its own:
-        plans are reused by tensor versions, which inference tensors lack."""
-        return nullcontext() if torch.is_inference_mode_enabled() == self._inference else torch.inference_mode(self._inference)
-
-    def _recording(self) -> bool:
-        return self._device.type == "cuda" and torch.cuda.is_current_stream_capturing()
-
-    def _bins_of_step(self, is_prefill: bool) -> torch.Tensor:
-        """The adapter indices as a step reads them.  A prefill step has a tensor of its own, written on the step's stream by
-        a kernel out of the launch's arguments: a copy from pageable memory waits for everything that is queued on the
-        stream, i.e. for the step before, while the next one is not even begun, and a copy from pinned memory needs a new
-        block for every step that is in flight (9 prompts of 2311 tokens, 8 layers, us a step: 559, 531 and 521 in this
-        form; the first pass on new inputs 688 -> 665 against pinned memory).  A decode step keeps that wait: its launches are sized by
-        the plan's item count, which the host has in time only where the stream is nearly idle when the
-        plan is built (23 tokens, 32 layers: 830 us, without the wait 1064)."""
-        if is_prefill and self._req_bins is None and self._device.type == "cuda":
-            with self._own_mode():
-                return store_ids(self._ids, self.key_buffer[0])
-        return self.req_bins
+    def _settle(self) -> None:
+        """The host waits, once, until the indices are on the device; also while this thread records a graph."""
+        if self._stored is not None:
+            self._stored.wait()
+            self._stored = None
 
     # ---- per step (forward(), :44-80) -----------------------------------------------------
     def begin_step(self, b_start_loc: torch.Tensor, b_seq_len: torch.Tensor, is_prefill: bool,
@@ -178,12 +157,20 @@ class LoraUnorderedBatchInfer:
         and ``total_token_num`` (the sum of ``b_seq_len``, an argument of the reference's ``forward``)
         the one inside ``repeat_interleave``, when the caller knows them: the step then starts
         without waiting for the device."""
-        n_req = len(self._ids) if self._req_bins is None else self._req_bins.shape[0]
-        assert b_start_loc.shape[0] == b_seq_len.shape[0] == n_req
-        bins = self._step_bins = self._bins_of_step(is_prefill)
+        bins = self._req_bins
+        assert b_start_loc.shape[0] == b_seq_len.shape[0] == bins.shape[0]
+        if self._stored is not None:
+            if is_prefill and not torch.cuda.is_current_stream_capturing():
+                self._stored.order()
+            else:
+                # A graph may be replayed on any stream.  The launches of a decode step are sized by the plan's item count,
+                # which the host has in time only where the stream is nearly idle when the plan is built (23 tokens, 32
+                # layers: 830 us, without the wait 1064).
+                self._settle()
         self.is_prefill = bool(is_prefill)
         self.b_start_loc, self.b_seq_len = b_start_loc, b_seq_len
         self.max_b_seq_len = int(max_b_seq_len) if max_b_seq_len is not None else int(torch.max(b_seq_len).item())
+        n_req = int(b_seq_len.shape[0])
         if self.is_prefill:
             self.batch_req_bins = torch.repeat_interleave(bins, b_seq_len.to(torch.long),
                                                           output_size=total_token_num)
@@ -216,7 +203,7 @@ class LoraUnorderedBatchInfer:
             self.use_segmented = False
             self._bins = bins
         self._n_tok = n_tok
-        dev = self._device
+        dev = bins.device
         # (one fill for all three where each starts on 16 bytes, as an allocation of its own would)
         shape = (n_tok, self.max_lora_dim)
         if self.max_lora_dim % 8 == 0:
@@ -230,12 +217,12 @@ class LoraUnorderedBatchInfer:
         refuse, and what only they take (tables that are not 1-D, pools of two page widths) they still take."""
         ia = self.infer_adapter
         if self.use_segmented:
-            return (ia.a_loc, ia.a_start, ia.a_len, self.b_start_loc, self.b_seq_len, self._step_bins), self.max_b_seq_len
+            return (ia.a_loc, ia.a_start, ia.a_len, self.b_start_loc, self.b_seq_len, self._req_bins), self.max_b_seq_len
         if self._prompts is None:
             return None
         if not segments_ok(self.key_buffer[0], key, val, ia.a_loc, ia.a_start, ia.a_len, self._n_tok, self.page_elems, x, *outs):
             return None
-        return (ia.a_loc, ia.a_start, ia.a_len, *self._prompts, self._step_bins), self._longest
+        return (ia.a_loc, ia.a_start, ia.a_len, *self._prompts, self._req_bins), self._longest
 
     def _one_call(self, key: torch.Tensor, val: torch.Tensor) -> bool:
         """Whether the per-token shrink and expand of a layer go out as one call (which wants whole 16-byte pieces of

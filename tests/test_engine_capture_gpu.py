@@ -64,15 +64,25 @@ def test_the_first_step_of_an_engine_is_recorded(gpu, is_prefill):
                 assert torch.equal(a, b), rep
 
 
-@pytest.mark.parametrize("n", [1, 447, 448, 449, 1000])
-def test_store_ids(gpu, n):
-    """Indices of the host in a device tensor, around the number one launch carries; the list may change at once."""
+@pytest.mark.parametrize("n", [0, 1, 447, 448, 449, 1000])
+def test_stored_ids(gpu, n):
+    """Indices of the host in a device tensor, around the number one launch carries, behind other work of the default stream;
+    the list may change at once, other streams and the host can wait.  Not on a stream that may be recorded."""
     from slora_hip._kernels import store_ids
+    like = torch.zeros(1, dtype=torch.float16, device=gpu)
     ids = np.random.default_rng(n).integers(-2**40, 2**40, size=n).tolist()
     want = list(ids)
-    got = store_ids(ids, torch.zeros(1, dtype=torch.float16, device=gpu))
+    torch.cuda._sleep(2_000_000)
+    stored = store_ids(ids, like)
     ids[:] = [0] * n
-    assert got.dtype == torch.long and got.cpu().tolist() == want
+    with torch.cuda.stream(torch.cuda.Stream()):
+        assert store_ids(ids, like) is None
+        stored.order()
+        copy = stored.ids.clone()
+    stored.wait()
+    assert stored.ids.dtype == torch.long and stored.ids.cpu().tolist() == want
+    torch.cuda.synchronize()
+    assert copy.tolist() == want
 
 
 def test_prefill_steps_begun_ahead_of_the_device(gpu):
@@ -127,6 +137,73 @@ def test_steps_under_inference_mode(gpu, is_prefill):
     with torch.inference_mode():
         _layer(eng, step, t, y)
     torch.cuda.synchronize()
-    assert all(torch.equal(a, b) for a, b in zip(y, want)) and not eng._step_bins.is_inference()
+    assert all(torch.equal(a, b) for a, b in zip(y, want)) and not eng.req_bins.is_inference()
     stats = slora_hip.plan_cache_stats()
     assert is_prefill or (stats["builds"], stats["hits"]) == (1, 1)
+
+
+@pytest.mark.parametrize("is_prefill", [False, True], ids=["decode", "prefill"])
+@pytest.mark.parametrize("warm_up", [False, True])
+def test_replays_follow_the_adapter_indices(gpu, is_prefill, warm_up):
+    """A recorded step reads req_bins: other adapters written there in place are those of the next replay."""
+    m, new, step, t = _engine(gpu, is_prefill)
+    eng, y = new(), [torch.zeros_like(v) for v in t[2:]]
+    if warm_up:
+        _layer(eng, step, t, y)
+        torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        _layer(eng, step, t, y)
+    for shift in (0, 1, 2):
+        other, want = new(), [torch.zeros_like(v) for v in t[2:]]
+        other.req_bins.copy_((other.req_bins + shift) % 3)
+        eng.req_bins.copy_(other.req_bins)
+        _layer(other, step, t, want)
+        g.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(y, want)), shift
+
+
+@pytest.mark.parametrize("is_prefill", [False, True], ids=["decode", "prefill"])
+@pytest.mark.parametrize("same_stream", [False, True])
+def test_a_capture_that_waits_for_nothing(gpu, is_prefill, same_stream):
+    """Recorded with capture_begin alone, which waits for no stream, by an object whose indices are still behind other work;
+    replayed at once on a stream that knows nothing of that work."""
+    m, new, step, t = _engine(gpu, is_prefill)
+    want, y = [torch.zeros_like(v) for v in t[2:]], [torch.zeros_like(v) for v in t[2:]]
+    _layer(new(), step, t, want)
+    records, replays = torch.cuda.Stream(), torch.cuda.Stream()
+    busy = records if same_stream else torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(busy):
+        torch.cuda._sleep(20_000_000)
+        eng = new()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(records):
+        g.capture_begin()
+        _layer(eng, step, t, y)
+        g.capture_end()
+    with torch.cuda.stream(replays):
+        g.replay()
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(y, want))
+
+
+def test_indices_looked_at_while_their_stream_is_recorded(gpu):
+    """The stream that an object was built on is being recorded; the host waits for the indices all the same, and the recording
+    goes on."""
+    m, new, step, t = _engine(gpu, False, hidden=512)
+    want = new().req_bins.tolist()
+    s, g, out = torch.cuda.Stream(), torch.cuda.CUDAGraph(), torch.zeros(4, device=gpu)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(s):
+        torch.cuda._sleep(20_000_000)
+        eng = new()
+        g.capture_begin(capture_error_mode="thread_local")
+    bins = eng.req_bins
+    with torch.cuda.stream(s):
+        out.add_(1)
+        g.capture_end()
+    g.replay()
+    torch.cuda.synchronize()
+    assert bins.tolist() == want and out.tolist() == [1, 1, 1, 1]
