@@ -112,8 +112,10 @@ class LoraUnorderedBatchInfer:
         # queued on the stream, i.e. for the step before, while the next one is not even begun, and a copy from pinned memory
         # needs a new block for every step that is in flight (9 prompts of 2311 tokens, 8 layers, us a step: 559, 531 and 526 in
         # this form).  `_stored`: what steps wait for until the host has.  On other streams it is the copy, which
-        # is also what refuses an object that is built while a graph is being recorded.
-        self._stored = store_ids(ids, self.key_buffer[0]) if dev.type == "cuda" else None
+        # is also what refuses an object that is built while a graph is being recorded, and so it is for a pool of another
+        # device than the current one, whose default stream the launch would go to.
+        here = dev.type == "cuda" and dev.index == torch.cuda.current_device()
+        self._stored = store_ids(ids, self.key_buffer[0]) if here else None
         self._req_bins = torch.tensor(ids, dtype=torch.long, device=dev) if self._stored is None else self._stored.ids
         kb = self.key_buffer[0]
         self.page_elems = int(kb.shape[1] * kb.shape[2])

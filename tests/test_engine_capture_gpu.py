@@ -85,6 +85,21 @@ def test_stored_ids(gpu, n):
     assert copy.tolist() == want
 
 
+def test_a_pool_of_another_device_than_the_current_one(gpu, monkeypatch):
+    """The indices' store is a launch on the current device's default stream; for a pool of another device they are copied."""
+    from slora_hip import lora_unordered_batch_infer as module
+    m, new, step, t = _engine(gpu, False, hidden=512)
+    stored = []
+    monkeypatch.setattr(module, "store_ids", lambda ids, like, store=module.store_ids: stored.append(ids) or store(ids, like))
+    want = new().req_bins.tolist()
+    assert len(stored) == 1
+    other = torch.cuda.current_device() + 1
+    with monkeypatch.context() as patch:
+        patch.setattr(torch.cuda, "current_device", lambda: other)
+        eng = new()
+    assert len(stored) == 1 and eng.req_bins.tolist() == want and eng.req_bins.device == eng.key_buffer[0].device
+
+
 def test_prefill_steps_begun_ahead_of_the_device(gpu):
     """Many prefill steps begun while the device is busy with the first: none takes a block of pinned memory (a block whose
     copy is still to come cannot be used again, so each of them would be a new allocation)."""
