@@ -146,8 +146,9 @@ class LoraUnorderedBatchInfer:
 
     def _settle(self) -> None:
         """The host waits, once, until the indices are on the device; also while this thread records a graph."""
-        if self._stored is not None:
-            self._stored.wait()
+        stored = self._stored  # (read once: another thread may have waited in between)
+        if stored is not None:
+            stored.wait()
             self._stored = None
 
     # ---- per step (forward(), :44-80) -----------------------------------------------------
@@ -159,11 +160,11 @@ class LoraUnorderedBatchInfer:
         and ``total_token_num`` (the sum of ``b_seq_len``, an argument of the reference's ``forward``)
         the one inside ``repeat_interleave``, when the caller knows them: the step then starts
         without waiting for the device."""
-        bins = self._req_bins
+        bins, stored = self._req_bins, self._stored
         assert b_start_loc.shape[0] == b_seq_len.shape[0] == bins.shape[0]
-        if self._stored is not None:
+        if stored is not None:
             if is_prefill and not torch.cuda.is_current_stream_capturing():
-                self._stored.order()
+                stored.order()
             else:
                 # A graph may be replayed on any stream.  The launches of a decode step are sized by the plan's item count,
                 # which the host has in time only where the stream is nearly idle when the plan is built (23 tokens, 32

@@ -57,6 +57,36 @@ def test_adapter_indices_are_of_the_mode_the_object_was_built_in(is_prefill, bui
     assert is_prefill or eng._bins is eng.req_bins
 
 
+def test_two_threads_look_at_the_adapter_indices():
+    """One thread has waited for the indices between another's look at what there is to wait for and its wait."""
+    from slora_hip import LoraUnorderedBatchInfer
+
+    class Stored:
+        waits = 0
+
+        def wait(self):
+            Stored.waits += 1
+
+    class Engine(LoraUnorderedBatchInfer):
+        _looks = None
+
+        @property
+        def _stored(self):
+            return self._looks.pop(0) if self._looks else None
+
+        @_stored.setter
+        def _stored(self, value):
+            pass
+
+    eng = Engine(_Table(32), [_Adapter("ab"[i % 2], 32) for i in range(4)])
+    eng._looks = [Stored()]  # what the second look finds: nothing
+    assert eng.req_bins.tolist() == [0, 1, 0, 1] and Stored.waits == 1
+    eng._looks = [Stored()]
+    b_seq_len = torch.tensor([1, 1, 1, 1], dtype=torch.int32)
+    eng.begin_step(torch.cumsum(b_seq_len, 0, dtype=torch.int32) - b_seq_len, b_seq_len, False)
+    assert eng._bins is eng.req_bins
+
+
 def segments(eng, rows, layer=0):
     x, q, k, v = (torch.zeros((rows, eng.page_elems), dtype=eng.delta_dtype) for _ in range(4))
     return eng._segments(eng.key_buffer[layer], eng.value_buffer[layer], x, q, k, v)
