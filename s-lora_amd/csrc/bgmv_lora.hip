@@ -155,8 +155,8 @@ int lora_common(const void* plan, int64_t n_items, int64_t rank_cap, void* const
                       batch, delta_cols, page_elems, n_pages, dtype, p.e, grid_e);
   const bool expands = rc != kNothingToDo;
   if (expands && rc != SLORA_OK) return rc;
-  // the delta rows are read 8 bytes at a time by device-scope loads
-  if ((delta_cols & 7) != 0) return SLORA_ERR_UNSUPPORTED;
+  // whole 16-byte pieces of delta, where anything reads it: a call without outputs is the shrink alone
+  if (expands && (delta_cols & 7) != 0) return SLORA_ERR_UNSUPPORTED;
   // an output that shares memory with the activations: two launches read all of those before the first output is written
   bool in_place = false;
   for (int i = 0; i < nproj; ++i) in_place = in_place || overlap(x, batch * h_in * 2, y[i], batch * h_out[i] * 2);

@@ -109,6 +109,37 @@ def test_decode_operators_through_the_c_abi(hip, dtype):
         assert np.all(np.abs(y_gpu - y_ref) <= ATOL + RTOL * np.abs(y_ref) + step)
 
 
+@pytest.mark.parametrize("R", [12, 16])
+def test_shrink_and_expand_in_one_call_without_outputs(hip, R):
+    """slora_bgmv_lora_planned over outputs of no columns is the shrink alone, of any delta width; with outputs a width that is no
+    multiple of 8 is refused and nothing is written."""
+    import cabi_ctypes as A
+    lib = A.load_library()
+    H, batch = 512, 7
+    c = make_case(24, H, [16, 8], batch, dtype="f16")
+    key, val = hip.upload(to_bits(c.key, "f16")), hip.upload(to_bits(c.value, "f16"))
+    tables = A.SloraTables(hip.upload(c.a_start.astype(np.int64)), hip.upload(c.a_len.astype(np.int64)),
+                           hip.upload(c.a_loc.astype(np.int64)), 2, int(c.a_loc.size))
+    bins, x = hip.upload(c.bins.astype(np.int64)), hip.upload(to_bits(c.x, "f16"))
+    scales = hip.upload(c.scales.astype(np.float16))
+    nbytes = lib.slora_bgmv_plan_bytes(batch, R)
+    plan = hip.upload(np.zeros(nbytes, np.uint8))
+    assert lib.slora_bgmv_plan_build(plan, nbytes, C.byref(tables), bins, batch, R, c.n_pages, None) == A.OK
+    y0 = np.full((batch, H), 0x3c00, np.uint16)
+    want = O.ref_bgmv_shrink(np.zeros((batch, R), np.float32), c.x, c.key, c.a_start, c.a_len, c.a_loc, c.bins, 1, "f16")
+    for h_out in (0, H):
+        delta, y = hip.upload(np.zeros((batch, R), np.uint16)), hip.upload(y0)
+        print(f"c-abi lora R {R} h_out {h_out}", flush=True)
+        rc = lib.slora_bgmv_lora_planned(plan, R, 0, 1, y, None, None, delta, None, None, x, key, val, C.byref(tables), bins,
+                                         scales, A.DTYPE_F16, batch, H, R, h_out, 0, 0, c.page_elems, c.n_pages, 1, A.DTYPE_F16,
+                                         None)
+        refused = h_out > 0 and R % 8 != 0
+        assert rc == (A.ERR_UNSUPPORTED if refused else A.OK), A.strerror(rc)
+        d_gpu = from_bits(hip.download(delta, (batch, R), np.uint16), "f16")
+        np.testing.assert_allclose(d_gpu, np.zeros_like(want) if refused else want, rtol=RTOL, atol=ATOL)
+        assert np.array_equal(hip.download(y, (batch, H), np.uint16), y0) == (h_out == 0 or refused)
+
+
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
 def test_prefill_operators_through_the_c_abi(hip, dtype):
     import cabi_ctypes as A
